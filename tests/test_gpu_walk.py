@@ -1,0 +1,111 @@
+"""The cooperative walk (walk_coop, one walk per wave) against the per-lane
+walk of the radix tree: lists, last candidates, mindist, v and the FP64 sums
+equal bit for bit, at the sizes where its cells per wave and the levels of its
+tree of boxes change, and on colonies that take its rarer branches -- cells in
+many places, cells without a neighbour beside crowded ones, queues longer than
+their room, waves of many small colonies."""
+import numpy as np
+import pytest
+
+from timothy_amd import generators as gen
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def ctx(tm):
+    c = tm.Context(0)
+    yield c
+    c.close()
+
+
+def gaussian(n):
+    return gen.gaussian_colony(n, 900 + n % 89, 146.6 * (n / 2e6) ** (1 / 3), frac_type1=0.05)
+
+
+def cells(pos, types=gen.CELLTYPES):
+    n = len(pos)
+    return gen._cells(np.asarray(pos, np.float64), np.zeros(n, np.int32), gen.Stream(7, 2), types)
+
+
+def wide_type(h):
+    return [dict(size=1.0, h=h, h2=h ** 2, h3=h ** 3, h4=h ** 4)]
+
+
+def scattered(n):
+    """far apart: no cell has a neighbour"""
+    return cells(gen.Stream(31, 1).uniform(3 * n).reshape(n, 3) * 4000.0)
+
+
+def crowd_and_strays(n):
+    """a dense ball and lone cells around it, a cutoff of seven radii: waves
+    with hundreds of candidates hold cells without a neighbour"""
+    st = gen.Stream(33, 1)
+    ball = gen.uniform_ball(n, 0.9 * n ** (1 / 3), st)
+    out = gen.uniform_ball(400, 60.0 * n ** (1 / 3) / 10, st)
+    out = out[(out ** 2).sum(1) > (0.9 * n ** (1 / 3) + 8) ** 2]
+    return cells(np.concatenate([ball, out]), wide_type(7.0))
+
+
+def clusters(k, m):
+    """k small clumps far apart, in an order that mixes them within waves"""
+    st = gen.Stream(35, 1)
+    at = st.uniform(3 * k).reshape(k, 3) * 900.0
+    return cells((at[:, None, :] + gen.Stream(36, 1).normal(3 * k * m).reshape(k, m, 3)).reshape(-1, 3))
+
+
+CASES = [(f"gaussian {n}", lambda n=n: gaussian(n))
+         for n in (2, 15, 63, 65, 1023, 1025, 32768, 32769, 65537, 131073)] + [
+    ("scattered", lambda: scattered(5000)),
+    ("crowd and strays", lambda: crowd_and_strays(6000)),
+    ("clusters", lambda: clusters(700, 5)),
+    ("far cutoff", lambda: dict(gen.ball_colony(9000, 41), types=wide_type(9.0))),
+]
+
+
+def outputs(tm, ctx, coop, lists):
+    ctx.set_param("walk_coop", coop)
+    ctx.step(tm.FP64)
+    return dict(ctx.results(), qstar=ctx.qstar(), **(dict(zip(("off", "nbr"), ctx.neighbor_lists())) if lists else {}))
+
+
+@pytest.mark.parametrize("name,make", CASES)
+@pytest.mark.parametrize("ratio", [64, 3])
+def test_matches_per_lane_walk(tm, ctx, name, make, ratio):
+    ctx.upload_colony(make())
+    ctx.set_param("walk_coop_ratio", ratio)
+    ref, got = outputs(tm, ctx, 0, True), outputs(tm, ctx, 1, True)
+    for k in ref:
+        assert np.array_equal(got[k], ref[k]), k
+    ctx.set_param("walk_coop_ratio", 64)
+
+
+def test_small_colonies_in_one_wave(tm, ctx):
+    cols = [gaussian(m) for m in [1, 2, 3, 5, 8, 13, 21, 34, 55, 89, 144, 233] * 30]
+    ctx.upload_colonies(cols)
+    ref, got = outputs(tm, ctx, 0, True), outputs(tm, ctx, 1, True)
+    for k in ref:
+        assert np.array_equal(got[k], ref[k]), k
+
+
+@pytest.mark.parametrize("n", [786433, 4194305 + 70])
+def test_matches_per_lane_walk_large(tm, ctx, n):
+    ctx.upload_colony(gaussian(n))
+    ref, got = outputs(tm, ctx, 0, False), outputs(tm, ctx, 1, False)
+    for k in ref:
+        assert np.array_equal(got[k], ref[k]), k
+
+
+def test_octree_on_demand(tm, ctx):
+    """the radix tree is made when asked for: after a cooperative step, and
+    anew after a replay of a captured one"""
+    ctx.upload_colony(gaussian(3000))
+    ctx.set_param("walk_coop", 0)
+    ctx.step(tm.MIXED)
+    ref = ctx.octree(0)
+    ctx.set_param("walk_coop", 1)
+    ctx.graph_capture(tm.MIXED)
+    for _ in range(3):
+        ctx.graph_launch()
+        assert np.array_equal(ctx.octree(0), ref)
+    ctx.graph_destroy()

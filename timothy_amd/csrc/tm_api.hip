@@ -41,10 +41,7 @@ tm_status alloc_cells(tm_ctx *c, int64_t n) {
   free_ptr(c->d_ctype_s);
   free_ptr(c->d_phase_s);
   free_ptr(c->d_span);
-  free_ptr(c->d_wn);
-  free_ptr(c->d_wchain);
-  free_ptr(c->d_range);
-  free_ptr(c->d_delta);
+  free_ptr(c->d_leaf);
   free_ptr(c->d_ncount);
   free_ptr(c->d_qstar);
   free_ptr(c->d_dens);
@@ -54,8 +51,6 @@ tm_status alloc_cells(tm_ctx *c, int64_t n) {
   free_ptr(c->d_fy);
   free_ptr(c->d_fz);
   free_ptr(c->d_out);
-  free_ptr(c->d_split);
-  free_ptr(c->d_parent);
   free_ptr(c->d_pos_o);
   free_ptr(c->d_aux_o);
   free_ptr(c->d_nbr);
@@ -69,12 +64,12 @@ tm_status alloc_cells(tm_ctx *c, int64_t n) {
       {(void **)&c->d_key, 8},      {(void **)&c->d_key_alt, 8},  {(void **)&c->d_val_alt, 4},
       {(void **)&c->d_perm, 4},     {(void **)&c->d_code, 16},    {(void **)&c->d_pos, 32},    {(void **)&c->d_posf, 16},
       {(void **)&c->d_young_s, 4},  {(void **)&c->d_ctype_s, 4},
-      {(void **)&c->d_phase_s, 4},  {(void **)&c->d_span, 4},
-      {(void **)&c->d_wn, 32},      {(void **)&c->d_wchain, 4},     {(void **)&c->d_range, 8},    {(void **)&c->d_delta, 4},    {(void **)&c->d_ncount, 4},
+      {(void **)&c->d_phase_s, 4},  {(void **)&c->d_span, 4},     {(void **)&c->d_leaf, 16},
+      {(void **)&c->d_ncount, 4},
       {(void **)&c->d_qstar, 4},    {(void **)&c->d_dens, 8},     {(void **)&c->d_v, 8},
       {(void **)&c->d_mind, 8},     {(void **)&c->d_fx, 8},       {(void **)&c->d_fy, 8},
-      {(void **)&c->d_fz, 8},       {(void **)&c->d_out, 48},     {(void **)&c->d_split, 4},
-      {(void **)&c->d_parent, 8},   {(void **)&c->d_pos_o, 32},   {(void **)&c->d_aux_o, 16},
+      {(void **)&c->d_fz, 8},       {(void **)&c->d_out, 48},     {(void **)&c->d_pos_o, 32},
+      {(void **)&c->d_aux_o, 16},
   };
   for (auto &a : list) {
     if (hipMalloc(a.p, a.bytes * (size_t)cap) != hipSuccess) {
@@ -309,6 +304,7 @@ void tm_destroy(tm_ctx *c) {
   free_ptr(c->d_ctype_s);
   free_ptr(c->d_phase_s);
   free_ptr(c->d_span);
+  free_ptr(c->d_leaf);
   free_ptr(c->d_wn);
   free_ptr(c->d_wchain);
   free_ptr(c->d_range);
@@ -356,6 +352,7 @@ void tm_destroy(tm_ctx *c) {
   free_ptr(c->d_didx);
   free_ptr(c->d_drange);
   free_ptr(c->d_vtk);
+  free_ptr(c->d_bvh);
   if (c->h_flags) (void)hipHostFree(c->h_flags);
   if (c->ev0) (void)hipEventDestroy(c->ev0);
   if (c->ev1) (void)hipEventDestroy(c->ev1);
@@ -811,6 +808,7 @@ tm_status capture(tm_ctx *c, tm_precision p) {
   }
   if (e != hipSuccess) return tm_fail(c, TM_ERR_HIP, std::string("hipStreamEndCapture: ") + hipGetErrorString(e));
   c->graph = g;
+  c->graph_tree = c->tree_valid;
   TM_HIP(c, hipGraphInstantiate(&c->gexec, g, nullptr, nullptr, 0));
   c->graph_prec = p;
   return TM_OK;
@@ -927,6 +925,7 @@ tm_status tm_graph_launch(tm_ctx *c) {
   if (!c) return TM_ERR_INVALID;
   if (!c->gexec) return tm_fail(c, TM_ERR_STATE, "no captured graph");
   TM_HIP(c, hipGraphLaunch(c->gexec, c->stream));
+  c->tree_valid = c->graph_tree;
   TM_TRY(check_flags(c));
   if (c->h_flags[1] > (unsigned)c->nbr_alloc) {
     // a cell outgrew the captured lists (and a captured move moved nothing):
@@ -954,8 +953,9 @@ tm_status tm_autotune(tm_ctx *c, tm_precision p, char *buf, size_t buflen) {
   // A candidate replaces the current shape only when it is faster by more
   // than KEEP (run-to-run noise must not flip a near tie).
   constexpr double KEEP = 0.02;
-  // neighbour walk workgroup and the tree window it stages in LDS
-  const int nb0 = c->nbr_block, win0 = c->walk_window;
+  // per-lane walk: workgroup and the tree window it stages in LDS
+  const int nb0 = c->nbr_block, win0 = c->walk_window, coop0 = c->walk_coop, f0 = c->walk_f32;
+  c->walk_coop = 0;
   int best_nb = nb0, best_win = win0;
   double best_t = 1e30, cur_t = 1e30;
   const int shapes[][2] = {{64, 0}, {128, 0}, {256, 0}, {256, 512}, {256, 1024}, {256, 1280}, {256, 2048}};
@@ -979,21 +979,9 @@ tm_status tm_autotune(tm_ctx *c, tm_precision p, char *buf, size_t buflen) {
   }
   c->nbr_block = best_nb;
   c->walk_window = best_win;
-  // that shape against one union walk per wave (same results)
-  {
-    double tl = 0, tc = 0;
-    TM_TRY(tm_time_stage(c, TM_STAGE_NEIGHBORS, p, 1, 3, &tl));
-    const int c0 = c->walk_coop;
-    c->walk_coop = 1;
-    TM_TRY(tm_time_stage(c, TM_STAGE_NEIGHBORS, p, 1, 3, &tc));
-    snprintf(line, sizeof(line), "trial neighbors walk_coop=0 ms=%.4f\ntrial neighbors walk_coop=1 walk_coop_ratio=%d ms=%.4f\n",
-             tl, c->walk_coop_ratio, tc);
-    rep += line;
-    c->walk_coop = c0 ? (tl * (1.0 + KEEP) < tc ? 0 : 1) : (tc * (1.0 + KEEP) < tl ? 1 : 0);
-  }
   // that shape with the FP32 candidate screening on and off (same results)
+  double lane_t = 0;
   {
-    const int f0 = c->walk_f32;
     double t[2] = {0, 0};
     for (int k = 0; k < 2; ++k) {
       c->walk_f32 = k == 0 ? f0 : !f0;
@@ -1001,7 +989,23 @@ tm_status tm_autotune(tm_ctx *c, tm_precision p, char *buf, size_t buflen) {
       snprintf(line, sizeof(line), "trial neighbors walk_f32=%d ms=%.4f\n", c->walk_f32, t[k]);
       rep += line;
     }
-    c->walk_f32 = t[1] * (1.0 + KEEP) < t[0] ? !f0 : f0;
+    const bool other = t[1] * (1.0 + KEEP) < t[0];
+    c->walk_f32 = other ? !f0 : f0;
+    lane_t = t[other ? 1 : 0];
+  }
+  // that walk against one walk per wave, which screens in FP32 (same results)
+  {
+    const int f = c->walk_f32;
+    double tc = 0;
+    c->walk_coop = 1;
+    c->walk_f32 = 1;
+    TM_TRY(tm_time_stage(c, TM_STAGE_NEIGHBORS, p, 1, 3, &tc));
+    snprintf(line, sizeof(line),
+             "trial neighbors walk_coop=0 ms=%.4f\ntrial neighbors walk_coop=1 walk_coop_ratio=%d ms=%.4f\n", lane_t,
+             c->walk_coop_ratio, tc);
+    rep += line;
+    c->walk_coop = coop0 && f0 ? (lane_t * (1.0 + KEEP) < tc ? 0 : 1) : (tc * (1.0 + KEEP) < lane_t ? 1 : 0);
+    if (!c->walk_coop) c->walk_f32 = f;
   }
   int &unroll = (p == TM_MIXED) ? c->sph_unroll_mixed : c->sph_unroll_fp64;
   const bool tiles = c->sph_tiles && c->dim == 3;

@@ -1,5 +1,7 @@
 // Build stage: per-colony affine map, 29-bit location codes, Morton order,
-// PR-octree leaf octants and the radix tree the neighbour walk descends.
+// PR-octree leaf octants and the tree of boxes over them that the neighbour
+// walk descends; on demand (the per-lane walks, the emitted octree) the radix
+// tree.
 //
 // Reference: octbuild (src/octree.c:145-207).  The reference inserts cells one
 // by one into a pointer PR-octree (one cell per leaf).  The octree is unique
@@ -285,39 +287,109 @@ __global__ __launch_bounds__(BT) void k_fixties(uint64_t *key, int64_t n, int32_
   }
 }
 
+// maximum over each row of 16 lanes, all active, in all of them
+__device__ __forceinline__ uint32_t row_max(uint32_t v) {
+#pragma unroll
+  for (int o = 8; o >= 1; o >>= 1) v = max(v, (uint32_t)__shfl_xor((int)v, o, 16));
+  return v;
+}
+
+// A region's bounds as maxima, so that unions of regions are maxima too: the
+// complement of the lower corner and the upper corner; an empty one is all 0.
+struct Bounds {
+  uint32_t nlx, nly, nlz, hx, hy, hz;
+};
+__device__ __forceinline__ void put_node(BvhNode *node, const Bounds &b) {
+  uint4 *const w = reinterpret_cast<uint4 *>(node);
+  w[0] = make_uint4(~b.nlx, ~b.nly, ~b.nlz, b.hx - ~b.nlx);
+  w[1] = make_uint4(b.hy - ~b.nly, b.hz - ~b.nlz, 0u, 0u);
+}
+__device__ __forceinline__ Bounds get_node(const BvhNode &v) {
+  return Bounds{~v.lx, ~v.ly, ~v.lz, v.lx + v.sx, v.ly + v.sy, v.lz + v.sz};
+}
+__device__ __forceinline__ Bounds row_union(Bounds b) {
+  return Bounds{row_max(b.nlx), row_max(b.nly), row_max(b.nlz), row_max(b.hx), row_max(b.hy), row_max(b.hz)};
+}
+__device__ __forceinline__ Bounds wave_union(Bounds b) {
+  b = row_union(b);
+  auto across = [](uint32_t v) -> uint32_t {
+    v = max(v, (uint32_t)__shfl_xor((int)v, 16, 64));
+    return max(v, (uint32_t)__shfl_xor((int)v, 32, 64));
+  };
+  return Bounds{across(b.nlx), across(b.nly), across(b.nlz), across(b.hx), across(b.hy), across(b.hz)};
+}
+
 // leaf octant exponent: min over the same-colony Morton neighbours of the
 // highest differing code bit (the level at which the PR-octree separates the
 // cell); 29 (the root) for a colony of one.  Flags duplicate codes and splits
 // below node level 3, where the reference shifts by negative counts
-// (src/octree.c:105-107).
-__global__ __launch_bounds__(BT) void k_leaf(const uint4 *__restrict__ code, int64_t n, int32_t *__restrict__ span,
-                                             uint32_t *__restrict__ chain, unsigned int *__restrict__ flags) {
-  int64_t i = (int64_t)blockIdx.x * BT + threadIdx.x;
-  if (i >= n) return;
-  chain[i] = 0;  // counted by k_karras
-  uint4 me = code[i];
-  int best = 99;
-  bool bad = false;
-  if (i > 0) {
-    uint4 o = code[i - 1];
-    if (o.w == me.w) {
-      int b = tm_diffbit(me, o);
-      if (b < 0) bad = true;
-      best = min(best, b);
+// (src/octree.c:105-107).  Also the cell's leaf record (its octant as in a
+// walk record, and the cell) and the boxes of levels 0 and 1 above it: a
+// workgroup takes the 1024 cells of one level-1 node.
+constexpr int LT = 1024;
+__global__ __launch_bounds__(LT) void k_leaf(const uint4 *__restrict__ code, int64_t n, int32_t *__restrict__ span,
+                                             uint4 *__restrict__ leaf, BvhNode *__restrict__ bvh, uint32_t l1,
+                                             unsigned int *__restrict__ flags) {
+  __shared__ uint32_t red[6][64];
+  const int64_t i = (int64_t)blockIdx.x * LT + threadIdx.x;
+  Bounds bd{0u, 0u, 0u, 0u, 0u, 0u};
+  if (i < n) {
+    const uint4 me = code[i];
+    int best = 99;
+    bool bad = false;
+    if (i > 0) {
+      const uint4 o = code[i - 1];
+      if (o.w == me.w) {
+        const int b = tm_diffbit(me, o);
+        if (b < 0) bad = true;
+        best = min(best, b);
+      }
     }
-  }
-  if (i + 1 < n) {
-    uint4 o = code[i + 1];
-    if (o.w == me.w) {
-      int b = tm_diffbit(me, o);
-      if (b < 0) bad = true;
-      best = min(best, b);
+    if (i + 1 < n) {
+      const uint4 o = code[i + 1];
+      if (o.w == me.w) {
+        const int b = tm_diffbit(me, o);
+        if (b < 0) bad = true;
+        best = min(best, b);
+      }
     }
+    if (best == 99) best = 29;
+    if (best <= 1) bad = true;
+    if (bad) atomicOr(flags, (unsigned)TM_FLAG_DEGENERATE);
+    const uint32_t L = best < 0 ? 0u : (uint32_t)best, s = 1u << L, m = ~(s - 1u);
+    span[i] = (int32_t)L;
+    const uint32_t lx = me.x & m, ly = me.y & m, lz = me.z & m;
+    leaf[i] = make_uint4(lx | ((L & 7u) << 29), ly | ((L >> 3) << 29) | 0x80000000u, lz, (uint32_t)i);
+    bd = Bounds{~lx, ~ly, ~lz, lx + s, ly + s, lz + s};
   }
-  if (best == 99) best = 29;
-  if (best <= 1) bad = true;
-  if (bad) atomicOr(flags, (unsigned)TM_FLAG_DEGENERATE);
-  span[i] = best < 0 ? 0 : best;
+  bd = row_union(bd);
+  const uint32_t row = threadIdx.x >> 4;
+  if ((threadIdx.x & 15u) == 0) {
+    if (i < n) put_node(bvh + (i >> 4), bd);
+    red[0][row] = bd.nlx;
+    red[1][row] = bd.nly;
+    red[2][row] = bd.nlz;
+    red[3][row] = bd.hx;
+    red[4][row] = bd.hy;
+    red[5][row] = bd.hz;
+  }
+  __syncthreads();
+  if (threadIdx.x < 64) {
+    const uint32_t t = threadIdx.x;
+    const Bounds u = wave_union(Bounds{red[0][t], red[1][t], red[2][t], red[3][t], red[4][t], red[5][t]});
+    if (t == 0) put_node(bvh + l1 + blockIdx.x, u);
+  }
+}
+
+// a level of the tree of boxes from the one below: one wave per node, over at
+// most 64 of its nchild children
+__global__ __launch_bounds__(64) void k_bvh_up(const BvhNode *__restrict__ child, uint32_t nchild,
+                                               BvhNode *__restrict__ node) {
+  const uint32_t i = blockIdx.x * 64 + threadIdx.x;
+  Bounds b{0u, 0u, 0u, 0u, 0u, 0u};
+  if (i < nchild) b = get_node(child[i]);
+  b = wave_union(b);
+  if (threadIdx.x == 0) put_node(node + blockIdx.x, b);
 }
 
 // Karras (2012) radix tree over (colony, Morton) keys: internal node i's key
@@ -464,6 +536,11 @@ __global__ __launch_bounds__(BT) void k_wnodes(const uint4 *__restrict__ code, c
   put_wnode(code, span, delta, n, k, f, l, pos, wn);
 }
 
+__global__ __launch_bounds__(BT) void k_clear_chain(uint32_t *__restrict__ chain, int64_t n) {
+  const int64_t i = (int64_t)blockIdx.x * BT + threadIdx.x;
+  if (i < n) chain[i] = 0u;
+}
+
 __global__ void k_zero_u32(unsigned int *p, int n) {
   int i = threadIdx.x;
   if (i < n) p[i] = 0;
@@ -475,6 +552,7 @@ tm_status tm_run_build(tm_ctx *c) {
   const int64_t n = c->n;
   if (c->stage < 1) return tm_fail(c, TM_ERR_STATE, "tm_build before tm_upload");
   c->moved = false;  // the sorted records are read afresh from the cells
+  c->tree_valid = false;
   c->sums_valid = false;
   if (n == 0) {
     c->stage = 2;
@@ -500,9 +578,42 @@ tm_status tm_run_build(tm_ctx *c) {
                                              c->d_posf, c->d_young_s, c->d_ctype_s, c->d_phase_s);
   k_fixties<<<tm_blocks(n, BT), BT, 0, st>>>(c->d_key, n, c->d_perm, c->d_code, c->d_pos, c->d_posf,
                                               c->d_young_s, c->d_ctype_s, c->d_phase_s, c->d_flags);
-  k_leaf<<<tm_blocks(n, BT), BT, 0, st>>>(c->d_code, n, c->d_span, c->d_wchain, c->d_flags);
+  const Bvh t = bvh_of(n);
+  TM_TRY(tm_ensure(c, &c->d_bvh, c->cap_bvh, t.total, "tree of boxes"));
+  k_leaf<<<tm_blocks(n, LT), LT, 0, st>>>(c->d_code, n, c->d_span, c->d_leaf, c->d_bvh, t.l1, c->d_flags);
+  if (n > 1 << 16) k_bvh_up<<<t.l3 - t.l2, 64, 0, st>>>(c->d_bvh + t.l1, t.l2 - t.l1, c->d_bvh + t.l2);
+  if (n > 1 << 22) k_bvh_up<<<t.total - t.l3, 64, 0, st>>>(c->d_bvh + t.l2, t.l3 - t.l2, c->d_bvh + t.l3);
   TM_HIP(c, hipGetLastError());
-  // radix tree
+  c->stage = 2;
+  return TM_OK;
+}
+
+tm_status tm_ensure_tree(tm_ctx *c) {
+  const int64_t n = c->n;
+  if (c->tree_valid || n == 0) return TM_OK;
+  hipStream_t st = c->stream;
+  if (c->cap_tree < n) {
+    const int64_t cap = n + (n >> 4) + 64;
+    struct A {
+      void **p;
+      size_t bytes;
+    } list[] = {{(void **)&c->d_wn, 32},   {(void **)&c->d_wchain, 4}, {(void **)&c->d_range, 8},
+                {(void **)&c->d_delta, 4}, {(void **)&c->d_split, 4},  {(void **)&c->d_parent, 8}};
+    c->cap_tree = 0;
+    for (auto &a : list) {
+      if (*a.p) (void)hipFree(*a.p);
+      *a.p = nullptr;
+    }
+    for (auto &a : list)
+      if (hipMalloc(a.p, a.bytes * (size_t)cap) != hipSuccess) {
+        *a.p = nullptr;
+        return tm_fail(c, TM_ERR_NOMEM, "hipMalloc failed for the radix tree");
+      }
+    c->cap_tree = cap;
+  }
+  int cb = 0;
+  while ((1ll << cb) < c->ncol) ++cb;
+  k_clear_chain<<<tm_blocks(n, BT), BT, 0, st>>>(c->d_wchain, n);
   if (n > 1)
     k_karras<<<tm_blocks(n - 1, BT), BT, 0, st>>>(c->d_code, c->d_key, n, cb, c->d_range, c->d_delta, c->d_split,
                                                    c->d_wchain);
@@ -511,6 +622,6 @@ tm_status tm_run_build(tm_ctx *c) {
   k_wnodes<<<tm_blocks(2 * n - 1, BT), BT, 0, st>>>(c->d_code, c->d_span, c->d_range, c->d_delta, c->d_col_off,
                                                      c->d_wchain, n, c->d_wn, c->d_flags);
   TM_HIP(c, hipGetLastError());
-  c->stage = 2;
+  c->tree_valid = true;
   return TM_OK;
 }

@@ -52,6 +52,23 @@ struct TypeDev {
   float hinv_f;
 };
 
+// A node of the tree of boxes over the Morton order: the union of its cells'
+// leaf octants, as lower corner and sides in codes.  Level 0 holds 16
+// consecutive cells per node, each level above 64 nodes of the one below, up
+// to the level at which one node holds all cells (levels above it are not
+// built, nor read).
+struct BvhNode {
+  uint32_t lx, ly, lz, sx, sy, sz, pad0, pad1;
+};
+// where the levels start (level 0 at 0), and the nodes in all
+struct Bvh {
+  uint32_t l1, l2, l3, total;
+};
+inline Bvh bvh_of(int64_t n) {
+  const uint32_t n0 = (uint32_t)((n + 15) >> 4), n1 = (uint32_t)((n + 1023) >> 10), n2 = (uint32_t)((n + 65535) >> 16);
+  return Bvh{n0, n0 + n1, n0 + n1 + n2, n0 + n1 + n2 + (uint32_t)((n + 4194303) >> 22)};
+}
+
 struct tm_ctx {
   int device = 0;
   hipStream_t stream = nullptr;
@@ -116,8 +133,13 @@ struct tm_ctx {
   float *d_young_s = nullptr;
   int32_t *d_ctype_s = nullptr, *d_phase_s = nullptr;
   int32_t *d_span = nullptr;
+  uint4 *d_leaf = nullptr;     // leaf octant (as in a walk record) and cell
+  BvhNode *d_bvh = nullptr;    // the tree of boxes (see BvhNode)
+  int64_t cap_bvh = 0;
 
-  // radix tree
+  // radix tree, made on demand (tm_ensure_tree): tree_valid while it is that
+  // of the last build
+  bool tree_valid = false;
   // the walk's tree: every colony's nodes in its descending pre-order (see
   // tm_build.hip), and the counts their slots are computed from
   uint4 *d_wn = nullptr;
@@ -132,7 +154,7 @@ struct tm_ctx {
   int64_t cap_octcnt = 0;
   char *d_octout = nullptr;
   int64_t cap_octout = 0;  // bytes
-  int64_t cap_tree_aux = 0;
+  int64_t cap_tree = 0;  // cells the radix tree's arrays hold
 
   // neighbours: slot k of cell p at nbr[tm_slot(p, k, nbr_alloc)]
   uint32_t *d_nbr = nullptr;
@@ -151,8 +173,8 @@ struct tm_ctx {
   uint16_t *d_tile_cell = nullptr;  // per tile: cell offset of each rank (longest list first)
   uint16_t *d_nbr16 = nullptr;      // slot k of rank r of tile g at tm_nbr16_at(g*TS + r, k, nbr_alloc)
   int tile_width = TM_TILE;         // cells per tile for the next tile build: 128, 256 or 512
-  int walk_coop = 0;                // 1: one union walk per wave (see k_neighbors)
-  int walk_coop_ratio = 64;         // union box volume / mean cell box volume above which a wave walks per lane
+  int walk_coop = 1;                // 1: one walk per wave for its cells together (see k_union)
+  int walk_coop_ratio = 64;         // its boxes' volume / mean cell box volume above which a wave's cells are parted
   int tiles_ts = 0;                 // cells per tile of the tiles as built (0: none)
   int tile_lds_ts = 0;              // the tile width tile_lds was sized for
   int64_t cap_tile_idx = 0, cap_tile_cnt = 0, cap_tile_cell = 0, cap_nbr16 = 0;
@@ -211,6 +233,7 @@ struct tm_ctx {
   hipGraphExec_t gexec = nullptr;
   tm_precision graph_prec = TM_FP64;
   bool graph_loop = false;     // the captured step also moves the cells
+  bool graph_tree = false;     // the captured step makes the radix tree
   tm_move graph_move{};        // its parameters
   uint8_t *graph_removecell = nullptr;
 };
@@ -248,6 +271,8 @@ tm_status tm_ensure(tm_ctx *c, T **p, int64_t &cap, int64_t need, const char *wh
 tm_status tm_sort_pairs(tm_ctx *c, uint64_t *keys, int32_t *vals, int64_t n, int lo_bit);
 tm_status tm_scan_u32(tm_ctx *c, const uint32_t *in, uint32_t *out, int64_t n);
 tm_status tm_run_build(tm_ctx *c);
+// the radix tree of the last build (the per-lane walks and the emitted octree)
+tm_status tm_ensure_tree(tm_ctx *c);
 tm_status tm_run_neighbors(tm_ctx *c, bool check);
 tm_status tm_run_tiles(tm_ctx *c, bool check);
 tm_status tm_run_sph(tm_ctx *c, tm_precision prec);

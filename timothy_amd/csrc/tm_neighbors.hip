@@ -1,7 +1,9 @@
-// Neighbour stage: one lane per cell walks its colony's radix tree with the
-// reference's query box and strict overlap test, visiting leaf octants in
-// descending Morton key -- the order the reference's LIFO DFS pops them
-// (children pushed 0..7, src/potential.c:111-131).  The tree is read in the
+// Neighbour stage: the cells whose leaf octants overlap a cell's query box (the
+// reference's, with its strict overlap test), visited in descending Morton
+// key -- the order the reference's LIFO DFS pops them (children pushed 0..7,
+// src/potential.c:111-131).  By default a wave looks for the candidates of
+// all its cells together (k_union, below).  With walk_coop or walk_f32 off one
+// lane per cell walks its colony's radix tree (k_neighbors), read in the
 // walk's own pre-order (built by k_wnodes): one 16-byte record per visited
 // node, the next slot after a hit and the escape slot after a miss.
 //
@@ -47,6 +49,191 @@ __device__ __forceinline__ double pot_fp64(double4 P, float yp, double4 Q, float
   return (2.0 * (xc * xc) / (5.0 * D)) * sqrt((s1 * s2) / (s1 + s2)) + area * 0.1;
 }
 
+// reference squared distance, src/potential.c:49 order (contraction is off)
+__device__ __forceinline__ double dist2_fp64(const double4 &P, const double4 &Q) {
+  const double dx = P.x - Q.x, dy = P.y - Q.y, dz = P.z - Q.z;
+  return (dx * dx + dy * dy) + dz * dz;
+}
+
+// lane moves within the wave (DPP): the lanes without a source get `old`
+template <int CTRL, int ROWS = 0xf>
+__device__ __forceinline__ uint32_t dpp(uint32_t old, uint32_t v) {
+  return (uint32_t)__builtin_amdgcn_update_dpp((int)old, (int)v, CTRL, ROWS, 0xf, false);
+}
+// maximum over the wave's 64 lanes, all active
+__device__ __forceinline__ uint32_t wave_max_u32(uint32_t v) {
+  v = max(v, dpp<0x111>(0u, v));  // row_shr 1, 2, 4, 8
+  v = max(v, dpp<0x112>(0u, v));
+  v = max(v, dpp<0x114>(0u, v));
+  v = max(v, dpp<0x118>(0u, v));
+  v = max(v, dpp<0x142, 0xa>(0u, v));  // row_bcast 15 into rows 1 and 3
+  v = max(v, dpp<0x143, 0xc>(0u, v));  // row_bcast 31 into rows 2 and 3
+  return (uint32_t)__builtin_amdgcn_readlane((int)v, 63);
+}
+// maximum over each row of 16 lanes, in all of them
+__device__ __forceinline__ uint32_t row_max_u32(uint32_t v) {
+  v = max(v, dpp<0x128>(0u, v));  // row_ror 8, 4, 2, 1
+  v = max(v, dpp<0x124>(0u, v));
+  v = max(v, dpp<0x122>(0u, v));
+  return max(v, dpp<0x121>(0u, v));
+}
+// set bits of m below this lane
+__device__ __forceinline__ uint32_t mbcnt64(uint64_t m) {
+  return __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
+}
+// the value of the row's first lane
+__device__ __forceinline__ float row_first(float v) {
+  return __uint_as_float(dpp<0x150>(0u, __float_as_uint(v)));  // row_newbcast 0
+}
+// v[g] of row b of lanes becomes v[b] of row g
+__device__ __forceinline__ void transpose4(uint32_t v[4]) {
+#pragma unroll
+  for (int k = 0; k < 2; ++k) {
+    const auto r = __builtin_amdgcn_permlane32_swap(v[k], v[k + 2], false, false);
+    v[k] = r[0];
+    v[k + 2] = r[1];
+  }
+#pragma unroll
+  for (int k = 0; k < 4; k += 2) {
+    const auto r = __builtin_amdgcn_permlane16_swap(v[k], v[k + 1], false, false);
+    v[k] = r[0];
+    v[k + 1] = r[1];
+  }
+}
+// mean over the lanes that are in
+__device__ __forceinline__ float wave_mean(float v, bool in) {
+  const uint64_t m = __ballot(in);
+  v = in ? v : 0.f;
+#pragma unroll
+  for (int o = 32; o >= 1; o >>= 1) v += __shfl_xor(v, o, 64);
+  return v / (float)__builtin_popcountll(m);
+}
+// minimum over the wave (no NaN)
+__device__ __forceinline__ double wave_min_f64(double v) {
+#pragma unroll
+  for (int o = 32; o >= 1; o >>= 1) v = fmin(v, __shfl_xor(v, o, 64));
+  return v;
+}
+// orders the wave's LDS accesses before and after it
+__device__ __forceinline__ void wave_lds_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// A cell's query box as mx - 1 and mx - mn - 1 per axis.  The strict overlap
+// of [mn, mx] with a region [lo, lo + s) on one axis, mx > lo and
+// mn < lo + s, is (mx - 1 - lo) < (mx - mn - 1) + s in 32-bit unsigned
+// arithmetic: the left side wraps past every right side when mx <= lo, and
+// otherwise the two compares agree (mx >= mn: both codes are the same
+// monotone map of x - h and x + h).
+struct QBox {
+  uint32_t ex0, ex1, ex2, dm0, dm1, dm2;
+};
+// query box, src/octree.c:246-266: ((x - h) - shift) / scale * 2^29
+__device__ __forceinline__ QBox query_box(const double4 &P, double h, const double4 &A) {
+  const uint32_t mn0 = box_code(P.x - h, A.x, A.w), mx0 = box_code(P.x + h, A.x, A.w);
+  const uint32_t mn1 = box_code(P.y - h, A.y, A.w), mx1 = box_code(P.y + h, A.y, A.w);
+  const uint32_t mn2 = box_code(P.z - h, A.z, A.w), mx2 = box_code(P.z + h, A.z, A.w);
+  return QBox{mx0 - 1u, mx1 - 1u, mx2 - 1u, mx0 - mn0 - 1u, mx1 - mn1 - 1u, mx2 - mn2 - 1u};
+}
+__device__ __forceinline__ float volume(const QBox &b) {
+  return (float)(b.dm0 + 1u) * (float)(b.dm1 + 1u) * (float)(b.dm2 + 1u);
+}
+// Morton order of two code triples (z, y, x within a level): the axis with the
+// highest differing bit decides
+__device__ __forceinline__ bool morton_less3(uint32_t ax, uint32_t ay, uint32_t az, uint32_t bx, uint32_t by,
+                                             uint32_t bz) {
+  const uint32_t dx = ax ^ bx, dy = ay ^ by, dz = az ^ bz;
+  const bool y = (dz < dy) & (dz < (dz ^ dy));
+  const uint32_t d = y ? dy : dz;
+  const bool x = (d < dx) & (d < (d ^ dx));
+  return x ? ax < bx : y ? ay < by : az < bz;
+}
+// a region: lower corner and sides in codes
+struct Octant {
+  uint32_t lx, ly, lz, sx, sy, sz;
+};
+__device__ __forceinline__ bool hits(const Octant &c, const QBox &b) {
+  return (b.ex0 - c.lx < b.dm0 + c.sx) & (b.ex1 - c.ly < b.dm1 + c.sy) & (b.ex2 - c.lz < b.dm2 + c.sz);
+}
+// the region of a tree record
+__device__ __forceinline__ Octant octant(const uint4 &a) {
+  const uint32_t sx = 1u << ((a.x >> 29) | (((a.y >> 29) & 3u) << 3));
+  return Octant{a.x & 0x1FFFFFFFu, a.y & 0x1FFFFFFFu,         a.z & 0x1FFFFFFFu,
+                sx,                sx >> ((a.z >> 30) & 1u), sx >> ((a.z >> 29) & 1u)};
+}
+// the same of a leaf record (a cube)
+__device__ __forceinline__ Octant leaf_octant(const uint4 &a) {
+  const uint32_t s = 1u << ((a.x >> 29) | (((a.y >> 29) & 3u) << 3));
+  return Octant{a.x & 0x1FFFFFFFu, a.y & 0x1FFFFFFFu, a.z & 0x1FFFFFFFu, s, s, s};
+}
+
+// the FP32 screening of one cell (see k_neighbors): thresholds, tin a further
+// in_by inwards
+struct Screen {
+  float tin, tout, beta;
+};
+__device__ __forceinline__ Screen screen_of(const double4 &A, double cut2, double in_by) {
+  Screen s;
+  const double K = 1.7321 * (A.w * 1.2e-7 + 1e-44);
+  const double hc = sqrt(cut2);
+  double ti = (hc * (1.0 - 1e-15) - (K + in_by)) / (1.0 + 1e-7);
+  ti = ti > 0.0 ? ti * ti / (1.0 + 3e-7) - 1e-44 : -1.0;
+  // a threshold outside FP32's normal range decides nothing
+  s.tin = (ti >= 1e-30 && ti <= 1e38) ? (float)(ti * (1.0 - 1e-6)) : -1.0f;
+  double to = (hc * (1.0 + 1e-15) + K) / (1.0 - 1e-7);
+  to = to * to * (1.0 + 3e-7) + 1e-44;
+  // (overflow gives inf and NaN stays NaN: both decide nothing; below
+  // FP32's normal range the threshold is raised, which only widens the
+  // band read in FP64)
+  s.tout = to < 1e-30 ? 1e-30f : (float)(to * (1.0 + 1e-6));
+  s.beta = (float)((40500.0 * K * K + 1e-37) * (1.0 + 1e-6));
+  return s;
+}
+
+// What every walk does last.  Pad each list to the longest one of its 64-cell
+// slot group (this wave) with cell index n, the far-away stand-in record the
+// build places after the cells: the pair kernels then read whole slot rows
+// without per-lane tests, and a stand-in pair contributes exactly zero to the
+// mixed sums (rows are written wave-wide, one 256-byte row per step).  Then
+// the count, mindist, the last candidate and v, the potential with it
+// (src/potential.c:124 assigns it per candidate; 0 beyond the cutoff and with
+// no candidate); the records are read again here rather than kept through
+// the walk.
+template <int NW>
+__device__ __forceinline__ void finish(int64_t p, bool live, uint32_t cnt, int32_t qs, double md2,
+                                       const double4 *__restrict__ pos, const int32_t *__restrict__ ctype_s,
+                                       const float *__restrict__ young_s, const TypeDev *__restrict__ types, int64_t n,
+                                       int64_t cap, uint32_t *__restrict__ nbr, uint32_t *__restrict__ count,
+                                       double *__restrict__ mindist, int32_t *__restrict__ qstar,
+                                       double *__restrict__ vout, unsigned int *__restrict__ flags) {
+  const uint32_t used = min(cnt, (uint32_t)cap);
+  uint32_t g = used, lo = live ? used : 0xFFFFFFFFu;
+#pragma unroll
+  for (int o = 32; o >= 1; o >>= 1) {
+    g = max(g, (uint32_t)__shfl_xor((int)g, o, 64));
+    lo = min(lo, (uint32_t)__shfl_xor((int)lo, o, 64));
+  }
+  if constexpr (NW > 1) {  // the group's cells lie in NW waves
+    __shared__ uint32_t most[NW];
+    if ((threadIdx.x & 63u) == 0) most[threadIdx.x >> 6] = g;
+    __syncthreads();
+#pragma unroll
+    for (int w = 0; w < NW; ++w) g = max(g, most[w]);
+  }
+  for (uint32_t k = lo; k < g; ++k)
+    if (live && k >= used) nbr[tm_slot(p, k, cap)] = (uint32_t)n;
+  if (!live) return;
+  count[p] = cnt;
+  mindist[p] = qs >= 0 ? sqrt(md2) : 1.7976931348623157e308;
+  qstar[p] = qs;
+  const double4 P = pos[p];
+  const double4 Qs = qs >= 0 ? pos[qs] : P;
+  vout[p] = qs >= 0 ? pot_fp64(P, young_s[p], Qs, young_s[qs], types[ctype_s[p]].h) : 0.0;
+  if (cnt > cap) atomicMax(flags + 1, cnt);
+}
+
 // WIN > 0: the workgroup first copies WIN consecutive slots of the
 // pre-ordered tree, centred on the leaves of its own cells, into LDS; its
 // walks read the nodes inside that window from LDS and the rest from memory.
@@ -54,12 +241,6 @@ __device__ __forceinline__ double pot_fp64(double4 P, float yp, double4 Q, float
 // share many nodes near their own leaves (about half of all visits fall in
 // 1024 slots around 256 cells), and a read from LDS spares the texture path
 // the per-lane gather that bounds the walk.
-// reference squared distance, src/potential.c:49 order (contraction is off)
-__device__ __forceinline__ double dist2_fp64(const double4 &P, const double4 &Q) {
-  const double dx = P.x - Q.x, dy = P.y - Q.y, dz = P.z - Q.z;
-  return (dx * dx + dy * dy) + dz * dz;
-}
-
 // F32: candidates are screened with their FP32 positions relative to the
 // colony's origin (16 bytes per candidate instead of 32); only a candidate
 // whose FP32 distance cannot decide the cutoff, or that may hold the minimum
@@ -86,25 +267,7 @@ __device__ __forceinline__ double dist2_fp64(const double4 &P, const double4 &Q)
 // that place (the newcomer, or the one it displaces) is read in FP64 at once
 // when it is still within reach of the smallest (rare), and the smallest is
 // read in FP64 at the end.
-// COOP: each wave (BS = 64) first walks the tree once for the union of its
-// cells' query boxes, reading the pre-ordered slots 64 at a time (one
-// coalesced load for all lanes, where the per-lane walk gathers one record
-// per lane per node).  A slot is visited when no missed internal node before
-// it in the window skips it (a prefix maximum of the missed nodes' escape
-// slots); the walk continues after the window or at the largest escape.
-// The leaves it finds that overlap the union box are, in visit order, the
-// wave's union candidates: every leaf whose octant overlaps a cell's own box
-// overlaps the union box, and its ancestors contain its octant, so a cell's
-// candidates are exactly the union candidates that overlap its own box, in
-// the same order.  They are staged in LDS (CB at a time with their FP32 or
-// FP64 records) and each lane takes its own from there -- its box test over
-// 64 staged candidates at a time as a bit mask, then the set bits in order.
-// A wave whose cells span two colonies, or whose union box is more than
-// coop_ratio times its cells' mean box volume (a Morton jump: the union would
-// hold far more candidates than any cell), walks per lane as without COOP.
-constexpr int CB = 128;  // union candidates staged per wave
-
-template <int BS, int WIN, bool F32, bool COOP>
+template <int BS, int WIN, bool F32>
 __global__ __launch_bounds__(BS) void k_neighbors(const double4 *__restrict__ pos, const float4 *__restrict__ posf,
                                                   const uint4 *__restrict__ code,
                                                   const int32_t *__restrict__ ctype_s,
@@ -116,8 +279,7 @@ __global__ __launch_bounds__(BS) void k_neighbors(const double4 *__restrict__ po
                                                   uint32_t *__restrict__ nbr,
                                                   uint32_t *__restrict__ count, double *__restrict__ mindist,
                                                   int32_t *__restrict__ qstar, double *__restrict__ vout,
-                                                  unsigned int *__restrict__ flags, float coop_ratio) {
-  static_assert(!COOP || (BS == 64 && WIN == 0), "a cooperative walk takes one wave per workgroup, no window");
+                                                  unsigned int *__restrict__ flags) {
   const int64_t cell = tm_xcd_block() * BS + threadIdx.x;
   const bool live = cell < n;
   const int64_t p = live ? cell : n - 1;  // idle lanes only join the padding step below
@@ -128,17 +290,7 @@ __global__ __launch_bounds__(BS) void k_neighbors(const double4 *__restrict__ po
   const double h = T.h;
   const double cut2 = T.cut2;
   const uint4 *winp = nullptr;
-  // query box, src/octree.c:246-266: ((x - h) - shift) / scale * 2^29
-  const uint32_t mn0 = box_code(P.x - h, A.x, A.w), mx0 = box_code(P.x + h, A.x, A.w);
-  const uint32_t mn1 = box_code(P.y - h, A.y, A.w), mx1 = box_code(P.y + h, A.y, A.w);
-  const uint32_t mn2 = box_code(P.z - h, A.z, A.w), mx2 = box_code(P.z + h, A.z, A.w);
-  // The strict overlap of [mn, mx] with a node's [lo, lo + s) on one axis,
-  // mx > lo and mn < lo + s, is (mx - 1 - lo) < (mx - mn - 1) + s in 32-bit
-  // unsigned arithmetic: the left side wraps past every right side when
-  // mx <= lo, and otherwise the two compares agree (mx >= mn: both codes
-  // are the same monotone map of x - h and x + h).
-  const uint32_t ex0 = mx0 - 1u, ex1 = mx1 - 1u, ex2 = mx2 - 1u;
-  const uint32_t dm0 = mx0 - mn0 - 1u, dm1 = mx1 - mn1 - 1u, dm2 = mx2 - mn2 - 1u;
+  const QBox box = query_box(P, h, A);
   // the window of slots staged in LDS: around the leaf slot of the
   // workgroup's middle cell, 2 s + 2 (e - k) for cell k of colony [s, e]
   // (up to its ancestor count), within the tree's 2 n - 1 slots
@@ -178,19 +330,10 @@ __global__ __launch_bounds__(BS) void k_neighbors(const double4 *__restrict__ po
     pfx = (float)(P.x - A.x);
     pfy = (float)(P.y - A.y);
     pfz = (float)(P.z - A.z);
-    const double K = 1.7321 * (A.w * 1.2e-7 + 1e-44);
-    const double hc = sqrt(cut2);
-    double ti = (hc * (1.0 - 1e-15) - K) / (1.0 + 1e-7);
-    ti = ti > 0.0 ? ti * ti / (1.0 + 3e-7) - 1e-44 : -1.0;
-    // a threshold outside FP32's normal range decides nothing
-    tin = (ti >= 1e-30 && ti <= 1e38) ? (float)(ti * (1.0 - 1e-6)) : -1.0f;
-    double to = (hc * (1.0 + 1e-15) + K) / (1.0 - 1e-7);
-    to = to * to * (1.0 + 3e-7) + 1e-44;
-    // (overflow gives inf and NaN stays NaN: both decide nothing; below
-    // FP32's normal range the threshold is raised, which only widens the
-    // band read in FP64)
-    tout = to < 1e-30 ? 1e-30f : (float)(to * (1.0 + 1e-6));
-    beta = (float)((40500.0 * K * K + 1e-37) * (1.0 + 1e-6));
+    const Screen s = screen_of(A, cut2, 0.0);
+    tin = s.tin;
+    tout = s.tout;
+    beta = s.beta;
   }
   // the reference's d2 of candidate q, read in FP64, into the minimum
   auto exact = [&](uint32_t q) -> double {
@@ -236,123 +379,6 @@ __global__ __launch_bounds__(BS) void k_neighbors(const double4 *__restrict__ po
   // issued, so waiting for them does not also wait for the store (vector
   // memory counters retire in order).  Candidates are still taken in visit
   // order.
-  bool coop = false;
-  if constexpr (COOP) {
-    // the wave's union box, over its live cells of one colony
-    const uint32_t lane = threadIdx.x;
-    uint32_t u[6] = {live ? mn0 : ~0u, live ? mn1 : ~0u, live ? mn2 : ~0u, live ? mx0 : 0u, live ? mx1 : 0u,
-                     live ? mx2 : 0u};
-    uint32_t cmin = live ? cid : ~0u, cmax = live ? cid : 0u;
-    float vl = live ? (float)(mx0 - mn0) * (float)(mx1 - mn1) * (float)(mx2 - mn2) : 0.f;
-    float nl = live ? 1.f : 0.f;
-#pragma unroll
-    for (int o = 32; o >= 1; o >>= 1) {
-#pragma unroll
-      for (int a = 0; a < 3; ++a) u[a] = min(u[a], (uint32_t)__shfl_xor((int)u[a], o, 64));
-#pragma unroll
-      for (int a = 3; a < 6; ++a) u[a] = max(u[a], (uint32_t)__shfl_xor((int)u[a], o, 64));
-      cmin = min(cmin, (uint32_t)__shfl_xor((int)cmin, o, 64));
-      cmax = max(cmax, (uint32_t)__shfl_xor((int)cmax, o, 64));
-      vl += __shfl_xor(vl, o, 64);
-      nl += __shfl_xor(nl, o, 64);
-    }
-    const float vu = (float)(u[3] - u[0]) * (float)(u[4] - u[1]) * (float)(u[5] - u[2]);
-    coop = nl > 0.f && cmin == cmax && vu <= coop_ratio * (vl / nl);
-    if (coop) {
-      __shared__ uint4 crec[CB];  // lo codes x, y, z and the cell
-      __shared__ uint4 csz[CB];   // octant sizes x, y, z
-      __shared__ QRec cq[CB];     // the cell's record
-      const uint32_t uex0 = u[3] - 1u, uex1 = u[4] - 1u, uex2 = u[5] - 1u;
-      const uint32_t udm0 = u[3] - u[0] - 1u, udm1 = u[4] - u[1] - 1u, udm2 = u[5] - u[2] - 1u;
-      const uint32_t wbeg = (uint32_t)(2 * col_off[cmin]), wend = (uint32_t)(2 * col_off[cmin + 1] - 1);
-      uint32_t nb = 0;
-      // each lane's candidates among the staged ones, in order
-      auto drain = [&]() {
-        for (uint32_t e = lane; e < nb; e += 64) {
-          if constexpr (F32) cq[e] = posf[crec[e].w];
-          else cq[e] = pos[crec[e].w];
-        }
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-        for (uint32_t b0 = 0; b0 < nb; b0 += 64) {
-          const uint32_t m = min(64u, nb - b0);
-          uint64_t mask = 0;
-          for (uint32_t j = 0; j < m; ++j) {
-            const uint4 r = crec[b0 + j], z = csz[b0 + j];
-            const bool hit = (ex0 - r.x < dm0 + z.x) & (ex1 - r.y < dm1 + z.y) & (ex2 - r.z < dm2 + z.z);
-            mask |= (uint64_t)(hit && live && r.w != (uint32_t)p) << j;
-          }
-          while (mask) {
-            const uint32_t j = (uint32_t)__builtin_ctzll(mask);
-            mask &= mask - 1;
-            const uint32_t q = crec[b0 + j].w;
-            const int64_t slot = visit(q, cq[b0 + j]);
-            if (slot >= 0) nbr[slot] = q;
-          }
-        }
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-        nb = 0;
-      };
-      // the window after this one is loaded with it: taken when the walk
-      // goes on there (no escape past it)
-      uint4 nxt = wbeg + lane < wend ? wn[wbeg + lane] : make_uint4(0u, 0u, 0u, 0u);
-      for (uint32_t cur = wbeg; cur < wend;) {
-        const uint32_t sl = cur + lane;
-        const bool valid = sl < wend;
-        const uint4 a = nxt;
-        nxt = sl + 64u < wend ? wn[sl + 64u] : make_uint4(0u, 0u, 0u, 0u);
-        const uint32_t L = (a.x >> 29) | (((a.y >> 29) & 3u) << 3);
-        const uint32_t lx = a.x & 0x1FFFFFFFu, ly = a.y & 0x1FFFFFFFu, lz = a.z & 0x1FFFFFFFu;
-        const uint32_t sx = 1u << L, sy = sx >> ((a.z >> 30) & 1u), sz = sx >> ((a.z >> 29) & 1u);
-        const bool hitu = (uex0 - lx < udm0 + sx) & (uex1 - ly < udm1 + sy) & (uex2 - lz < udm2 + sz);
-        const bool leaf = (a.y & 0x80000000u) != 0u;
-        const bool miss = valid && !hitu && !leaf;
-        // slots skipped by a missed node earlier in the window
-        uint32_t pm = miss ? a.w : 0u;
-#pragma unroll
-        for (int o = 1; o < 64; o <<= 1) {
-          const uint32_t y = (uint32_t)__shfl_up((int)pm, o, 64);
-          if (lane >= (uint32_t)o) pm = max(pm, y);
-        }
-        uint32_t before = (uint32_t)__shfl_up((int)pm, 1, 64);
-        if (lane == 0) before = 0u;
-        const uint32_t mall = (uint32_t)__shfl((int)pm, 63, 64);
-        const bool visited = valid && before <= sl;
-        // a malformed tree: a visited miss that does not move forward, or a
-        // leaf naming no cell
-        if (__ballot(visited && ((miss && a.w <= sl) || (leaf && a.w >= (uint32_t)n)))) {
-          if (lane == 0) atomicOr(flags, (unsigned)TM_FLAG_WALK);
-          break;
-        }
-        const bool cand = visited && leaf && hitu;
-        const uint64_t cm = __ballot(cand);
-        const uint32_t k = (uint32_t)__builtin_popcountll(cm);
-        if (k) {
-          if (nb + k > (uint32_t)CB) drain();
-          if (cand) {
-            const uint32_t e = nb + (uint32_t)__builtin_popcountll(cm & tm_lanemask_lt());
-            crec[e] = make_uint4(lx, ly, lz, a.w);
-            csz[e] = make_uint4(sx, sy, sz, 0u);
-          }
-          nb += k;
-        }
-        if (mall > cur + 64u) {
-          cur = mall;
-          nxt = cur + lane < wend ? wn[cur + lane] : make_uint4(0u, 0u, 0u, 0u);
-        } else {
-          cur += 64u;
-        }
-      }
-      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-      __builtin_amdgcn_wave_barrier();
-      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-      if (nb) drain();
-      node = end;  // the per-lane walk below has nothing left to do
-    }
-  }
   uint32_t pq = 0xFFFFFFFFu;  // the candidate whose record is in flight
   QRec Qp{};
   while (node < end) {
@@ -369,11 +395,7 @@ __global__ __launch_bounds__(BS) void k_neighbors(const double4 *__restrict__ po
       slot = visit(pq, Qp);
       pq = 0xFFFFFFFFu;
     }
-    const uint32_t L = (a.x >> 29) | (((a.y >> 29) & 3u) << 3);
-    const uint32_t lx = a.x & 0x1FFFFFFFu, ly = a.y & 0x1FFFFFFFu, lz = a.z & 0x1FFFFFFFu;
-    const uint32_t sx = 1u << L, sy = sx >> ((a.z >> 30) & 1u), sz = sx >> ((a.z >> 29) & 1u);
-    // mx > lo and mn < lo + s, as one unsigned compare per axis
-    const bool hit = (ex0 - lx < dm0 + sx) & (ex1 - ly < dm1 + sy) & (ex2 - lz < dm2 + sz);
+    const bool hit = hits(octant(a), box);
     const bool leaf = (a.y & 0x80000000u) != 0u;
     const uint32_t next = (hit || leaf) ? node + 1 : a.w;
     if (next <= node || (leaf && a.w >= (uint32_t)n)) {  // a malformed tree: a well-formed one only moves forward
@@ -393,43 +415,575 @@ __global__ __launch_bounds__(BS) void k_neighbors(const double4 *__restrict__ po
     const int64_t slot = visit(pq, Qp);
     if (slot >= 0) nbr[slot] = pq;
   }
-  // Pad each list to the longest one of its 64-cell slot group (this wave)
-  // with cell index n, the far-away stand-in record the build places after
-  // the cells: the pair kernels then read whole slot rows without per-lane
-  // tests, and a stand-in pair contributes exactly zero to the mixed sums.
-  // (rows are written wave-wide, one 256-byte row per step)
-  const uint32_t used = min(cnt, (uint32_t)cap);
-  uint32_t g = used, lo = live ? used : 0xFFFFFFFFu;
-#pragma unroll
-  for (int o = 32; o >= 1; o >>= 1) {
-    g = max(g, (uint32_t)__shfl_xor((int)g, o, 64));
-    lo = min(lo, (uint32_t)__shfl_xor((int)lo, o, 64));
-  }
-  for (uint32_t k = lo; k < g; ++k)
-    if (live && k >= used) nbr[tm_slot(p, k, cap)] = (uint32_t)n;
-  if (!live) return;
   if constexpr (F32) {
     // the smallest
     if (c1 != 0xFFFFFFFFu) (void)exact(c1);
   }
-  count[p] = cnt;
-  mindist[p] = qs >= 0 ? sqrt(md2) : 1.7976931348623157e308;
-  qstar[p] = qs;
-  // v: the potential with the last candidate visited (src/potential.c:124
-  // assigns it per candidate; 0 beyond the cutoff and with no candidate)
-  // the record of the last candidate, read again here rather than kept
-  // through the walk
-  const double4 Qs = qs >= 0 ? pos[qs] : P;
-  vout[p] = qs >= 0 ? pot_fp64(P, young_s[p], Qs, young_s[qs], h) : 0.0;
-  if (cnt > cap) atomicMax(flags + 1, cnt);
+  finish<1>(p, live, cnt, qs, md2, pos, ctype_s, young_s, types, n, cap, nbr, count, mindist, qstar, vout, flags);
 }
 
-template <int BS, int WIN, bool COOP = false>
+// The cooperative walk: a wave looks once for all cells that any of its own G
+// may take, and its lanes pick theirs from those.  The per-lane walk above
+// reads a tree record per node and lane (257 per cell in the 2M-cell Gaussian
+// colony, 25 K vector instructions per wave of 64 cells); here a wave issues
+// 12 K, and half of its loads fetch 64 consecutive records.
+//
+//   1. The wave's cells are cut in two at the highest Morton step between two
+//      of them, and the union of either part's query boxes is formed (a run of
+//      Morton order often lies in two places; one box over both held 1.7 times
+//      as many candidates, and up to 33 K).  Each row of 16 lanes gets two
+//      boxes the same way.
+//   2. From the top of the tree of boxes (BvhNode) the wave finds the blocks
+//      of 16 cells that overlap the two boxes, 64 nodes per load, then tests
+//      their cells' leaf octants, four blocks per load, in descending Morton
+//      order.  Every leaf that overlaps a cell's own box overlaps its part's
+//      union, and boxes above it contain it, so none is missed.
+//   3. The leaves found (547 per 64 cells at 2M) are staged in LDS, CB at a
+//      time; each row keeps a list of those that overlap its own boxes (about
+//      250; one byte each).
+//   4. The last candidate of each lane (qstar) comes from its row's list, from
+//      the end.
+//   5. The entries within a lane's cutoff: FP32 squared distances of 16
+//      entries to the row's 16 cells as outer products on the matrix cores,
+//      with a margin that covers their rounding; the lane then takes those
+//      marked, in order, with the FP32 screening of the per-lane walk: tin is
+//      taken four code units further in, so that a candidate at most that far
+//      away also overlaps the query box strictly (its code differs from both
+//      corners'); between tin and tout the distance and the octant are
+//      evaluated exactly.  Candidates beyond the cutoff matter only for qstar
+//      and, where a cell has none within, for mindist.
+//   6. mindist: the smallest FP32 distance and the second smallest are kept;
+//      the first is read in FP64, and the cell's list once more where the
+//      second is within reach of it.  A cell with candidates but none within
+//      its cutoff takes the minimum over all of them, the wave's lanes sharing
+//      the work.
+// A group whose cells lie in more places than two boxes serve (its queue full
+// and the boxes more than `ratio` times the cells' own) is taken in parts, cut
+// at the step; a wave's colonies are taken one after another.
+//
+// What bounds it: vector issue (80% of the SIMDs' cycles at 2M cells with the
+// four waves per SIMD that 127 registers allow; the list entries cost 12 K
+// instructions per wave), below about 500 K cells the longest wave, whose
+// cells lie in many places: a wave then takes fewer cells (launch_union).
+// Walk alone, per-lane before and this: 20 K-cell ball 119 and 43 us, 300 K
+// ball 208 and 175 us, 2M Gaussian 1,729 and 858 us, 4M cells in 128 colonies
+// 3,358 and 1,900 us, 3M of two types 3,605 and 1,580 us; the build, which no
+// longer makes the radix tree for it, 168 -> 143, 216 -> 178, 498 -> 367,
+// 872 -> 620 and 718 -> 531 us.  Also measured: the per-lane walk's tree read
+// 64 slots at a time in its pre-order (103 dependent loads per wave against 48
+// here) 450 us of a 1.46 ms walk; distances on the vector unit 5% slower at
+// 2M; blocks of 32 cells 8% more loads.
+constexpr int CB = 255;  // candidates staged at a time (a byte names one; 255 names none)
+// FP32 rounding of |c|^2 + |p|^2 - 2 c.p (five products and sums, operands
+// rounded to 2^-24) stays within 1.5e-6 (|c|^2 + |p|^2): the squares are
+// taken 2^-18 too small
+constexpr float LESS = 1.0f - 0x1p-18f;
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+constexpr int BQ = 320;  // blocks queued (a node's 64 children must fit beside the ratio's)
+constexpr int UC = 512;  // candidates of a wave kept for its cells without a neighbour
+
+template <int G>
+__global__ __launch_bounds__(4096 / G, 4) void k_union(
+    const double4 *__restrict__ pos, const float4 *__restrict__ posf, const uint4 *__restrict__ code,
+    const int32_t *__restrict__ ctype_s, const float *__restrict__ young_s, const uint4 *__restrict__ leaf,
+    const BvhNode *__restrict__ bvh, Bvh tree, const int64_t *__restrict__ col_off, const double4 *__restrict__ aff,
+    const TypeDev *__restrict__ types, int64_t n, int64_t cap, uint32_t *__restrict__ nbr,
+    uint32_t *__restrict__ count, double *__restrict__ mindist, int32_t *__restrict__ qstar,
+    double *__restrict__ vout, unsigned int *__restrict__ flags, uint32_t ratio) {
+  constexpr int NW = 64 / G;     // waves per workgroup
+  constexpr int ROWS = G < 16 ? 1 : G / 16;  // rows of lanes with cells
+  __shared__ uint4 crec_[NW][CB + 1];  // a staged candidate: its octant and cell, later its record and cell
+  // per row of 16 lanes the staged candidates it may take, one byte each
+  __shared__ __align__(16) uint32_t sub_[NW][4 * 64];
+  __shared__ QBox rbox_[NW][2 * ROWS];  // per row its two boxes
+  __shared__ uint32_t queue_[NW][BQ];   // blocks of 16 cells to look into
+  __shared__ uint32_t ucell_[NW][UC];   // the first candidates (cells)
+  const uint32_t lane = threadIdx.x & 63u, row = lane >> 4, wv = threadIdx.x >> 6;
+  uint4 *const crec = crec_[wv];
+  uint32_t *const sub = sub_[wv];
+  QBox *const rbox = rbox_[wv];
+  uint32_t *const queue = queue_[wv];
+  uint32_t *const ucell = ucell_[wv];
+  uint8_t *const sub8 = reinterpret_cast<uint8_t *>(sub);
+  const int64_t cell = tm_xcd_block() * 64 + G * (int64_t)wv + lane;
+  const bool live = lane < (uint32_t)G && cell < n;
+  const int64_t p = live ? cell : n - 1;  // idle lanes only join the wave-wide steps
+  // values used once per group of cells, or rarely, are read again where they
+  // are used rather than held in registers through the walk
+  auto again = [&]() {
+    int64_t v = p;
+    asm volatile("" : "+v"(v));
+    return v;
+  };
+  const uint32_t cid = code[p].w;
+  QBox own;
+  float pfx, pfy, pfz, tin, tout;
+  {
+    const double4 P = pos[p], A = aff[cid];
+    const TypeDev &T = types[ctype_s[p]];
+    own = query_box(P, T.h, A);
+    pfx = (float)(P.x - A.x);
+    pfy = (float)(P.y - A.y);
+    pfz = (float)(P.z - A.z);
+    // tin four code units further in, so that a candidate it accepts also
+    // overlaps the query box; none is accepted where the coordinates are so
+    // large beside W that FP64 rounding moves a code
+    const double far = fmax(fmax(fabs(A.x), fabs(A.y)), fabs(A.z)) + A.w;
+    const Screen s = screen_of(A, T.cut2, far <= A.w * 1048576.0 ? A.w * 0x1p-27 : 1.0 / 0.0);
+    tin = s.tin;
+    tout = s.tout;
+  }
+  auto dist2_f32 = [&](const float4 &Q) {
+    const float dx = pfx - Q.x, dy = pfy - Q.y, dz = pfz - Q.z;
+    return fmaf(dz, dz, fmaf(dy, dy, dx * dx));
+  };
+  uint32_t cnt = 0;
+  int32_t qs = -1;
+  double md2 = 1.0 / 0.0;
+  uint64_t todo = __ballot(live), solo = 0;
+  uint32_t upto = 64;  // lanes from here on wait (after a group that held too many candidates)
+  while (todo) {
+    // the group: the first waiting cell's colony, up to lane upto; or that
+    // cell alone
+    const uint32_t first = (uint32_t)__builtin_ctzll(todo);
+    const uint32_t scid = (uint32_t)__builtin_amdgcn_readlane((int)cid, (int)first);
+    const bool single = (solo >> first) & 1u;
+    const bool mine = single ? lane == first : ((todo & ~solo) >> lane & 1u) && cid == scid && lane < upto;
+    if (mine) {
+      cnt = 0;
+      qs = -1;
+      md2 = 1.0 / 0.0;
+    }
+    // the smallest FP32 distance accepted by tin, with its cell, and the
+    // second smallest
+    float s1 = 1.0f / 0.0f, s2 = 1.0f / 0.0f;
+    uint32_t c1 = 0xFFFFFFFFu;
+    // the group cut at the highest Morton step between two of its cells, and
+    // each row's cells at the row's: the place of the highest bit that differs
+    // from the lane before (0: none)
+    uint32_t step = 0;
+    {
+      const uint4 me = code[again()];
+      const uint32_t ox = me.x ^ dpp<0x138>(0u, me.x), oy = me.y ^ dpp<0x138>(0u, me.y),
+                     oz = me.z ^ dpp<0x138>(0u, me.z);  // wave_shr 1
+      const uint32_t o = ox | oy | oz;
+      if (mine && lane > first && o) {
+        const uint32_t b = (uint32_t)tm_msb32(o);
+        step = ((3u * b + ((oz >> b) & 1u ? 2u : (oy >> b) & 1u ? 1u : 0u) + 1u) << 6) | lane;
+      }
+    }
+    const uint32_t wstep = wave_max_u32(step);
+    const uint32_t rstep = row_max_u32((lane & 15u) ? step : 0u);
+    const uint32_t wcut = wstep ? wstep & 63u : 64u, rcut = rstep ? rstep & 63u : 64u;
+    auto box_of = [&](bool in, auto &&reduce) {
+      QBox b;
+      auto axis = [&](uint32_t ex, uint32_t dm, uint32_t &bex, uint32_t &bdm) {
+        const uint32_t h = reduce(in ? ex + 1u : 0u), l = ~reduce(in ? ~(ex - dm) : 0u);
+        bex = h - 1u;  // no cells: ex = 2^32 - 1, dm = 0, which overlaps nothing
+        bdm = h - l - 1u;
+      };
+      axis(own.ex0, own.dm0, b.ex0, b.dm0);
+      axis(own.ex1, own.dm1, b.ex1, b.dm1);
+      axis(own.ex2, own.dm2, b.ex2, b.dm2);
+      return b;
+    };
+    auto on_wave = [](uint32_t v) { return wave_max_u32(v); };
+    auto on_row = [](uint32_t v) { return row_max_u32(v); };
+    const QBox boxa = box_of(mine && lane < wcut, on_wave), boxb = box_of(mine && lane >= wcut, on_wave);
+#pragma unroll
+    for (int half = 0; half < 2; ++half) {
+      const QBox b = box_of(mine && (half ? lane >= rcut : lane < rcut), on_row);
+      if ((lane & 15u) == 0 && row < (uint32_t)ROWS) rbox[2 * row + half] = b;
+    }
+    // the cell's side of the products below, relative to the row's first cell;
+    // where FP32 cannot hold the squares everything is near
+    const float ox = row_first(pfx), oy = row_first(pfy), oz = row_first(pfz);
+    float mx = pfx - ox, my = pfy - oy, mz = pfz - oz, mw;
+    {
+      const float p2 = fmaf(mz, mz, fmaf(my, my, mx * mx));
+      const bool fits = p2 < 1e37f && tout < 1e37f;
+      mw = fits ? p2 * LESS - (tout * (1.0f + 1e-6f) + 1e-36f) : -1e38f;
+      mx = fits ? mx : 0.f;
+      my = fits ? my : 0.f;
+      mz = fits ? mz : 0.f;
+    }
+    uint32_t nb = 0;  // staged candidates
+    auto drain = [&]() {
+      reinterpret_cast<uint4 *>(sub)[lane] = make_uint4(~0u, ~0u, ~0u, ~0u);
+      wave_lds_sync();
+      // the staged candidates of each row, in order: those that overlap one
+      // of its two boxes
+      float4 f[(CB + 64) / 64];
+      uint32_t len[4] = {0u, 0u, 0u, 0u};
+#pragma unroll
+      for (int b = 0; b < (CB + 64) / 64; ++b) {
+        f[b] = make_float4(0.f, 0.f, 0.f, 0.f);
+        if (64u * b < nb) {
+          const uint32_t e = 64u * b + lane;
+          const bool ok = e < nb;
+          const uint4 r = crec[ok ? e : 0u];
+          f[b] = posf[r.w];
+          const Octant c = leaf_octant(r);
+#pragma unroll
+          for (int q = 0; q < ROWS; ++q) {
+            uint32_t at = 2u * q;  // (opaque: two boxes in registers at a time, not all eight)
+            asm volatile("" : "+v"(at));
+            const bool h0 = hits(c, rbox[at]), h1 = hits(c, rbox[at + 1]);
+            const bool hit = ok & (h0 | h1);
+            const uint64_t m = __ballot(hit);
+            if (hit) sub8[256 * q + len[q] + mbcnt64(m)] = (uint8_t)e;
+            len[q] += (uint32_t)__builtin_popcountll(m);
+          }
+        }
+      }
+      wave_lds_sync();
+      const uint32_t mylen = row == 0 ? len[0] : row == 1 ? len[1] : row == 2 ? len[2] : len[3];
+      const uint8_t *const mysub = sub8 + 256 * row;
+      // The last candidate so far: the row's list backwards to the first octant
+      // that overlaps the lane's box.  An octant that does holds a code at or
+      // above the box's lower corner on every axis, so its last key is no
+      // smaller than that corner's: the octants of the list's end with smaller
+      // ones are skipped by a binary search (the list's keys descend).
+      {
+        const uint32_t nx = own.ex0 - own.dm0, ny = own.ex1 - own.dm1, nz = own.ex2 - own.dm2;
+        uint32_t at = 0;
+#pragma unroll 1
+        for (uint32_t b = 128; b > 0; b >>= 1) {
+          const uint4 r = crec[mysub[min(at + b - 1, 255u)]];
+          const Octant c = leaf_octant(r);
+          const bool skip = morton_less3(c.lx + c.sx - 1, c.ly + c.sy - 1, c.lz + c.sz - 1, nx, ny, nz);
+          at += ((at + b <= mylen) & !skip) ? b : 0u;
+        }
+        // upwards from there, as far as an octant's first key exceeds the
+        // box's upper corner's
+        bool want = mine & (at > 0);
+        for (int k = 0; k < 8 && __ballot(want); ++k) {
+          if (want) {
+            --at;
+            const uint4 r = crec[mysub[at]];
+            const Octant c = leaf_octant(r);
+            const bool hit = hits(c, own) & (r.w != (uint32_t)p);
+            qs = hit ? (int32_t)r.w : qs;
+            want = !hit & (at > 0) & !morton_less3(own.ex0, own.ex1, own.ex2, c.lx, c.ly, c.lz);
+          }
+        }
+        // a lane that needs more steps has the rest searched by the whole
+        // wave, 64 entries at a time
+        for (uint64_t left = __ballot(want); left; left &= left - 1) {
+          const int who = __builtin_ctzll(left);
+          auto of = [&](uint32_t v) { return (uint32_t)__builtin_amdgcn_readlane((int)v, who); };
+          const QBox b{of(own.ex0), of(own.ex1), of(own.ex2), of(own.dm0), of(own.dm1), of(own.dm2)};
+          const uint32_t wp = of((uint32_t)p);
+          const uint8_t *const wsub = sub8 + 256 * (who >> 4);
+          for (int k1 = (int)of(at); k1 > 0; k1 -= 64) {
+            const int k = k1 - 64 + (int)lane;
+            const uint4 r = crec[k >= 0 ? wsub[k] : CB];
+            const uint64_t m = __ballot((k >= 0) & hits(leaf_octant(r), b) & (r.w != wp));
+            if (m) {
+              const int32_t q = __builtin_amdgcn_readlane((int)r.w, 63 - __builtin_clzll(m));
+              if ((int)lane == who) qs = q;
+              break;
+            }
+          }
+        }
+      }
+      if (single) {
+        // a cell alone: every staged candidate but itself is one of its own
+        const int64_t pf = (int64_t)__builtin_amdgcn_readlane((int)p, (int)first);
+        const double4 W = pos[pf];
+        double least = 1.0 / 0.0;
+        for (uint32_t e = lane; e < nb; e += 64) {
+          const uint32_t q = crec[e].w;
+          if (q != (uint32_t)pf) least = fmin(least, dist2_fp64(W, pos[q]));
+        }
+        least = wave_min_f64(least);
+        if (mine) md2 = least < md2 ? least : md2;
+      }
+      wave_lds_sync();
+      float4 *const cq = reinterpret_cast<float4 *>(crec);
+#pragma unroll
+      for (int b = 0; b < (CB + 64) / 64; ++b) {
+        const uint32_t e = 64u * b + lane;
+        if (e < nb) cq[e] = make_float4(f[b].x, f[b].y, f[b].z, __uint_as_float(crec[e].w));
+      }
+      if (lane == 0) cq[CB] = make_float4(1.0e15f, 1.0e15f, 1.0e15f, 0.f);  // far from every cell
+      wave_lds_sync();
+      const uint32_t most = max(max(len[0], len[1]), max(len[2], len[3]));
+      for (uint32_t k0 = 0; k0 < most; k0 += 128) {
+        // Which of the row's next 16 T entries may be within a lane's cutoff:
+        // bit 31 - b of word g for entry 4 T g + b, b < 4 T.  The squared
+        // distances of 16 entries to the row's 16 cells, for the four rows at
+        // once, as |c|^2 + |p|^2 - 2 c.p by five outer products (relative to
+        // the row's first cell); lane 16 g + j holds those of entries 4 g + k
+        // of each row to the row's cell j, whose signs (less the threshold,
+        // with a margin for the rounding) are collected per row and then
+        // exchanged between the rows of lanes.
+        const uint32_t T = min(8u, (most - k0 + 15) >> 4);
+        uint32_t near[4] = {0u, 0u, 0u, 0u};
+        const uint8_t *const mine8 = mysub + k0 + 4 * T * ((lane & 15u) >> 2) + (lane & 3u);
+        float4 Qn = cq[mine8[0]];
+#pragma unroll 1
+        for (uint32_t t = 0; t < T; ++t) {
+          const float4 Q = Qn;
+          Qn = cq[mine8[4 * min(t + 1, T - 1)]];
+          const float x = Q.x - ox, y = Q.y - oy, z = Q.z - oz;
+          const float c2 = fmaf(z, z, fmaf(y, y, x * x));
+          const bool fits = c2 < 1e37f;
+          f32x16 d{};
+          d = __builtin_amdgcn_mfma_f32_16x16x1f32(fits ? -2.0f * x : 0.f, mx, d, 0, 0, 0);
+          d = __builtin_amdgcn_mfma_f32_16x16x1f32(fits ? -2.0f * y : 0.f, my, d, 0, 0, 0);
+          d = __builtin_amdgcn_mfma_f32_16x16x1f32(fits ? -2.0f * z : 0.f, mz, d, 0, 0, 0);
+          d = __builtin_amdgcn_mfma_f32_16x16x1f32(fits ? c2 * LESS : -1e38f, 1.0f, d, 0, 0, 0);
+          d = __builtin_amdgcn_mfma_f32_16x16x1f32(1.0f, mw, d, 0, 0, 0);
+#pragma unroll
+          for (int k = 0; k < 4; ++k)
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+              near[q] = __builtin_amdgcn_alignbit(near[q], __float_as_uint(d[4 * q + k]), 31);
+        }
+        transpose4(near);
+#pragma unroll
+        for (int q = 0; q < 4; ++q) near[q] = mine ? near[q] << (32u - 4u * T) : 0u;
+        // those, in order
+        uint32_t kb = k0;
+        while (near[0] | near[1] | near[2] | near[3]) {
+          if (near[0] == 0u) {
+            near[0] = near[1];
+            near[1] = near[2];
+            near[2] = near[3];
+            near[3] = 0u;
+            kb += 4 * T;
+          }
+          if (near[0] != 0u) {
+            const uint32_t j = (uint32_t)__clz((int)near[0]);
+            near[0] ^= 0x80000000u >> j;
+            const uint32_t e = mysub[kb + j];
+            const float4 Q = cq[e];
+            const uint32_t q = __float_as_uint(Q.w);
+            if (q != (uint32_t)p && e != (uint32_t)CB) {
+              const float sq = dist2_f32(Q);
+              bool in = sq <= tin;
+              if (in) {
+                s2 = __builtin_amdgcn_fmed3f(s1, s2, sq);
+                c1 = sq < s1 ? q : c1;
+                s1 = fminf(s1, sq);
+              } else {
+                // the FP32 distance leaves the cutoff or the octant open
+                const int64_t pa = again();
+                const double d2 = dist2_fp64(pos[pa], pos[q]);
+                in = d2 <= types[ctype_s[pa]].cut2 && hits(leaf_octant(leaf[q]), own);
+                if (in) md2 = d2 < md2 ? d2 : md2;
+              }
+              if (in) {
+                if (cnt < cap) nbr[tm_slot(p, cnt, cap)] = q;
+                ++cnt;
+              }
+            }
+          }
+        }
+      }
+      wave_lds_sync();
+      nb = 0;
+    };
+    // The colony's cells whose octants overlap one of the two boxes, in
+    // descending order: the blocks of 16 cells that overlap, found from the
+    // top of the tree of boxes down into a queue, then their cells, four
+    // blocks at a time.  Bits of a mask are taken from the highest.
+    const uint32_t s = (uint32_t)col_off[scid], e = (uint32_t)(col_off[scid + 1] - 1);
+    // lane's child of the 64 of node g, and the children that overlap and hold
+    // cells of the colony
+    auto child = [&](const BvhNode *lv, uint32_t sh, uint32_t g) {
+      const uint32_t lo = s >> sh, hi = e >> sh, i = 64u * g + lane;
+      const BvhNode *const b = lv + min(max(i, lo), hi);
+      const uint4 u = *reinterpret_cast<const uint4 *>(b);
+      const uint2 v = *reinterpret_cast<const uint2 *>(&b->sy);
+      return Octant{u.x, u.y, u.z, u.w, v.x, v.y};
+    };
+    auto overlapping = [&](const Octant &c, uint32_t sh, uint32_t g) -> uint64_t {
+      const uint32_t i = 64u * g + lane;
+      const bool ha = hits(c, boxa), hb = hits(c, boxb);
+      return __ballot((i >= s >> sh) & (i <= e >> sh) & (ha | hb));
+    };
+    // (a level with a single node for the colony is not read)
+    auto children = [&](const BvhNode *lv, uint32_t sh, uint32_t g) -> uint64_t {
+      const uint32_t lo = s >> sh;
+      return lo == e >> sh ? 1ull << (lo & 63u) : overlapping(child(lv, sh, g), sh, g);
+    };
+    auto top = [](uint64_t m) { return 63u - (uint32_t)__builtin_clzll(m); };
+    uint64_t m3 = 0, m2 = 0, m1 = 0;
+    uint32_t i3 = 0, i2 = 0, found = 0;
+    int g3 = (int)(e >> 28);
+    bool over = false;
+    for (bool last = false, full = false; !last && !over; full = false) {
+      uint32_t nq = 0;
+      for (;;) {
+        for (;;) {
+          for (;;) {
+            if (m1) {
+              uint32_t i1 = 64u * i2 + top(m1);
+              Octant next = child(bvh, 4, i1);
+              do {
+                const Octant c = next;
+                const uint64_t m = m1 & ~(1ull << (i1 & 63u));
+                const uint32_t j1 = 64u * i2 + (m ? top(m) : 0u);
+                if (m) next = child(bvh, 4, j1);
+                const uint64_t m0 = overlapping(c, 4, i1);
+                const uint32_t k = (uint32_t)__builtin_popcountll(m0);
+                full = nq + k > (uint32_t)BQ;
+                if (full) break;
+                if ((m0 >> lane) & 1u) queue[nq + k - 1 - mbcnt64(m0)] = 64u * i1 + lane;
+                nq += k;
+                m1 = m;
+                i1 = j1;
+              } while (m1);
+            }
+            if (full || !m2) break;
+            i2 = 64u * i3 + top(m2);
+            m2 &= ~(1ull << (i2 & 63u));
+            m1 = children(bvh + tree.l1, 10, i2);
+          }
+          if (full || !m3) break;
+          i3 = 64u * (uint32_t)(g3 + 1) + top(m3);
+          m3 &= ~(1ull << (i3 & 63u));
+          m2 = children(bvh + tree.l2, 16, i3);
+        }
+        if (full) break;
+        last = g3 < (int)(s >> 28);
+        if (last) break;
+        m3 = children(bvh + tree.l3, 22, (uint32_t)g3);
+        --g3;
+      }
+      // many blocks, and boxes much larger than the cells' own: the cells lie
+      // in several places, and those before the cut are taken first
+      if (wstep && nq > min(4u * ratio, (uint32_t)BQ - 64u) &&
+          volume(boxa) + volume(boxb) > (float)ratio * wave_mean(volume(own), mine)) {
+        over = true;
+        break;
+      }
+      wave_lds_sync();
+      auto block = [&](uint32_t i) { return i + row < nq ? queue[i + row] : ~0u; };
+      auto load = [&](uint32_t blk) {
+        const uint32_t q = blk * 16u + (15u - (lane & 15u));
+        const bool ok = (blk != ~0u) & (q >= s) & (q <= e);
+        uint4 r = leaf[ok ? q : s];
+        r.w = ok ? r.w : ~0u;
+        return r;
+      };
+      uint4 rn = load(block(0));
+      uint32_t bn = block(4);
+      for (uint32_t i = 0;; i += 4) {
+        const bool more = i < nq;
+        const uint4 r = rn;
+        rn = load(bn);
+        bn = block(i + 8);
+        const Octant c = leaf_octant(r);
+        const bool ha = hits(c, boxa), hb = hits(c, boxb);
+        const bool cand = (r.w != ~0u) & (ha | hb);  // none past the queue's end
+        const uint64_t cm = __ballot(cand);
+        const uint32_t k = (uint32_t)__builtin_popcountll(cm);
+        if (nb + k > (uint32_t)CB || (!more && last && nb > 0)) drain();
+        if (!more) break;
+        if (cand) {
+          const uint32_t at = mbcnt64(cm);
+          crec[nb + at] = r;
+          if (found + at < (uint32_t)UC) ucell[found + at] = r.w;
+        }
+        nb += k;
+        found += k;
+      }
+    }
+    if (over) {
+      upto = wcut;
+      continue;
+    }
+    upto = 64;
+    const uint64_t group = __ballot(mine);
+    todo &= ~group;
+    solo &= ~group;
+    // Cells with candidates but none within the cutoff: the minimum distance
+    // takes every candidate.  One such cell at a time, the lanes taking the
+    // group's candidates; with more of those than are kept, the cell is
+    // walked alone.
+    uint64_t bare = single ? 0ull : __ballot(mine && cnt == 0 && qs >= 0);
+    if (found > (uint32_t)UC) {
+      todo |= bare;
+      solo |= bare;
+    } else if (bare) {
+      wave_lds_sync();
+      while (bare) {
+        const int w0 = __builtin_ctzll(bare);
+        bare &= bare - 1;
+        const int w1 = bare ? __builtin_ctzll(bare) : w0;
+        bare &= bare - 1;
+        auto box_at = [&](int w) {
+          auto of = [&](uint32_t v) { return (uint32_t)__builtin_amdgcn_readlane((int)v, w); };
+          return QBox{of(own.ex0), of(own.ex1), of(own.ex2), of(own.dm0), of(own.dm1), of(own.dm2)};
+        };
+        const QBox b0 = box_at(w0), b1 = box_at(w1);
+        const uint32_t p0 = (uint32_t)__builtin_amdgcn_readlane((int)p, w0),
+                       p1 = (uint32_t)__builtin_amdgcn_readlane((int)p, w1);
+        const double4 W0 = pos[p0], W1 = pos[p1];
+        double l0 = 1.0 / 0.0, l1 = 1.0 / 0.0;
+#pragma unroll 2
+        for (uint32_t k = lane; k < found; k += 64) {
+          const uint32_t q = ucell[k];
+          const Octant c = leaf_octant(leaf[q]);
+          const bool h0 = hits(c, b0) & (q != p0), h1 = hits(c, b1) & (q != p1);
+          if (h0 | h1) {
+            const double4 Q = pos[q];
+            if (h0) l0 = fmin(l0, dist2_fp64(W0, Q));
+            if (h1) l1 = fmin(l1, dist2_fp64(W1, Q));
+          }
+        }
+        l0 = wave_min_f64(l0);
+        l1 = wave_min_f64(l1);
+        if ((int)lane == w0) md2 = l0;
+        else if ((int)lane == w1) md2 = l1;
+      }
+    }
+    if (mine && c1 != 0xFFFFFFFFu) {
+      // the smallest in FP64, and with it the others of the lane's list within
+      // its reach
+      const int64_t pa = again();
+      const double4 P = pos[pa];
+      const float reach = fmaf(1.0002f, s1, screen_of(aff[cid], 1.0, 0.0).beta);
+      double d2 = dist2_fp64(P, pos[c1]);
+      md2 = d2 < md2 ? d2 : md2;
+      if (s2 <= reach) {
+        for (uint32_t k = 0; k < min(cnt, (uint32_t)cap); ++k) {
+          const uint32_t q = nbr[tm_slot(p, k, cap)];
+          if (dist2_f32(posf[q]) <= reach) {
+            d2 = dist2_fp64(P, pos[q]);
+            md2 = d2 < md2 ? d2 : md2;
+          }
+        }
+      }
+    }
+  }
+  finish<NW>(again(), live, cnt, qs, md2, pos, ctype_s, young_s, types, n, cap, nbr, count, mindist, qstar, vout,
+             flags);
+}
+
+template <int BS, int WIN>
 void launch_walk(tm_ctx *c) {
-  auto kern = c->walk_f32 ? k_neighbors<BS, WIN, true, COOP> : k_neighbors<BS, WIN, false, COOP>;
+  auto kern = c->walk_f32 ? k_neighbors<BS, WIN, true> : k_neighbors<BS, WIN, false>;
   kern<<<tm_blocks(c->n, BS), BS, 0, c->stream>>>(
       c->d_pos, c->d_posf, c->d_code, c->d_ctype_s, c->d_young_s, c->d_wn, c->d_col_off, c->d_aff, c->d_types, c->n,
-      c->nbr_alloc, c->d_nbr, c->d_ncount, c->d_mind, c->d_qstar, c->d_v, c->d_flags, (float)c->walk_coop_ratio);
+      c->nbr_alloc, c->d_nbr, c->d_ncount, c->d_mind, c->d_qstar, c->d_v, c->d_flags);
+}
+
+// Cells per wave.  A wave costs about as much for 16 cells as 0.5 waves of
+// 64, so 64 is best where the waves fill the chip several times over; below,
+// the longest wave's time counts, and it falls with its cells.  Walk, us, with
+// 8 / 16 / 32 / 64 cells: Gaussian 30 K cells 81 / 90 / 101 / 294, 65 K 138 /
+// 116 / 173 / 339, 130 K - / 163 / 175 / 346, 260 K - / 275 / 215 / 343, 600 K
+// - / 562 / 398 / 549, 1M - / 910 / 736 / 748; ball 1M - / 591 / 401 / 339.
+template <int G>
+void launch_union(tm_ctx *c) {
+  k_union<G><<<tm_blocks(c->n, 64), 4096 / G, 0, c->stream>>>(
+      c->d_pos, c->d_posf, c->d_code, c->d_ctype_s, c->d_young_s, c->d_leaf, c->d_bvh, bvh_of(c->n), c->d_col_off,
+      c->d_aff, c->d_types, c->n, c->nbr_alloc, c->d_nbr, c->d_ncount, c->d_mind, c->d_qstar, c->d_v, c->d_flags,
+      (uint32_t)c->walk_coop_ratio);
 }
 
 }  // namespace
@@ -456,7 +1010,12 @@ tm_status tm_run_neighbors(tm_ctx *c, bool check) {
     }
     c->nbr_alloc = c->nbr_cap;
     const int bs = c->nbr_block;
-    if (c->walk_coop) launch_walk<64, 0, true>(c);
+    const bool coop = c->walk_coop && c->walk_f32;
+    if (!coop) TM_TRY(tm_ensure_tree(c));
+    if (coop && n <= 1 << 15) launch_union<8>(c);
+    else if (coop && n <= 1 << 17) launch_union<16>(c);
+    else if (coop && n <= 3 << 18) launch_union<32>(c);
+    else if (coop) launch_union<64>(c);
     else if (bs == 64) launch_walk<64, 0>(c);
     else if (bs == 128) launch_walk<128, 0>(c);
     else if (c->walk_window == 2048 && 2 * n - 1 >= 2048) launch_walk<256, 2048>(c);

@@ -180,6 +180,7 @@ tm_status tm_run_octree(tm_ctx *c, int colony, void *nodes, int64_t *count) {
   }
   const int64_t n = c->n;
   int32_t root = 0;
+  TM_TRY(tm_ensure_tree(c));
   TM_HIP(c, hipMemcpyAsync(&root, c->d_colroot + colony, 4, hipMemcpyDeviceToHost, c->stream));
   TM_HIP(c, hipStreamSynchronize(c->stream));
   if (root < 0 || root > n - 2) return tm_fail(c, TM_ERR_STATE, "colony has no internal root");
