@@ -109,3 +109,31 @@ def test_octree_on_demand(tm, ctx):
         ctx.graph_launch()
         assert np.array_equal(ctx.octree(0), ref)
     ctx.graph_destroy()
+
+
+def test_fp64_sums_with_and_without_tiles(tm, ctx):
+    """a step's one FP64 sum is taken from the lists, later sums over tiles:
+    the same bits; a mixed sum after it is the one of a mixed step; tiles of a
+    replay's lists are not those of the lists before"""
+    ctx.upload_colony(gaussian(20011))
+    ctx.step(tm.MIXED)
+    mixed = ctx.results()
+    ctx.step(tm.FP64)
+    first = ctx.results()
+    for _ in range(10):
+        ctx.sph(tm.FP64)
+    over_tiles = ctx.results()
+    ctx.sph(tm.MIXED)
+    again = ctx.results()
+    for k in first:
+        assert np.array_equal(over_tiles[k], first[k]) and np.array_equal(again[k], mixed[k]), k
+    ctx.graph_capture_loop(tm.Move.make([0.2, 0.2], seed=5), tm.FP64)
+    for _ in range(2):
+        ctx.sph(tm.MIXED)
+        ctx.graph_launch()
+        got = ctx.results()
+        ctx.sph(tm.MIXED)
+        ctx.sph(tm.FP64)
+        for k in got:
+            assert np.array_equal(ctx.results()[k], got[k]), k
+    ctx.graph_destroy()

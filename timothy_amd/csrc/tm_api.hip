@@ -226,17 +226,23 @@ tm_status check_flags(tm_ctx *c) {
   return TM_OK;
 }
 
+// Whether a step makes LDS tiles for its one sum.  In the mixed form the
+// sums' rounding goes with them.  The FP64 sums are the same bits either way,
+// and one sum from the lists takes less time than the tiles and the sum over
+// them: 300 K-cell ball 18 against 39 us, 2M Gaussian 152 against 285 us.
+bool step_tiles(const tm_ctx *c, tm_precision p) { return p == TM_MIXED && tm_tiles_serve(c); }
+
 tm_status run_stage(tm_ctx *c, tm_stage s, tm_precision p) {
   switch (s) {
     case TM_STAGE_BUILD: return tm_run_build(c);
-    case TM_STAGE_NEIGHBORS: return tm_run_neighbors(c, false);
+    case TM_STAGE_NEIGHBORS: return tm_run_neighbors(c, false, tm_tiles_serve(c));
     case TM_STAGE_SPH: return tm_run_sph(c, p);
     case TM_STAGE_CIC:
       if (!c->last_prod) return tm_fail(c, TM_ERR_STATE, "no tm_cic_deposit call to repeat");
       return tm_run_deposit(c, &c->last_grid, c->last_weight, c->last_prod);
     case TM_STAGE_STEP:
       TM_TRY(tm_run_build(c));
-      TM_TRY(tm_run_neighbors(c, false));
+      TM_TRY(tm_run_neighbors(c, false, step_tiles(c, p)));
       return tm_run_sph(c, p);
     case TM_STAGE_TILES:
       return tm_run_tiles(c, false);
@@ -462,6 +468,9 @@ tm_status tm_set_param(tm_ctx *c, const char *key, int64_t v) {
 
 tm_status tm_get_param(tm_ctx *c, const char *key, int64_t *v) {
   if (!c || !key || !v) return TM_ERR_INVALID;
+  // the lists' tiles, where the last step made none
+  if ((!strcmp(key, "tile_lds") || !strcmp(key, "tiles_over")) && c->stage >= 3 && c->sph_tiles && c->tiles_ts == 0)
+    TM_TRY(tm_run_tiles(c, true));
   if (!strcmp(key, "nbr_cap")) *v = c->nbr_cap;
   else if (!strcmp(key, "sph_block")) *v = c->sph_block;
   else if (!strcmp(key, "sph_unroll_fp64")) *v = c->sph_unroll_fp64;
@@ -504,7 +513,7 @@ tm_status tm_build(tm_ctx *c) {
 
 tm_status tm_neighbors(tm_ctx *c) {
   if (!c) return TM_ERR_INVALID;
-  return tm_run_neighbors(c, true);
+  return tm_run_neighbors(c, true, tm_tiles_serve(c));
 }
 
 tm_status tm_sph(tm_ctx *c, tm_precision p) {
@@ -516,7 +525,7 @@ tm_status tm_sph(tm_ctx *c, tm_precision p) {
 tm_status tm_step(tm_ctx *c, tm_precision p) {
   if (!c) return TM_ERR_INVALID;
   TM_TRY(tm_run_build(c));
-  TM_TRY(tm_run_neighbors(c, true));
+  TM_TRY(tm_run_neighbors(c, true, step_tiles(c, p)));
   return tm_sph(c, p);
 }
 
@@ -797,7 +806,7 @@ tm_status capture(tm_ctx *c, tm_precision p) {
   tm_graph_destroy(c);
   TM_HIP(c, hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
   tm_status s = tm_run_build(c);
-  if (s == TM_OK) s = tm_run_neighbors(c, false);
+  if (s == TM_OK) s = tm_run_neighbors(c, false, step_tiles(c, p));
   if (s == TM_OK) s = tm_run_sph(c, p);
   if (s == TM_OK && c->graph_loop) s = tm_run_move(c, &c->graph_move, nullptr, c->graph_removecell, true);
   hipGraph_t g = nullptr;
@@ -809,6 +818,7 @@ tm_status capture(tm_ctx *c, tm_precision p) {
   if (e != hipSuccess) return tm_fail(c, TM_ERR_HIP, std::string("hipStreamEndCapture: ") + hipGetErrorString(e));
   c->graph = g;
   c->graph_tree = c->tree_valid;
+  c->graph_tiles_ts = c->tiles_ts;
   TM_HIP(c, hipGraphInstantiate(&c->gexec, g, nullptr, nullptr, 0));
   c->graph_prec = p;
   return TM_OK;
@@ -926,11 +936,13 @@ tm_status tm_graph_launch(tm_ctx *c) {
   if (!c->gexec) return tm_fail(c, TM_ERR_STATE, "no captured graph");
   TM_HIP(c, hipGraphLaunch(c->gexec, c->stream));
   c->tree_valid = c->graph_tree;
+  c->tiles_ts = c->graph_tiles_ts;
+  c->direct_sums = 0;
   TM_TRY(check_flags(c));
   if (c->h_flags[1] > (unsigned)c->nbr_alloc) {
     // a cell outgrew the captured lists (and a captured move moved nothing):
     // grow, redo the step eagerly from this replay's tree, recapture
-    TM_TRY(tm_run_neighbors(c, true));
+    TM_TRY(tm_run_neighbors(c, true, step_tiles(c, c->graph_prec)));
     TM_TRY(tm_run_sph(c, c->graph_prec));
     if (c->graph_loop) TM_TRY(tm_run_move(c, &c->graph_move, nullptr, c->graph_removecell, true));
     TM_TRY(capture(c, c->graph_prec));
@@ -1017,7 +1029,7 @@ tm_status tm_autotune(tm_ctx *c, tm_precision p, char *buf, size_t buflen) {
     cur_t = 1e30;
     for (int w : {128, 256, 512}) {
       c->tile_width = w;
-      TM_TRY(tm_run_neighbors(c, true));  // lists, and tiles of this width sized for LDS
+      TM_TRY(tm_run_neighbors(c, true, tm_tiles_serve(c)));  // lists, and tiles of this width sized for LDS
       double tt = 0;
       TM_TRY(tm_time_stage(c, TM_STAGE_TILES, p, 1, 5, &tt));
       for (int u : {2, 4, 8}) {
@@ -1042,10 +1054,10 @@ tm_status tm_autotune(tm_ctx *c, tm_precision p, char *buf, size_t buflen) {
     if (best_w != w0) tm_graph_destroy(c);  // a captured graph holds tiles of the old width
     c->tile_width = best_w;
     unroll = best_u;
-    TM_TRY(tm_run_neighbors(c, true));
+    TM_TRY(tm_run_neighbors(c, true, tm_tiles_serve(c)));
   } else {
     // direct pair kernel: workgroup size x neighbours per trip (x lanes per cell)
-    TM_TRY(tm_run_neighbors(c, true));
+    TM_TRY(tm_run_neighbors(c, true, tm_tiles_serve(c)));
     int best_sb = c->sph_block, best_u = unroll, best_l = c->sph_lanes;
     best_t = 1e30;
     const std::vector<int> lanes = (p == TM_MIXED) ? std::vector<int>{1, 2, 4, 8} : std::vector<int>{1};

@@ -176,6 +176,8 @@ struct tm_ctx {
   int walk_coop = 1;                // 1: one walk per wave for its cells together (see k_union)
   int walk_coop_ratio = 64;         // its boxes' volume / mean cell box volume above which a wave's cells are parted
   int tiles_ts = 0;                 // cells per tile of the tiles as built (0: none)
+  bool lists_tiles = false;         // whether tiles served when the current lists were made
+  int direct_sums = 0;              // FP64 sums taken from the current lists without tiles
   int tile_lds_ts = 0;              // the tile width tile_lds was sized for
   int64_t cap_tile_idx = 0, cap_tile_cnt = 0, cap_tile_cell = 0, cap_nbr16 = 0;
 
@@ -234,6 +236,7 @@ struct tm_ctx {
   tm_precision graph_prec = TM_FP64;
   bool graph_loop = false;     // the captured step also moves the cells
   bool graph_tree = false;     // the captured step makes the radix tree
+  int graph_tiles_ts = 0;      // and tiles of this width (0: none)
   tm_move graph_move{};        // its parameters
   uint8_t *graph_removecell = nullptr;
 };
@@ -273,7 +276,8 @@ tm_status tm_scan_u32(tm_ctx *c, const uint32_t *in, uint32_t *out, int64_t n);
 tm_status tm_run_build(tm_ctx *c);
 // the radix tree of the last build (the per-lane walks and the emitted octree)
 tm_status tm_ensure_tree(tm_ctx *c);
-tm_status tm_run_neighbors(tm_ctx *c, bool check);
+// tiles: also the LDS tiles (otherwise tm_run_sph makes them where it needs them)
+tm_status tm_run_neighbors(tm_ctx *c, bool check, bool tiles);
 tm_status tm_run_tiles(tm_ctx *c, bool check);
 tm_status tm_run_sph(tm_ctx *c, tm_precision prec);
 tm_status tm_run_unpermute(tm_ctx *c);
@@ -313,6 +317,12 @@ __device__ __forceinline__ int tm_msb32(uint32_t v) { return 31 - __clz((int)v);
 __device__ __forceinline__ int tm_diffbit(uint4 a, uint4 b) {
   uint32_t o = (a.x ^ b.x) | (a.y ^ b.y) | (a.z ^ b.z);
   return o ? tm_msb32(o) : -1;
+}
+
+// whether the pair kernels can read tiles: 3-D, and 32-bit offsets into the
+// position records
+inline bool tm_tiles_serve(const tm_ctx *c) {
+  return c->sph_tiles && c->dim == 3 && 32 * (c->n + 1) <= (int64_t)0xFFFFFFFF;
 }
 
 inline unsigned tm_blocks(int64_t n, int threads) { return (unsigned)((n + threads - 1) / threads); }

@@ -989,7 +989,7 @@ void launch_union(tm_ctx *c) {
 }  // namespace
 
 // grows the neighbour lists and repeats the walk when a cell overflowed them
-tm_status tm_run_neighbors(tm_ctx *c, bool check) {
+tm_status tm_run_neighbors(tm_ctx *c, bool check, bool tiles) {
   if (c->stage < 2) return tm_fail(c, TM_ERR_STATE, "tm_neighbors before tm_build");
   const int64_t n = c->n;
   if (n == 0) {
@@ -1038,7 +1038,10 @@ tm_status tm_run_neighbors(tm_ctx *c, bool check) {
     if (mx <= c->nbr_alloc) break;
     c->nbr_cap = (mx + 7) & ~7ll;  // grow to the largest count seen, rounded up
   }
-  TM_TRY(tm_run_tiles(c, check));
+  c->tiles_ts = 0;
+  c->lists_tiles = tm_tiles_serve(c);
+  c->direct_sums = 0;
+  if (tiles) TM_TRY(tm_run_tiles(c, check));
   c->stage = 3;
   return TM_OK;
 }
