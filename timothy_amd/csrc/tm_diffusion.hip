@@ -13,185 +13,118 @@
 // diagonal, so Jacobi-preconditioned CG (plain CG scaled by that constant,
 // with the same stopping norm) reaches the same solution to that tolerance.
 //
-// Matrix-free, one lane per node, nodes in the field's layout ([i][j][k], k
-// fastest).  An iteration is two streaming kernels and two one-block
-// reductions:
-//   k_cg_dir     p_new = r + beta p_old at the node and its 6 neighbours,
-//                Ap = A p_new, partial sums of p_new . Ap      (reads r, p;
-//                writes p_new, Ap: 32 B/node when neighbours come from cache)
-//   k_cg_alpha   alpha = rr / pAp (fixed-order sum of the partials)
-//   k_cg_update  x += alpha p, r -= alpha Ap, partial sums of r . r
-//                                                             (48 B/node)
-//   k_cg_beta    beta = rr_new / rr, convergence test, iteration count
-// The scalars live in device memory; once converged, every kernel of the
-// remaining iterations returns at once, so the host launches iterations in
-// batches and reads the state once per batch.  The partial sums are added
-// in a fixed order: results do not depend on timing.
+// Matrix-free, nodes in the field's layout ([i][j][k], k fastest).  An
+// iteration is two streaming kernels:
+//   k_cg<DIR>     beta = rr_new / rr, p_new = r + beta p_old, partial sums of
+//                 p_new . A p_new              (reads r, p; writes p: 24 B/node)
+//   k_cg<UPDATE>  alpha = rr / pAp, x += alpha p, r -= alpha A p, partial sums
+//                 of r . r              (reads p, x, r; writes x, r: 40 B/node)
+// A p is formed twice from the stencil rather than stored and read (16 B/node
+// less), and every workgroup adds the partial sums itself, in one fixed order,
+// so that no launch stands between the two and results do not depend on
+// timing.  The scalars live in device memory; once converged, the kernels of
+// the remaining iterations return at once, so the host launches iterations in
+// batches and reads the state once per batch.
 #include <mutex>
 
 #include "tm_internal.h"
 
 namespace {
 
-constexpr int BD = 256;
 constexpr int MAXBLK = 4096;  // partial sums per reduction
 
 struct CGState {
-  double rr, bb, pAp, alpha, beta, tol2;
+  double bb, tol2;
+  double rr[2];  // residual norm before iteration k at [k & 1]
+  double last;   // and after the last one checked
   unsigned long long iters;
-  int done;
-  int pad;
+  // 0, or one more than the pass that set it: pass 0 is k_cg_start, DIR and
+  // UPDATE of iteration k are 2k + 1 and 2k + 2.  A pass stops for an earlier
+  // pass's mark only, so all its waves agree, also where its own first
+  // workgroup has set one meanwhile.
+  unsigned int done;
+  unsigned int pad;
 };
 
 struct Op {
   int64_t lx, ly, lz;
-  double diag, z;
+  double diag, z, zbc;
 };
 
+// sum over the workgroup's T threads, in all of them, always in the same
+// order; sh: T / 64 doubles that nothing else uses until the next barrier
+template <int T>
 __device__ __forceinline__ double block_sum(double v, double *sh) {
 #pragma unroll
   for (int o = 32; o >= 1; o >>= 1) v += __shfl_xor(v, o, 64);
-  const int w = threadIdx.x >> 6;
-  if ((threadIdx.x & 63) == 0) sh[w] = v;
+  if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = v;
   __syncthreads();
   double s = 0.0;
-  if (threadIdx.x == 0)
-    for (int i = 0; i < BD / 64; ++i) s += sh[i];
+  for (int i = 0; i < T / 64; ++i) s += sh[i];
   return s;
 }
-
-// nodes [chunk * b, chunk * (b + 1)) belong to block b (contiguous, so a
-// block's neighbour planes are mostly its own or its neighbours')
-__device__ __forceinline__ void block_range(int64_t total, int64_t chunk, int64_t &lo, int64_t &hi) {
-  lo = (int64_t)blockIdx.x * chunk;
-  hi = min(lo + chunk, total);
+template <int T>
+__device__ __forceinline__ double sum_parts(const double *__restrict__ part, int n, double *sh) {
+  double a = 0.0;
+  for (int i = threadIdx.x; i < n; i += T) a += part[i];
+  return block_sum<T>(a, sh);
 }
 
-// right-hand side, residual of the initial guess, first direction
-__global__ __launch_bounds__(BD) void k_cg_init(Op A, double zbc, const double *__restrict__ src,
-                                                const double *__restrict__ x, double *__restrict__ b,
-                                                double *__restrict__ r, double *__restrict__ p, int64_t chunk,
-                                                double *__restrict__ part_rr, double *__restrict__ part_bb) {
-  __shared__ double sh[BD / 64];
-  const int64_t total = A.lx * A.ly * A.lz, sx = A.ly * A.lz, sy = A.lz;
-  int64_t lo, hi;
-  block_range(total, chunk, lo, hi);
-  double rr = 0.0, bb = 0.0;
-  for (int64_t node = lo + threadIdx.x; node < hi; node += BD) {
-    const int64_t k = node % A.lz, j = (node / A.lz) % A.ly, i = node / sx;
-    const double xc = x[node];
-    // b in the reference's order: u_old, the faces x-, x+, y-, y+, z-, z+, then s
-    double bv = xc;
-    if (i == 0) bv += zbc;
-    if (i == A.lx - 1) bv += zbc;
-    if (j == 0) bv += zbc;
-    if (j == A.ly - 1) bv += zbc;
-    if (k == 0) bv += zbc;
-    if (k == A.lz - 1) bv += zbc;
-    if (src) bv += src[node];
-    double nb = 0.0;
-    if (i > 0) nb += x[node - sx];
-    if (i < A.lx - 1) nb += x[node + sx];
-    if (j > 0) nb += x[node - sy];
-    if (j < A.ly - 1) nb += x[node + sy];
-    if (k > 0) nb += x[node - 1];
-    if (k < A.lz - 1) nb += x[node + 1];
-    const double rv = bv - (A.diag * xc - A.z * nb);
-    b[node] = bv;
-    r[node] = rv;
-    p[node] = rv;
-    rr += rv * rv;
-    bb += bv * bv;
-  }
-  const double s1 = block_sum(rr, sh);
-  __syncthreads();
-  const double s2 = block_sum(bb, sh);
-  if (threadIdx.x == 0) {
-    part_rr[blockIdx.x] = s1;
-    part_bb[blockIdx.x] = s2;
-  }
+// right-hand side at a node, in the reference's order: u_old, the faces x-,
+// x+, y-, y+, z-, z+, then s
+__device__ __forceinline__ double rhs(const Op &A, double u, int64_t i, int64_t j, int64_t k, const double *src,
+                                      int64_t node) {
+  if (i == 0) u += A.zbc;
+  if (i == A.lx - 1) u += A.zbc;
+  if (j == 0) u += A.zbc;
+  if (j == A.ly - 1) u += A.zbc;
+  if (k == 0) u += A.zbc;
+  if (k == A.lz - 1) u += A.zbc;
+  if (src) u += src[node];
+  return u;
 }
 
-__global__ void k_cg_start(const double *__restrict__ part_rr, const double *__restrict__ part_bb, int nblk,
-                           double tol, int maxiter, CGState *st) {
-  __shared__ double sh[BD / 64];
-  double a = 0.0, c = 0.0;
-  for (int i = threadIdx.x; i < nblk; i += BD) {
-    a += part_rr[i];
-    c += part_bb[i];
-  }
-  const double rr = block_sum(a, sh);
-  __syncthreads();
-  const double bb = block_sum(c, sh);
-  if (threadIdx.x == 0) {
-    st->rr = rr;
-    st->bb = bb;
-    st->tol2 = tol * tol;
-    st->beta = 0.0;
-    st->iters = 0;
-    st->done = (rr <= st->tol2 * bb || maxiter <= 0) ? 1 : 0;
-  }
-}
-
-// p_new = r + beta p_old (at the node and its neighbours), Ap = A p_new
-__global__ __launch_bounds__(BD) void k_cg_dir(Op A, const double *__restrict__ r, const double *__restrict__ pold,
-                                               double *__restrict__ pnew, double *__restrict__ Ap, int64_t chunk,
-                                               const CGState *__restrict__ st, double *__restrict__ part) {
-  __shared__ double sh[BD / 64];
-  if (st->done) return;
-  const double beta = st->beta;
-  const int64_t total = A.lx * A.ly * A.lz, sx = A.ly * A.lz, sy = A.lz;
-  int64_t lo, hi;
-  block_range(total, chunk, lo, hi);
-  double acc = 0.0;
-  for (int64_t node = lo + threadIdx.x; node < hi; node += BD) {
-    const int64_t k = node % A.lz, j = (node / A.lz) % A.ly, i = node / sx;
-    const double pc = r[node] + beta * pold[node];
-    double nb = 0.0;
-    if (i > 0) nb += r[node - sx] + beta * pold[node - sx];
-    if (i < A.lx - 1) nb += r[node + sx] + beta * pold[node + sx];
-    if (j > 0) nb += r[node - sy] + beta * pold[node - sy];
-    if (j < A.ly - 1) nb += r[node + sy] + beta * pold[node + sy];
-    if (k > 0) nb += r[node - 1] + beta * pold[node - 1];
-    if (k < A.lz - 1) nb += r[node + 1] + beta * pold[node + 1];
-    const double ap = A.diag * pc - A.z * nb;
-    pnew[node] = pc;
-    Ap[node] = ap;
-    acc += pc * ap;
-  }
-  const double s = block_sum(acc, sh);
-  if (threadIdx.x == 0) part[blockIdx.x] = s;
-}
-
-// The same, marching along i: a workgroup owns an MJ x MK block of (j, k)
-// columns over a run of planes [i0, i1).  Per plane it forms p_new once per
-// node (and once per node of the block's edge ring, which the neighbouring
-// blocks also form) into LDS; the i-1 and i+1 values of its own column stay
-// in registers.  r and p_old are read about once instead of once per
-// neighbour through the caches.  Each node's p_new and Ap are the values
-// k_cg_dir forms (the same expressions, the neighbours added in the same
-// order); only the partial sums of p_new . Ap group differently.
-constexpr int MJ = 4, MK = 64, MT = MJ * MK;
+// The three streaming passes, marching along i: a workgroup owns an MJ x MK
+// block of (j, k) columns over a run of planes.  Per plane the operand of the
+// stencil (x, p_new or p) is formed once per node, and once per node of the
+// block's edge ring (which the neighbouring blocks also form), into LDS; the
+// values of its own column one plane before and after stay in registers.
+//   INIT    r = b - A x                  parts: r . r, b . b
+//   DIR     p_new = r + beta p_old       parts: p_new . A p_new
+//   UPDATE  x += alpha p, r -= alpha A p parts: r . r
+// Odd passes take the blocks and planes in the opposite order (`down`): what
+// the pass before touched last is then read first, from the 256 MB memory-side
+// cache.
+//
+// Bound by the bytes: 256^3 takes 195 us an iteration, 64 B a node at 5.5 TB/s
+// (some of it from that cache), where storing A p and the one-workgroup
+// reductions between the kernels took 80 B and 280 us.  The loads of a plane
+// go out two planes ahead, and those of the first planes before the scalars are
+// known: without that 217 against 280 us at 256^3, and a kernel of a 32^3 grid,
+// which is latency from end to end, 9 us instead of 6.5.  The 8 x 64 block in
+// two workgroups a CU: 4 x 64 in four takes 205 us, 16 x 64 in one 189 us but
+// 20 % more than 8 x 64 at 64^3 and below; one workgroup a CU takes 250 us,
+// four 217 us.
+enum Pass { INIT, DIR, UPDATE };
+struct Blocks {
+  unsigned int nk, nj, run;  // blocks along k and j, planes a run
+  unsigned int count;        // workgroups' worth of work: at most MAXBLK are launched
+};
+constexpr int MJ = 8, MK = 64, MT = MJ * MK;
 constexpr int MHALO = 2 * MJ + 2 * MK;  // the edge ring without its corners
 
-__global__ __launch_bounds__(MT) void k_cg_dir_march(Op A, const double *__restrict__ r,
-                                                     const double *__restrict__ pold, double *__restrict__ pnew,
-                                                     double *__restrict__ Ap, int nseg,
-                                                     const CGState *__restrict__ st, double *__restrict__ part) {
+template <int PASS>
+__global__ __launch_bounds__(MT) void k_cg(Op A, const double *__restrict__ src, double *__restrict__ x,
+                                           double *__restrict__ r, const double *__restrict__ pold,
+                                           double *__restrict__ pnew, Blocks B, int iter,
+                                           CGState *__restrict__ st, const double *__restrict__ in,
+                                           double *__restrict__ out, double *__restrict__ out2) {
   __shared__ double pl[2][MJ + 2][MK + 2];
-  __shared__ double sh[MT / 64];
-  if (st->done) return;
-  const double beta = st->beta;
+  __shared__ double sh[2][MT / 64];
+  constexpr bool down = PASS == UPDATE;
+  constexpr int64_t d = down ? -1 : 1;
   const int64_t sx = A.ly * A.lz, sy = A.lz;
-  const int ntk = (int)((A.lz + MK - 1) / MK), ntj = (int)((A.ly + MJ - 1) / MJ);
-  int b = blockIdx.x;
-  const int kt = b % ntk;
-  b /= ntk;
-  const int jt = b % ntj, seg = b / ntj;
-  const int64_t i0 = A.lx * seg / nseg, i1 = A.lx * (seg + 1) / nseg;
   const int tk = (int)threadIdx.x % MK, tj = (int)threadIdx.x / MK;
-  const int64_t j = (int64_t)jt * MJ + tj, k = (int64_t)kt * MK + tk;
-  const bool own = j < A.ly && k < A.lz;
   // this thread's place on the edge ring, if any: (a, c) in the (MJ+2) x (MK+2) frame
   int ha = -1, hc = -1;
   {
@@ -210,122 +143,298 @@ __global__ __launch_bounds__(MT) void k_cg_dir_march(Op A, const double *__restr
       hc = MK + 1;
     }
   }
-  const int64_t hj = (int64_t)jt * MJ + ha - 1, hk = (int64_t)kt * MK + hc - 1;
-  const bool halo = ha >= 0 && hj >= 0 && hj < A.ly && hk >= 0 && hk < A.lz;
-  // plane i into LDS buffer q; returns this column's value
-  auto plane = [&](int64_t i, int q) -> double {
-    double v = 0.0;
-    if (own) {
-      const int64_t node = i * sx + j * sy + k;
-      v = r[node] + beta * pold[node];
-      pl[q][tj + 1][tk + 1] = v;
+  double acc = 0.0, acc2 = 0.0;
+  double scale = 0.0;  // beta or alpha
+  const unsigned int b0 = (unsigned int)tm_xcd_block();
+  for (unsigned int c = b0; c < B.count; c += gridDim.x) {
+    const unsigned int b = down ? B.count - 1 - c : c;
+    const unsigned int kt = b % B.nk, bj = b / B.nk, jt = bj % B.nj, seg = bj / B.nj;
+    const int64_t i0 = (int64_t)seg * B.run, i1 = i0 + B.run < A.lx ? i0 + B.run : A.lx;
+    const int64_t j = (int64_t)jt * MJ + tj, k = (int64_t)kt * MK + tk;
+    const bool own = j < A.ly && k < A.lz;
+    const int64_t hj = (int64_t)jt * MJ + ha - 1, hk = (int64_t)kt * MK + hc - 1;
+    const bool halo = ha >= 0 && hj >= 0 && hj < A.ly && hk >= 0 && hk < A.lz;
+    const int64_t col = j * sy + k, hcol = hj * sy + hk;
+    const int64_t first = down ? i1 - 1 : i0, stop = down ? i0 - 1 : i1;
+    // what the operand of the stencil is formed from: own column, edge ring
+    struct Raw {
+      double a, b, ha, hb;
+    };
+    auto load = [&](int64_t i) -> Raw {
+      Raw w{0.0, 0.0, 0.0, 0.0};
+      if (i < 0 || i >= A.lx) return w;
+      const double *u = PASS == INIT ? x : PASS == UPDATE ? pold : r;
+      if (own) w.a = u[i * sx + col];
+      if (halo) w.ha = u[i * sx + hcol];
+      if constexpr (PASS == DIR) {
+        if (iter > 0) {
+          if (own) w.b = pold[i * sx + col];
+          if (halo) w.hb = pold[i * sx + hcol];
+        }
+      }
+      return w;
+    };
+    auto form = [&](double u, double v) -> double {
+      if constexpr (PASS == DIR) return iter > 0 ? u + scale * v : u;
+      return u;
+    };
+    auto place = [&](int64_t i, const Raw &w) {
+      if (own) pl[i & 1][tj + 1][tk + 1] = form(w.a, w.b);
+      if (halo) pl[i & 1][ha][hc] = form(w.ha, w.hb);
+    };
+    // the first planes' loads go out before the scalars are known
+    const Raw wb = load(first - d);
+    Raw w = load(first);
+    Raw wn = load(first + d);
+    double xn = 0.0, rn = 0.0;
+    if constexpr (PASS == UPDATE) {
+      if (own) {
+        xn = x[first * sx + col];
+        rn = r[first * sx + col];
+      }
     }
-    if (halo) {
-      const int64_t node = i * sx + hj * sy + hk;
-      pl[q][ha][hc] = r[node] + beta * pold[node];
-    }
-    return v;
-  };
-  double acc = 0.0;
-  double pprev = 0.0, pcur = 0.0, pnext = 0.0;
-  if (i0 < i1) {
-    if (i0 > 0 && own) {
-      const int64_t node = (i0 - 1) * sx + j * sy + k;
-      pprev = r[node] + beta * pold[node];
-    }
-    pcur = plane(i0, (int)(i0 & 1));
-  }
-  for (int64_t i = i0; i < i1; ++i) {
-    __syncthreads();  // plane i is in its buffer; the reads of plane i - 1 are done
-    const int q = (int)(i & 1);
-    if (i + 1 < A.lx) pnext = plane(i + 1, q ^ 1);
-    if (own) {
-      double nb = 0.0;
-      if (i > 0) nb += pprev;
-      if (i < A.lx - 1) nb += pnext;
-      if (j > 0) nb += pl[q][tj][tk + 1];
-      if (j < A.ly - 1) nb += pl[q][tj + 2][tk + 1];
-      if (k > 0) nb += pl[q][tj + 1][tk];
-      if (k < A.lz - 1) nb += pl[q][tj + 1][tk + 2];
-      const double ap = A.diag * pcur - A.z * nb;
-      const int64_t node = i * sx + j * sy + k;
-      pnew[node] = pcur;
-      Ap[node] = ap;
-      acc += pcur * ap;
-    }
-    pprev = pcur;
-    pcur = pnext;
-  }
-  __syncthreads();
-  double v = acc;
-#pragma unroll
-  for (int o = 32; o >= 1; o >>= 1) v += __shfl_xor(v, o, 64);
-  if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = v;
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    double s = 0.0;
-    for (int w = 0; w < MT / 64; ++w) s += sh[w];
-    part[blockIdx.x] = s;
-  }
-}
-
-__global__ void k_cg_alpha(const double *__restrict__ part, int nblk, CGState *st) {
-  __shared__ double sh[BD / 64];
-  if (st->done) return;
-  double a = 0.0;
-  for (int i = threadIdx.x; i < nblk; i += BD) a += part[i];
-  const double pAp = block_sum(a, sh);
-  if (threadIdx.x == 0) {
-    st->pAp = pAp;
-    if (!(pAp > 0.0)) {
-      st->done = 1;  // breakdown: the residual is zero (or the operator is not positive definite)
-      st->alpha = 0.0;
+    if (c == b0) {
+      if constexpr (PASS != INIT) {
+        const unsigned int pass = 2u * (unsigned int)iter + (PASS == DIR ? 1u : 2u), mark = st->done;
+        if constexpr (PASS == DIR) {
+          if (iter > 0) {
+            const double before = st->rr[(iter - 1) & 1], limit = st->tol2 * st->bb;
+            const double rr = sum_parts<MT>(in, (int)gridDim.x, sh[0]);
+            if (mark && mark <= pass) return;
+            const bool end = rr <= limit;
+            if (blockIdx.x == 0 && threadIdx.x == 0) {
+              st->rr[iter & 1] = rr;
+              st->last = rr;
+              st->iters = (unsigned long long)iter;
+              if (end) st->done = pass + 1u;
+            }
+            if (end) return;
+            scale = rr / before;
+          } else if (mark) {
+            return;
+          }
+        } else {
+          const double rr = st->rr[iter & 1];
+          const double pAp = sum_parts<MT>(in, (int)gridDim.x, sh[0]);
+          if (mark && mark <= pass) return;
+          if (!(pAp > 0.0)) {  // breakdown: the residual is zero (or the operator is not positive definite)
+            if (blockIdx.x == 0 && threadIdx.x == 0) st->done = pass + 1u;
+            return;
+          }
+          scale = rr / pAp;
+        }
+      }
     } else {
-      st->alpha = st->rr / pAp;
+      __syncthreads();  // the buffers' last readers are done
+    }
+    double behind = form(wb.a, wb.b), cur = form(w.a, w.b);
+    place(first, w);
+    for (int64_t i = first; i != stop; i += d) {
+      const int64_t node = i * sx + col;
+      w = wn;
+      const double xv = xn, rv = rn;
+      if (i + d != stop) {
+        wn = load(i + d + d);
+        if constexpr (PASS == UPDATE) {
+          if (own) {
+            xn = x[node + d * sx];
+            rn = r[node + d * sx];
+          }
+        }
+      }
+      __syncthreads();  // plane i is in its buffer; the reads of plane i - d are done
+      const double ahead = form(w.a, w.b);
+      if (i + d != stop) place(i + d, w);
+      if (own) {
+        const int q = (int)(i & 1);
+        double nb = 0.0;
+        if (i > 0) nb += down ? ahead : behind;
+        if (i < A.lx - 1) nb += down ? behind : ahead;
+        if (j > 0) nb += pl[q][tj][tk + 1];
+        if (j < A.ly - 1) nb += pl[q][tj + 2][tk + 1];
+        if (k > 0) nb += pl[q][tj + 1][tk];
+        if (k < A.lz - 1) nb += pl[q][tj + 1][tk + 2];
+        const double ap = A.diag * cur - A.z * nb;
+        if constexpr (PASS == INIT) {
+          const double bv = rhs(A, cur, i, j, k, src, node);
+          const double res = bv - ap;
+          r[node] = res;
+          acc += res * res;
+          acc2 += bv * bv;
+        } else if constexpr (PASS == DIR) {
+          pnew[node] = cur;
+          acc += cur * ap;
+        } else {
+          x[node] = xv + scale * cur;
+          const double now = rv - scale * ap;
+          r[node] = now;
+          acc += now * now;
+        }
+      }
+      behind = cur;
+      cur = ahead;
     }
   }
-}
-
-__global__ __launch_bounds__(BD) void k_cg_update(int64_t total, double *__restrict__ x, double *__restrict__ r,
-                                                  const double *__restrict__ p, const double *__restrict__ Ap,
-                                                  int64_t chunk, const CGState *__restrict__ st,
-                                                  double *__restrict__ part) {
-  __shared__ double sh[BD / 64];
-  if (st->done) return;
-  const double alpha = st->alpha;
-  int64_t lo, hi;
-  block_range(total, chunk, lo, hi);
-  double acc = 0.0;
-  for (int64_t node = lo + threadIdx.x; node < hi; node += BD) {
-    x[node] += alpha * p[node];
-    const double rv = r[node] - alpha * Ap[node];
-    r[node] = rv;
-    acc += rv * rv;
+  const double s = block_sum<MT>(acc, sh[1]);
+  if (threadIdx.x == 0) out[b0] = s;
+  if constexpr (PASS == INIT) {
+    const double s2 = block_sum<MT>(acc2, sh[0]);
+    if (threadIdx.x == 0) out2[b0] = s2;
   }
-  const double s = block_sum(acc, sh);
-  if (threadIdx.x == 0) part[blockIdx.x] = s;
 }
 
-__global__ void k_cg_beta(const double *__restrict__ part, int nblk, int maxiter, CGState *st) {
-  __shared__ double sh[BD / 64];
-  if (st->done) return;
-  double a = 0.0;
-  for (int i = threadIdx.x; i < nblk; i += BD) a += part[i];
-  const double rr = block_sum(a, sh);
+__global__ __launch_bounds__(256) void k_cg_start(const double *__restrict__ part_rr,
+                                                  const double *__restrict__ part_bb, int nblk, double tol,
+                                                  int maxiter, CGState *st) {
+  __shared__ double sh[2][4];
+  const double rr = sum_parts<256>(part_rr, nblk, sh[0]), bb = sum_parts<256>(part_bb, nblk, sh[1]);
   if (threadIdx.x == 0) {
-    st->beta = rr / st->rr;
-    st->rr = rr;
-    st->iters += 1;
-    if (rr <= st->tol2 * st->bb || st->iters >= (unsigned long long)maxiter) st->done = 1;
+    st->rr[0] = st->last = rr;
+    st->bb = bb;
+    st->tol2 = tol * tol;
+    st->iters = 0;
+    st->done = (rr <= st->tol2 * bb || maxiter <= 0) ? 1u : 0u;
+  }
+}
+
+// after `iters` iterations: their residual, and whether to stop
+__global__ __launch_bounds__(256) void k_cg_check(const double *__restrict__ part, int nblk, int iters, int maxiter,
+                                                  CGState *st) {
+  __shared__ double sh[4];
+  if (st->done) return;
+  const double rr = sum_parts<256>(part, nblk, sh);
+  if (threadIdx.x == 0) {
+    st->last = rr;
+    st->iters = (unsigned long long)iters;
+    if (rr <= st->tol2 * st->bb || iters >= maxiter) st->done = 1u;
+  }
+}
+
+// The whole solve of a small grid in one workgroup: thread t holds x and r of
+// nodes t + ST m in registers, the direction lies in LDS.
+// Latency-bound: two barriers with a sum over 16 waves and one more an
+// iteration, 3 to 6 us against 12 to 14 us for the two streaming kernels.  17^3
+// with three iterations: 36 us a solve (62 us streaming); 22^3 with 100: 0.62
+// ms (1.3 ms).  Ten nodes a thread is the limit, as more spill: 25^3 took 1.4 ms
+// for 108 iterations, streaming 1.3 ms, and with three 92 us against 65 us.
+constexpr int ST = 1024;
+constexpr int64_t SMALL_NODES = 10 * ST;
+template <int NPT>
+__global__ __launch_bounds__(ST) void k_cg_small(Op A, const double *__restrict__ src, double *__restrict__ x,
+                                                 double tol, int maxiter, int substeps, CGState *st) {
+  __shared__ double p[ST * NPT];
+  __shared__ double sh[3][ST / 64];
+  const int lz = (int)A.lz, lyz = (int)(A.ly * A.lz), total = (int)(A.lx * lyz);
+  double xv[NPT], rv[NPT];
+  uint32_t in[NPT];  // which neighbours lie inside the grid: i-1, i+1, j-1, j+1, k-1, k+1
+#pragma unroll
+  for (int m = 0; m < NPT; ++m) {
+    const int node = (int)threadIdx.x + ST * m;
+    const int i = node / lyz, j = (node - i * lyz) / lz, k = node - i * lyz - j * lz;
+    in[m] = (i > 0 ? 1u : 0u) | (i < (int)A.lx - 1 ? 2u : 0u) | (j > 0 ? 4u : 0u) | (j < (int)A.ly - 1 ? 8u : 0u) |
+            (k > 0 ? 16u : 0u) | (k < lz - 1 ? 32u : 0u);
+    xv[m] = node < total ? x[node] : 0.0;
+  }
+  auto apply = [&](int node, uint32_t w) -> double {
+    double nb = 0.0;
+    if (w & 1u) nb += p[node - lyz];
+    if (w & 2u) nb += p[node + lyz];
+    if (w & 4u) nb += p[node - lz];
+    if (w & 8u) nb += p[node + lz];
+    if (w & 16u) nb += p[node - 1];
+    if (w & 32u) nb += p[node + 1];
+    return A.diag * p[node] - A.z * nb;
+  };
+  const double tol2 = tol * tol;
+  unsigned long long its = 0;
+  double rr = 0.0, bb = 0.0;
+  for (int s = 0; s < substeps; ++s) {
+    __syncthreads();
+#pragma unroll
+    for (int m = 0; m < NPT; ++m) {
+      const int node = (int)threadIdx.x + ST * m;
+      if (node < total) p[node] = xv[m];
+    }
+    __syncthreads();
+    double a = 0.0, c = 0.0;
+#pragma unroll
+    for (int m = 0; m < NPT; ++m) {
+      const int node = (int)threadIdx.x + ST * m;
+      rv[m] = 0.0;
+      if (node < total) {
+        const uint32_t w = in[m];
+        double b = xv[m];
+        if (!(w & 1u)) b += A.zbc;
+        if (!(w & 2u)) b += A.zbc;
+        if (!(w & 4u)) b += A.zbc;
+        if (!(w & 8u)) b += A.zbc;
+        if (!(w & 16u)) b += A.zbc;
+        if (!(w & 32u)) b += A.zbc;
+        if (src) b += src[node];
+        rv[m] = b - apply(node, w);
+        a += rv[m] * rv[m];
+        c += b * b;
+      }
+    }
+    rr = block_sum<ST>(a, sh[0]);
+    bb = block_sum<ST>(c, sh[1]);
+    double beta = 0.0;
+    for (int it = 0; it < maxiter && !(rr <= tol2 * bb); ++it) {
+#pragma unroll
+      for (int m = 0; m < NPT; ++m) {
+        const int node = (int)threadIdx.x + ST * m;
+        if (node < total) p[node] = it > 0 ? rv[m] + beta * p[node] : rv[m];
+      }
+      __syncthreads();
+      double ap[NPT];
+      a = 0.0;
+#pragma unroll
+      for (int m = 0; m < NPT; ++m) {
+        const int node = (int)threadIdx.x + ST * m;
+        ap[m] = 0.0;
+        if (node < total) {
+          ap[m] = apply(node, in[m]);
+          a += p[node] * ap[m];
+        }
+      }
+      const double pAp = block_sum<ST>(a, sh[2]);
+      if (!(pAp > 0.0)) break;
+      const double alpha = rr / pAp;
+      a = 0.0;
+#pragma unroll
+      for (int m = 0; m < NPT; ++m) {
+        const int node = (int)threadIdx.x + ST * m;
+        if (node < total) {
+          xv[m] += alpha * p[node];
+          rv[m] -= alpha * ap[m];
+          a += rv[m] * rv[m];
+        }
+      }
+      const double now = block_sum<ST>(a, sh[it & 1]);
+      beta = now / rr;
+      rr = now;
+      ++its;
+    }
+  }
+#pragma unroll
+  for (int m = 0; m < NPT; ++m) {
+    const int node = (int)threadIdx.x + ST * m;
+    if (node < total) x[node] = xv[m];
+  }
+  if (threadIdx.x == 0) {
+    st->bb = bb;
+    st->last = rr;
+    st->iters = its;
+    st->done = 1u;
   }
 }
 
 }  // namespace
 
-// doubles of work memory for a grid of `total` nodes: b, r, two directions,
-// Ap; two arrays of partial sums; the state
+// doubles of work memory for a grid of `total` nodes: r and two directions;
+// three arrays of partial sums; the state
 static constexpr int64_t work_doubles(int64_t total) {
-  return 5 * total + 2 * MAXBLK + (int64_t)((sizeof(CGState) + 7) / 8);
+  return 3 * total + 3 * MAXBLK + (int64_t)((sizeof(CGState) + 7) / 8);
 }
 
 // The allocation-free entry point's work memory: one buffer per device, in
@@ -340,23 +449,54 @@ constexpr int MAX_DEVICES = 64;
 static std::mutex scratch_mu;
 static double *scratch_addr[MAX_DEVICES];
 
+// (j, k) blocks times runs of planes: the number of runs that takes the
+// fullest of 256 CUs the fewest planes, each run costing RUN_COST planes more
+// (it reads one more at either end, and every workgroup adds all the partial
+// sums).  A CU needs two workgroups to be busy, so one counts as two.
+static Blocks blocks_for(int64_t lx, int64_t ly, int64_t lz) {
+  constexpr int64_t CUS = 256, FULL = 1024 / MT, MOST = 4 * FULL * CUS / 2, MIN_RUN = 2, RUN_COST = 3;
+  Blocks B;
+  B.nk = (unsigned int)((lz + MK - 1) / MK);
+  B.nj = (unsigned int)((ly + MJ - 1) / MJ);
+  const int64_t ncol = (int64_t)B.nk * B.nj;
+  int64_t best = 0;
+  for (int64_t nseg = 1; nseg == 1 || (nseg * MIN_RUN <= lx + 1 && nseg * ncol <= MOST); ++nseg) {
+    const int64_t run = (lx + nseg - 1) / nseg, count = ncol * ((lx + run - 1) / run);
+    const int64_t cost = std::max((count + CUS - 1) / CUS, FULL) * (run + RUN_COST);
+    if (nseg > 1 && cost >= best) continue;
+    best = cost;
+    B.run = (unsigned int)run;
+    B.count = (unsigned int)count;
+  }
+  return B;
+}
+
+// CG's bound on the iterations to a relative residual of tol, from the
+// operator's least and greatest eigenvalue
+static double iterations_for(const Op &A, double tol) {
+  const double n = 2.0 * A.z * (cos(M_PI / (double)(A.lx + 1)) + cos(M_PI / (double)(A.ly + 1)) +
+                                cos(M_PI / (double)(A.lz + 1)));
+  const double k = sqrt((A.diag + n) / (A.diag - n));
+  const double its = log(2.0 / std::max(tol, 1e-300)) / log((k + 1.0) / (k - 1.0));
+  return its > 1.0 ? its : 1.0;  // (one also where there is no such number)
+}
+
 // the solve with its work arrays at `work` (work_doubles(total) doubles)
 static tm_status run_diffusion(tm_ctx *c, double *work, const tm_grid *g, const tm_diffusion *d, const double *src,
                                double *field, int32_t *iterations, double *residual) {
-  const int64_t lx = g->localsize[0], ly = g->localsize[1], lz = g->localsize[2];
+  int64_t lx = g->localsize[0], ly = g->localsize[1], lz = g->localsize[2];
   const int64_t total = lx * ly * lz;
-  double *b = work, *r = b + total, *p0 = r + total, *p1 = p0 + total, *Ap = p1 + total;
-  double *part = Ap + total, *part2 = part + MAXBLK;
-  CGState *st = (CGState *)(part2 + MAXBLK);
-  const int64_t nblk0 = std::min<int64_t>(MAXBLK, (total + BD - 1) / BD);
-  const int64_t chunk = (((total + nblk0 - 1) / nblk0) + BD - 1) / BD * BD;
-  const int nblk = (int)((total + chunk - 1) / chunk);
-  // the marching direction kernel: (j, k) blocks times runs of planes, about
-  // 2,048 workgroups, at most MAXBLK (else the one-lane-per-node kernel)
-  const int64_t ncol = ((ly + MJ - 1) / MJ) * ((lz + MK - 1) / MK);
-  const int nseg = (int)std::max<int64_t>(1, std::min<int64_t>(lx, std::max<int64_t>(1, 2048 / ncol)));
-  const bool march = ncol * nseg <= MAXBLK;
-  const int nblk_dir = march ? (int)(ncol * nseg) : nblk;
+  // Axes of one node go to the front, where the passes march: the layout, the
+  // order of a node's neighbours and its six equal face terms stay the same.
+  for (int q = 0; q < 2 && lz == 1; ++q) {
+    lz = ly;
+    ly = lx;
+    lx = 1;
+  }
+  if (ly == 1) std::swap(lx, ly);
+  double *r = work, *p0 = r + total, *p1 = p0 + total;
+  double *part = p1 + total, *part2 = part + MAXBLK, *partb = part2 + MAXBLK;
+  CGState *st = (CGState *)(partb + MAXBLK);
   Op A;
   A.lx = lx;
   A.ly = ly;
@@ -364,36 +504,53 @@ static tm_status run_diffusion(tm_ctx *c, double *work, const tm_grid *g, const 
   const float res2 = g->resolution * g->resolution;  // FP32 product, as the reference forms it
   A.z = d->diffusion * d->dt / (double)res2;
   A.diag = 1 + 6.0 * A.z + d->lambda * d->dt;
-  const double zbc = A.z * d->boundary;
+  A.zbc = A.z * d->boundary;
   int32_t it_total = 0;
   double last_res = 0.0;
-  for (int s = 0; s < d->substeps; ++s) {
-    k_cg_init<<<nblk, BD, 0, c->stream>>>(A, zbc, src, field, b, r, p0, chunk, part, part2);
-    k_cg_start<<<1, BD, 0, c->stream>>>(part, part2, nblk, d->tol, d->maxiter, st);
+  // the state is read back into pinned host memory set aside at tm_create
+  CGState &h = *reinterpret_cast<CGState *>(c->h_flags + TM_HFLAGS_CG);
+  auto read_state = [&]() -> tm_status {
     TM_HIP(c, hipGetLastError());
-    // p0 holds r for the first direction (beta = 0); the directions then alternate
-    double *pold = p0, *pnew = p1;
-    int32_t launched = 0;
-    // the state is read back into pinned host memory set aside at tm_create
-    CGState &h = *reinterpret_cast<CGState *>(c->h_flags + TM_HFLAGS_CG);
-    for (;;) {
-      const int32_t batch = std::min<int32_t>(8, d->maxiter - launched);
-      for (int32_t q = 0; q < batch; ++q) {
-        if (march) k_cg_dir_march<<<nblk_dir, MT, 0, c->stream>>>(A, r, pold, pnew, Ap, nseg, st, part);
-        else k_cg_dir<<<nblk, BD, 0, c->stream>>>(A, r, pold, pnew, Ap, chunk, st, part);
-        k_cg_alpha<<<1, BD, 0, c->stream>>>(part, nblk_dir, st);
-        k_cg_update<<<nblk, BD, 0, c->stream>>>(total, field, r, pnew, Ap, chunk, st, part);
-        k_cg_beta<<<1, BD, 0, c->stream>>>(part, nblk, d->maxiter, st);
-        std::swap(pold, pnew);
-      }
-      launched += batch;
-      TM_HIP(c, hipGetLastError());
-      TM_HIP(c, hipMemcpyAsync(&h, st, sizeof(CGState), hipMemcpyDeviceToHost, c->stream));
-      TM_HIP(c, hipStreamSynchronize(c->stream));
-      if (h.done || launched >= d->maxiter || batch == 0) break;
-    }
+    TM_HIP(c, hipMemcpyAsync(&h, st, sizeof(CGState), hipMemcpyDeviceToHost, c->stream));
+    TM_HIP(c, hipStreamSynchronize(c->stream));
+    last_res = h.bb > 0.0 ? sqrt(h.last / h.bb) : sqrt(h.last);
     it_total += (int32_t)h.iters;
-    last_res = h.bb > 0.0 ? sqrt(h.rr / h.bb) : sqrt(h.rr);
+    return TM_OK;
+  };
+  if (total <= SMALL_NODES && d->substeps > 0) {
+    auto kern = total <= ST * 5 ? k_cg_small<5> : k_cg_small<10>;
+    kern<<<1, ST, 0, c->stream>>>(A, src, field, d->tol, d->maxiter, d->substeps, st);
+    TM_TRY(read_state());
+  } else {
+    const Blocks B = blocks_for(lx, ly, lz);
+    const int nblk = (int)std::min<unsigned int>(MAXBLK, B.count);
+    // most iterations are launched before the first look at the state (CG takes
+    // 0.7 to 0.9 of its bound), the others a few at a time
+    const int32_t first = (int32_t)std::min(0.8 * iterations_for(A, d->tol) + 1.0, 256.0);
+    for (int s = 0; s < d->substeps; ++s) {
+      k_cg<INIT><<<nblk, MT, 0, c->stream>>>(A, src, field, r, nullptr, nullptr, B, 0, st, nullptr,
+                                             part2, partb);
+      k_cg_start<<<1, 256, 0, c->stream>>>(part2, partb, nblk, d->tol, d->maxiter, st);
+      // the first direction is r; the two arrays then alternate
+      double *pold = p0, *pnew = p1;
+      int32_t launched = 0;
+      for (;;) {
+        const int32_t batch = std::min(launched ? std::min(std::max(4, launched / 8), 64) : first, d->maxiter - launched);
+        for (int32_t q = launched; q < launched + batch; ++q) {
+          k_cg<DIR><<<nblk, MT, 0, c->stream>>>(A, nullptr, nullptr, r, pold, pnew, B, q, st, part2,
+                                                part, nullptr);
+          k_cg<UPDATE><<<nblk, MT, 0, c->stream>>>(A, nullptr, field, r, pnew, nullptr, B, q, st, part,
+                                                   part2, nullptr);
+          std::swap(pold, pnew);
+        }
+        launched += batch;
+        if (batch > 0) k_cg_check<<<1, 256, 0, c->stream>>>(part2, nblk, launched, d->maxiter, st);
+        const int32_t before = it_total;
+        TM_TRY(read_state());
+        if (h.done || launched >= d->maxiter || batch == 0) break;
+        it_total = before;
+      }
+    }
   }
   if (iterations) *iterations = it_total;
   if (residual) *residual = last_res;
