@@ -291,7 +291,7 @@ tm_status tm_diffusion_step(tm_ctx *ctx, const tm_grid *grid, const tm_diffusion
  * hipMalloc): identical kernels and results, but the work arrays (right-hand
  * side, residual, two directions, A p, partial sums, solver state) live in
  * one static device buffer of the library, sized for grids of at most
- * TM_NOALLOC_MAX_NODES nodes (about 80 MiB, held on every device the library
+ * TM_NOALLOC_MAX_NODES nodes (about 48 MiB, held on every device the library
  * runs on until the process ends).  The call allocates nothing; larger grids
  * are refused with TM_ERR_INVALID.  Every context on one device shares that
  * buffer: calls that overlap on one device (two host threads, or two

@@ -9,7 +9,7 @@
 //   cicCoord = lower + (double)((float)cellIdx * resolution)   the product is
 //              int64 * float, evaluated in float by C's usual conversions
 //   d = (x - cicCoord) / resolution, t = 1 - d, corner weight a*d + (1-a)*t
-// so corner indices match bit for bit and the interpolation (one lane per
+// so corner indices match bit for bit and the interpolation (four lanes per
 // cell, corners in the reference's ax, ay, az order) matches bit for bit.
 // The deposit sums the reference's terms into each node owned by a grid
 // tile in LDS (k_dep_tile): the same terms in a different order (<= ~1e-15
@@ -454,63 +454,177 @@ __global__ __launch_bounds__(DEP_T) void k_dep_tile(const double4 *__restrict__ 
   }
 }
 
+// A lane sets up one cell (its node, weights and place in the output) and
+// leaves that in LDS; then four lanes serve each of the wave's cells, 16 cells
+// at a time.  The two nodes of an (ax, ay) row are next to each other along z:
+// the four lanes read the row's two field values (lane 0) and six gradient
+// values (lanes 1 to 3), two each, and trade them so that lane q adds
+// component q in the reference's order and stores it.  Cells at the grid's
+// faces are left to their own lane.
+//
+// Bound by memory, the lines of field and gradient that the cells touch and the
+// scattered 32-byte results, once the address units are: a lane per cell with
+// a load per value took 32 divergent loads a cell, 239 us for 2M cells over
+// 256^3 FP64 and 511 us for 5M over 384^3 FP32; with the widest loads per lane
+// 178 (alone) and 396 us; four lanes a cell, so that a load's 64 lanes touch 16
+// or 32 lines instead of 64, 148 (alone) and 354 us.
+struct alignas(16) InterpCell {
+  double w[6];   // weight of ax = 0, 1, of ay = 0, 1, of az = 0, 1
+  int64_t node;  // of corner (0, 0, 0)
+  int32_t o;     // the cell's place in the output, or -1
+  int32_t pad[5];  // 80 bytes: 16 cells' 16-byte reads fall on different banks
+};
+
+// lane q's value from lane p of its four, p = P0..P3 for q = 0..3
+template <int P0, int P1, int P2, int P3, typename F>
+__device__ __forceinline__ F quad_perm(F v) {
+  constexpr int ctrl = P0 | (P1 << 2) | (P2 << 4) | (P3 << 6);
+  if constexpr (sizeof(F) == 4) {
+    return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), ctrl, 0xf, 0xf, true));
+  } else {
+    return __hiloint2double(__builtin_amdgcn_mov_dpp(__double2hiint(v), ctrl, 0xf, 0xf, true),
+                            __builtin_amdgcn_mov_dpp(__double2loint(v), ctrl, 0xf, 0xf, true));
+  }
+}
+
 template <typename F>
 __global__ __launch_bounds__(256) void k_interp(const double4 *__restrict__ pos, const int32_t *__restrict__ perm,
                                                 int64_t n, GridDev g, const F *__restrict__ field,
                                                 const F *__restrict__ grad, double *__restrict__ out) {
+  typedef F two __attribute__((ext_vector_type(2), aligned(sizeof(F))));
+  __shared__ InterpCell cells[4][64];
   const int64_t i = tm_xcd_block() * 256 + threadIdx.x;
-  if (i >= n) return;
-  const double4 P = pos[i];
-  int64_t ci[3];
-  double d[3], t[3];
-  cic_setup(g, P.x, P.y, P.z, ci, d, t);
-  double val = 0.0, gx = 0.0, gy = 0.0, gz = 0.0;
+  const int lane = threadIdx.x & 63, q = lane & 3;
+  InterpCell *wc = cells[threadIdx.x >> 6];
+  const int64_t sy = g.ls[2], sx = g.ls[1] * g.ls[2];
+  int32_t mine = -1;
+  if (i < n) {
+    const double4 P = pos[i];
+    const int32_t o = perm[i];
+    int64_t ci[3];
+    double d[3], t[3];
+    cic_setup(g, P.x, P.y, P.z, ci, d, t);
+    double w[6];
 #pragma unroll
-  for (int ax = 0; ax < 2; ++ax)
+    for (int a = 0; a < 3; ++a) {
+      w[2 * a] = 0 * d[a] + 1 * t[a];
+      w[2 * a + 1] = 1 * d[a] + 0 * t[a];
+    }
+    auto node_of = [&](int ax, int ay, int az) -> int64_t {
+      return ((ci[0] + ax - g.lo[0]) * g.ls[1] + (ci[1] + ay - g.lo[1])) * g.ls[2] + (ci[2] + az - g.lo[2]);
+    };
+    if (cic_inrange(g, ci, 0, 0, 0) && cic_inrange(g, ci, 1, 1, 1)) {
+      mine = o;
 #pragma unroll
-    for (int ay = 0; ay < 2; ++ay)
-#pragma unroll
-      for (int az = 0; az < 2; ++az) {
+      for (int a = 0; a < 6; ++a) wc[lane].w[a] = w[a];
+      wc[lane].node = node_of(0, 0, 0);
+    } else {
+      double4 r = make_double4(0.0, 0.0, 0.0, 0.0);
+      for (int c = 0; c < 8; ++c) {
+        const int ax = c >> 2, ay = (c >> 1) & 1, az = c & 1;
         if (!cic_inrange(g, ci, ax, ay, az)) continue;
-        const int64_t node = ((ci[0] + ax - g.lo[0]) * g.ls[1] + (ci[1] + ay - g.lo[1])) * g.ls[2] +
-                             (ci[2] + az - g.lo[2]);
-        const double wx = (ax * d[0] + (1 - ax) * t[0]);
-        const double wy = (ay * d[1] + (1 - ay) * t[1]);
-        const double wz = (az * d[2] + (1 - az) * t[2]);
-        val += (double)field[node] * wx * wy * wz;
-        gx += (double)grad[3 * node + 0] * wx * wy * wz;
-        gy += (double)grad[3 * node + 1] * wx * wy * wz;
-        gz += (double)grad[3 * node + 2] * wx * wy * wz;
+        const int64_t node = node_of(ax, ay, az);
+        const double wx = ax ? w[1] : w[0], wy = ay ? w[3] : w[2], wz = az ? w[5] : w[4];
+        r.x += (double)field[node] * wx * wy * wz;
+        r.y += (double)grad[3 * node + 0] * wx * wy * wz;
+        r.z += (double)grad[3 * node + 1] * wx * wy * wz;
+        r.w += (double)grad[3 * node + 2] * wx * wy * wz;
       }
-  const int64_t o = perm[i];
-  double4 r = make_double4(val, gx, gy, gz);
-  reinterpret_cast<double4 *>(out)[o] = r;
+      reinterpret_cast<double4 *>(out)[o] = r;
+    }
+  }
+  wc[lane].o = mine;
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+#pragma unroll
+  for (int h = 0; h < 4; ++h) {
+    const InterpCell *c = wc + 16 * h + (lane >> 2);
+    const int32_t o = c->o;
+    if (o < 0) continue;  // (all four lanes of the cell)
+    const int64_t node = c->node;
+    const F *src = q == 0 ? field + node : grad + 3 * node + 2 * (q - 1);
+    const int64_t dx = q == 0 ? sx : 3 * sx, dy = q == 0 ? sy : 3 * sy;
+    two v[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v[e] = *(const two *)(src + (e >> 1) * dx + (e & 1) * dy);
+    double acc = 0.0;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      // the row: (v0, v1), (gx0, gy0), (gz0, gx1), (gy1, gz1)
+      const F x0 = quad_perm<0, 1, 1, 2>(v[e].x), y0 = quad_perm<1, 1, 1, 1>(v[e].y);
+      const F y1 = quad_perm<0, 2, 2, 3>(v[e].y), x1 = quad_perm<3, 3, 3, 3>(v[e].x);
+      const F a0 = q == 2 ? y0 : x0, a1 = q == 2 ? x1 : y1;
+      acc += (double)a0 * c->w[e >> 1] * c->w[2 + (e & 1)] * c->w[4];
+      acc += (double)a1 * c->w[e >> 1] * c->w[2 + (e & 1)] * c->w[5];
+    }
+    out[4 * (int64_t)o + q] = acc;
+  }
 }
 
-// one lane per node, k fastest; faces one-sided (no neighbouring ranks)
+// interior (f[i+1]-f[i-1])/res; faces one-sided (no neighbouring ranks):
+// (f[1]-f[0])/res, (f[L-1]-f[L-2])/res
+//
+// A lane owns one (j, k) column of a run of planes and marches along i, so that
+// its i neighbours stay in registers; the j and k neighbours come from the
+// caches.  A wave's 64 nodes are consecutive in the plane: their 192 results go
+// through LDS and out in 16-byte stores that pass by the caches: three times the
+// field, they would push it out of the memory-side cache and be gone before
+// they are read.  256^3 FP64 (134 MB in, 403 MB out): 158 us with a lane per
+// node and strided stores, 149 us marching, 79 us with such stores (6.8 TB/s,
+// the field partly from that cache); 384^3 FP32: 267, 237, 137 us.
 template <typename F>
 __global__ __launch_bounds__(256) void k_gradient(const F *__restrict__ f, F *__restrict__ g, int64_t lx, int64_t ly,
-                                                  int64_t lz, float res) {
-  const int64_t node = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  const int64_t total = lx * ly * lz;
-  if (node >= total) return;
-  const int64_t k = node % lz;
-  const int64_t j = (node / lz) % ly;
-  const int64_t i = node / (lz * ly);
-  const int64_t sx = ly * lz, sy = lz;
-  // interior (f[i+1]-f[i-1])/res; faces (f[1]-f[0])/res, (f[L-1]-f[L-2])/res
-  const int64_t ip = (i == lx - 1) ? node : node + sx, im = (i == 0) ? node : node - sx;
-  const int64_t jp = (j == ly - 1) ? node : node + sy, jm = (j == 0) ? node : node - sy;
-  const int64_t kp = (k == lz - 1) ? node : node + 1, km = (k == 0) ? node : node - 1;
-  F r = (F)res;
-  if (sizeof(F) == 8) {
-    g[3 * node + 0] = (F)(((double)f[ip] - (double)f[im]) / (double)res);
-    g[3 * node + 1] = (F)(((double)f[jp] - (double)f[jm]) / (double)res);
-    g[3 * node + 2] = (F)(((double)f[kp] - (double)f[km]) / (double)res);
-  } else {
-    g[3 * node + 0] = (f[ip] - f[im]) / r;
-    g[3 * node + 1] = (f[jp] - f[jm]) / r;
-    g[3 * node + 2] = (f[kp] - f[km]) / r;
+                                                  int64_t lz, unsigned int nchunk, int64_t run, float res) {
+  constexpr int E = 16 / (int)sizeof(F);
+  typedef F vec __attribute__((ext_vector_type(E), aligned(sizeof(F))));
+  typedef F lvec __attribute__((ext_vector_type(E)));
+  __shared__ __align__(16) F stage[4][3 * 64];
+  const unsigned int b = (unsigned int)tm_xcd_block();
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int64_t plane = ly * lz, m0 = (int64_t)(b % nchunk) * 256 + wave * 64;
+  const int64_t i0 = (int64_t)(b / nchunk) * run, i1 = i0 + run < lx ? i0 + run : lx;
+  if (m0 >= plane) return;
+  const int64_t m = m0 + lane < plane ? m0 + lane : plane - 1;  // lanes past the plane repeat its last node
+  const int64_t j = m / lz, k = m - j * lz;
+  const int nv = 3 * (int)(plane - m0 < 64 ? plane - m0 : 64);
+  const int64_t jm = j > 0 ? -lz : 0, jp = j < ly - 1 ? lz : 0;
+  const int km = k > 0 ? -1 : 0, kp = k < lz - 1 ? 1 : 0;
+  struct Cross {
+    F jm, jp, km, kp;
+  };
+  auto cross = [&](const F *q) -> Cross { return Cross{q[jm], q[jp], q[km], q[kp]}; };
+  const F *c = f + i0 * plane + m;
+  F cur = c[0], prev = i0 > 0 ? c[-plane] : cur, next = i0 < lx - 1 ? c[plane] : cur;
+  Cross x = cross(c);
+  F *st = stage[wave];
+  for (int64_t i = i0; i < i1; ++i, c += plane) {
+    F after = next;
+    Cross xn = x;
+    if (i + 1 < i1) {
+      if (i + 2 < lx) after = c[2 * plane];
+      xn = cross(c + plane);
+    }
+    if constexpr (sizeof(F) == 8) {
+      st[3 * lane + 0] = (F)(((double)next - (double)prev) / (double)res);
+      st[3 * lane + 1] = (F)(((double)x.jp - (double)x.jm) / (double)res);
+      st[3 * lane + 2] = (F)(((double)x.kp - (double)x.km) / (double)res);
+    } else {
+      st[3 * lane + 0] = (next - prev) / (F)res;
+      st[3 * lane + 1] = (x.jp - x.jm) / (F)res;
+      st[3 * lane + 2] = (x.kp - x.km) / (F)res;
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    F *dst = g + 3 * (i * plane + m0);
+    for (int v = lane; v < nv / E; v += 64) __builtin_nontemporal_store(*(const lvec *)(st + E * v), (vec *)(dst + E * v));
+    const int rest = nv / E * E + lane;
+    if (rest < nv) dst[rest] = st[rest];
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    prev = cur;
+    cur = next;
+    next = after;
+    x = xn;
   }
 }
 
@@ -601,9 +715,12 @@ static tm_status gradient_impl(tm_ctx *c, const tm_grid *grid, const F *field, F
   if (!c) return TM_ERR_INVALID;
   TM_TRY(check_grid(c, grid));
   if (!field || !gradient) return tm_fail(c, TM_ERR_INVALID, "field or gradient is NULL");
-  const int64_t total = grid->localsize[0] * grid->localsize[1] * grid->localsize[2];
-  k_gradient<F><<<tm_blocks(total, 256), 256, 0, c->stream>>>(field, gradient, grid->localsize[0], grid->localsize[1],
-                                                               grid->localsize[2], grid->resolution);
+  // chunks of 256 columns times runs of planes: about 2,048 workgroups, runs of
+  // at least four planes
+  const int64_t lx = grid->localsize[0], nchunk = tm_blocks(grid->localsize[1] * grid->localsize[2], 256);
+  const int64_t want = std::max<int64_t>(1, std::min<int64_t>((lx + 3) / 4, 2048 / nchunk)), run = (lx + want - 1) / want;
+  k_gradient<F><<<(unsigned)(nchunk * ((lx + run - 1) / run)), 256, 0, c->stream>>>(
+      field, gradient, lx, grid->localsize[1], grid->localsize[2], (unsigned)nchunk, run, grid->resolution);
   TM_HIP(c, hipGetLastError());
   return TM_OK;
 }
@@ -621,7 +738,14 @@ static tm_status interp_impl(tm_ctx *c, const tm_grid *grid, const F *field, con
   TM_TRY(check_cells_grid(c, grid));
   if (!field || !gradient || !out) return tm_fail(c, TM_ERR_INVALID, "NULL array");
   if (c->n == 0) return TM_OK;
-  k_interp<F><<<tm_blocks(c->n, 256), 256, 0, c->stream>>>(c->d_pos, c->d_perm, c->n, to_dev(grid), field, gradient,
+  // Where field and gradient do not fit the L2 caches (8 x 4 MB), three
+  // workgroups a CU instead of eight, by their LDS: more evict each other's
+  // lines.  384^3 FP32, 5M cells: 321 against 354 us, with two or four 335 us;
+  // 256^3 FP64, 2M: 132 against 148 us.  Below, more in flight win: 100^3 FP64,
+  // 300K: 13 against 14 us.
+  const int64_t bytes = 4 * (int64_t)sizeof(F) * grid->localsize[0] * grid->localsize[1] * grid->localsize[2];
+  const size_t lds = bytes > (int64_t)32 << 20 ? 30 << 10 : 0;
+  k_interp<F><<<tm_blocks(c->n, 256), 256, lds, c->stream>>>(c->d_pos, c->d_perm, c->n, to_dev(grid), field, gradient,
                                                             out);
   TM_HIP(c, hipGetLastError());
   return TM_OK;
