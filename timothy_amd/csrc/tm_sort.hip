@@ -1,8 +1,9 @@
 // Device-wide exclusive scan and stable LSD radix sort of (u64 key, i32 value)
 // pairs, 8-bit digits, for the Morton ordering of cells.
 //
-// Each pass: histogram per 4096-key tile (LDS atomics) -> exclusive scan of
-// the digit-major histogram -> stable scatter.  Stable ranks inside a tile
+// Each pass: histogram per tile (LDS atomics) -> exclusive scan of the
+// digit-major histogram (up to FEW_N keys each tile of the scatter adds up the
+// tiles' histograms itself) -> stable scatter.  Stable ranks inside a tile
 // come from 64-lane ballots: the lanes holding the same digit are found with
 // eight ballots, the leader of each group advances a per-wave digit counter
 // in LDS.
@@ -11,8 +12,6 @@
 namespace {
 
 constexpr int RS_THREADS = 256;
-constexpr int RS_ITEMS = 16;
-constexpr int RS_TILE = RS_THREADS * RS_ITEMS;
 constexpr int RS_WAVES = RS_THREADS / 64;
 
 constexpr int SC_THREADS = 256;
@@ -31,8 +30,10 @@ __device__ __forceinline__ unsigned long long tm_match8(uint32_t d, bool valid) 
   return m;
 }
 
+template <int RS_ITEMS, bool FEW>
 __global__ __launch_bounds__(RS_THREADS) void k_rs_hist(const uint64_t *__restrict__ keys, int64_t n, int shift,
                                                         uint32_t *__restrict__ hist, int nblocks) {
+  constexpr int RS_TILE = RS_THREADS * RS_ITEMS;
   __shared__ uint32_t h[RS_WAVES][256];
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
   for (int j = tid; j < RS_WAVES * 256; j += RS_THREADS) (&h[0][0])[j] = 0;
@@ -53,7 +54,7 @@ __global__ __launch_bounds__(RS_THREADS) void k_rs_hist(const uint64_t *__restri
   uint32_t s = 0;
 #pragma unroll
   for (int k = 0; k < RS_WAVES; ++k) s += h[k][tid];
-  hist[(int64_t)tid * nblocks + blockIdx.x] = s;
+  hist[FEW ? (int64_t)blockIdx.x * 256 + tid : (int64_t)tid * nblocks + blockIdx.x] = s;
 }
 
 // Exclusive scan of each digit's row of per-tile counts (one workgroup per
@@ -92,11 +93,13 @@ __global__ __launch_bounds__(RS_THREADS) void k_rs_rowscan(uint32_t *__restrict_
 // The tile's keys are ranked stably (by digit, then input order), placed in
 // LDS in that order, and written out from there: consecutive lanes write
 // consecutive slots of one digit's run instead of 64 scattered records.
+template <int RS_ITEMS, bool FEW>
 __global__ __launch_bounds__(RS_THREADS) void k_rs_scatter(const uint64_t *__restrict__ keys,
                                                            const int32_t *__restrict__ vals,
                                                            uint64_t *__restrict__ okeys, int32_t *__restrict__ ovals,
                                                            int64_t n, int shift, const uint32_t *__restrict__ offs,
                                                            int nblocks) {
+  constexpr int RS_TILE = RS_THREADS * RS_ITEMS;
   __shared__ uint32_t cnt[RS_WAVES][256];
   __shared__ uint32_t pre[RS_WAVES][256];
   __shared__ uint32_t gbase[256];
@@ -106,26 +109,6 @@ __global__ __launch_bounds__(RS_THREADS) void k_rs_scatter(const uint64_t *__res
   __shared__ int32_t sval[RS_TILE];
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
   for (int j = tid; j < RS_WAVES * 256; j += RS_THREADS) (&cnt[0][0])[j] = 0;
-  // this tile's first slot for digit tid: its row prefix (offs, per digit
-  // over the tiles) plus the keys of all smaller digits (the row totals
-  // after the rows, scanned here)
-  {
-    const uint32_t rt = offs[(int64_t)256 * nblocks + tid];
-    uint32_t inc = rt;
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-      const uint32_t y = __shfl_up(inc, o, 64);
-      if (lane >= o) inc += y;
-    }
-    if (lane == 63) wsum[w] = inc;
-    __syncthreads();
-    uint32_t wb = 0;
-#pragma unroll
-    for (int q = 0; q < RS_WAVES; ++q)
-      if (q < w) wb += wsum[q];
-    gbase[tid] = offs[(int64_t)tid * nblocks + blockIdx.x] + wb + inc - rt;
-    __syncthreads();
-  }
   const int64_t tile0 = (int64_t)blockIdx.x * RS_TILE;
   const int64_t base = tile0 + (int64_t)w * (64 * RS_ITEMS);
   uint64_t k[RS_ITEMS];
@@ -138,7 +121,41 @@ __global__ __launch_bounds__(RS_THREADS) void k_rs_scatter(const uint64_t *__res
     k[it] = valid ? keys[i] : 0ull;
     v[it] = valid ? vals[i] : 0;
   }
-  __syncthreads();
+  // this tile's first slot for digit tid: its keys in the tiles before (FEW:
+  // added up here, else scanned by k_rs_rowscan) plus the keys of all smaller
+  // digits (the digits' totals, scanned here)
+  {
+    uint32_t rt = 0, before = 0;
+    if constexpr (FEW) {
+      for (int b = 0; b < nblocks; b += 16) {
+        uint32_t h[16];
+#pragma unroll
+        for (int q = 0; q < 16; ++q) h[q] = b + q < nblocks ? offs[(b + q) * 256 + tid] : 0u;
+#pragma unroll
+        for (int q = 0; q < 16; ++q) {
+          rt += h[q];
+          if (b + q < (int)blockIdx.x) before += h[q];
+        }
+      }
+    } else {
+      rt = offs[(int64_t)256 * nblocks + tid];
+      before = offs[(int64_t)tid * nblocks + blockIdx.x];
+    }
+    uint32_t inc = rt;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      const uint32_t y = __shfl_up(inc, o, 64);
+      if (lane >= o) inc += y;
+    }
+    if (lane == 63) wsum[w] = inc;
+    __syncthreads();
+    uint32_t wb = 0;
+#pragma unroll
+    for (int q = 0; q < RS_WAVES; ++q)
+      if (q < w) wb += wsum[q];
+    gbase[tid] = before + wb + inc - rt;
+    __syncthreads();
+  }
 #pragma unroll
   for (int it = 0; it < RS_ITEMS; ++it) {
     const bool valid = base + it * 64 + lane < n;
@@ -297,29 +314,42 @@ tm_status tm_scan_u32(tm_ctx *c, const uint32_t *in, uint32_t *out, int64_t n) {
   return TM_OK;
 }
 
+template <int ITEMS, bool FEW>
+static tm_status sort_passes(tm_ctx *c, uint64_t *keys, int32_t *vals, int64_t n, int lo_bit) {
+  const int64_t tile = RS_THREADS * ITEMS;
+  const int nblocks = (int)((n + tile - 1) / tile);
+  TM_TRY(tm_ensure(c, &c->d_hist, c->cap_hist, (int64_t)256 * nblocks + 256, "radix histogram"));
+  uint64_t *k0 = keys, *k1 = c->d_key_alt;
+  int32_t *v0 = vals, *v1 = c->d_val_alt;
+  for (int shift = lo_bit; shift < 64; shift += 8) {
+    k_rs_hist<ITEMS, FEW><<<nblocks, RS_THREADS, 0, c->stream>>>(k0, n, shift, c->d_hist, nblocks);
+    if (!FEW) k_rs_rowscan<<<256, RS_THREADS, 0, c->stream>>>(c->d_hist, nblocks);
+    k_rs_scatter<ITEMS, FEW><<<nblocks, RS_THREADS, 0, c->stream>>>(k0, v0, k1, v1, n, shift, c->d_hist, nblocks);
+    TM_HIP(c, hipGetLastError());
+    std::swap(k0, k1);
+    std::swap(v0, v1);
+  }
+  return TM_OK;
+}
+
+// Keys a tile, by the number of keys.  A tile's items are ranked one after the
+// other, so that few keys, whose passes are latency, take small tiles on more
+// CUs; many keys take large ones, whose runs of a digit are written in longer
+// pieces, and fewer of them to scan.  Times of a build, 4096 / 2048 / 1024 keys a
+// tile: 300K cells 174 / 138 / 129 us, 800K 222 / 195 / 197, 1.2M 274 / 245 /
+// 258, 2M 364 / 357 / 407, 6M 914 / 953 / 1115.  Adding up the histograms in
+// the scatter against scanning them in a kernel of their own: 4K 65 against 79 us,
+// 30K 76 / 85, 65K 91 / 90, 150K 128 / 106.
+constexpr int64_t FEW_N = 1 << 16, SMALL_N = 3 << 18, MEDIUM_N = 1 << 22;
+
 // Stable sort of (keys, vals) by key bits [lo_bit, 64) (lo_bit a multiple
 // of 16, so the passes are even in number); the result ends in the input
 // arrays (the passes ping-pong through c->d_key_alt / d_val_alt).
 tm_status tm_sort_pairs(tm_ctx *c, uint64_t *keys, int32_t *vals, int64_t n, int lo_bit) {
   if (n <= 1) return TM_OK;
   if (lo_bit < 0 || lo_bit >= 64 || lo_bit % 16) return tm_fail(c, TM_ERR_INVALID, "sort: lo_bit");
-  int nblocks = (int)((n + RS_TILE - 1) / RS_TILE);
-  TM_TRY(tm_ensure(c, &c->d_hist, c->cap_hist, (int64_t)256 * nblocks + 256, "radix histogram"));
-  uint64_t *k0 = keys, *k1 = c->d_key_alt;
-  int32_t *v0 = vals, *v1 = c->d_val_alt;
-  for (int shift = lo_bit; shift < 64; shift += 8) {
-    k_rs_hist<<<nblocks, RS_THREADS, 0, c->stream>>>(k0, n, shift, c->d_hist, nblocks);
-    TM_HIP(c, hipGetLastError());
-    k_rs_rowscan<<<256, RS_THREADS, 0, c->stream>>>(c->d_hist, nblocks);
-    TM_HIP(c, hipGetLastError());
-    k_rs_scatter<<<nblocks, RS_THREADS, 0, c->stream>>>(k0, v0, k1, v1, n, shift, c->d_hist, nblocks);
-    TM_HIP(c, hipGetLastError());
-    uint64_t *tk = k0;
-    k0 = k1;
-    k1 = tk;
-    int32_t *tv = v0;
-    v0 = v1;
-    v1 = tv;
-  }
-  return TM_OK;
+  if (n <= FEW_N) return sort_passes<4, true>(c, keys, vals, n, lo_bit);
+  if (n <= SMALL_N) return sort_passes<4, false>(c, keys, vals, n, lo_bit);
+  if (n <= MEDIUM_N) return sort_passes<8, false>(c, keys, vals, n, lo_bit);
+  return sort_passes<16, false>(c, keys, vals, n, lo_bit);
 }
