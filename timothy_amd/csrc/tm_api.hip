@@ -51,8 +51,7 @@ tm_status alloc_cells(tm_ctx *c, int64_t n) {
   free_ptr(c->d_fy);
   free_ptr(c->d_fz);
   free_ptr(c->d_out);
-  free_ptr(c->d_pos_o);
-  free_ptr(c->d_aux_o);
+  free_ptr(c->d_rec);
   free_ptr(c->d_nbr);
   c->nbr_alloc = 0;
   c->nbr_elems = 0;
@@ -68,8 +67,7 @@ tm_status alloc_cells(tm_ctx *c, int64_t n) {
       {(void **)&c->d_ncount, 4},
       {(void **)&c->d_qstar, 4},    {(void **)&c->d_dens, 8},     {(void **)&c->d_v, 8},
       {(void **)&c->d_mind, 8},     {(void **)&c->d_fx, 8},       {(void **)&c->d_fy, 8},
-      {(void **)&c->d_fz, 8},       {(void **)&c->d_out, 48},     {(void **)&c->d_pos_o, 32},
-      {(void **)&c->d_aux_o, 16},
+      {(void **)&c->d_fz, 8},       {(void **)&c->d_out, 48},     {(void **)&c->d_rec, 64},
   };
   for (auto &a : list) {
     if (hipMalloc(a.p, a.bytes * (size_t)cap) != hipSuccess) {
@@ -342,8 +340,7 @@ void tm_destroy(tm_ctx *c) {
   free_ptr(c->d_flags);
   free_ptr(c->d_split);
   free_ptr(c->d_parent);
-  free_ptr(c->d_pos_o);
-  free_ptr(c->d_aux_o);
+  free_ptr(c->d_rec);
   free_ptr(c->d_chunk_start);
   free_ptr(c->d_chunk_cid);
   free_ptr(c->d_cbox);

@@ -96,24 +96,34 @@ __device__ __forceinline__ int key_delta64(uint64_t ki, uint64_t kj, const uint4
 // bounding box of x -+ (h_type + 0.01) per colony (src/octree.c:161-174): one
 // workgroup per chunk of one colony, reduced in registers and LDS into the
 // chunk's six order-preserving integer images of the doubles (k_affine
-// reduces a colony's chunks; no atomics on six shared words)
+// reduces a colony's chunks; no atomics on six shared words).  Four cells a
+// thread, loaded together: a loop over eight took 8.5 us for 30K cells, one
+// latency after the other, now 5.1; 43 -> 38 us for 6M, which is bandwidth.
 __global__ __launch_bounds__(BT) void k_bbox(const double *__restrict__ x, const double *__restrict__ y,
                                              const double *__restrict__ z, const int32_t *__restrict__ ctype,
                                              const int64_t *__restrict__ chunk_start,
                                              const int32_t *__restrict__ chunk_cid,
                                              const TypeDev *__restrict__ types, int ntypes,
-                                             unsigned long long *__restrict__ cbox, unsigned int *__restrict__ flags) {
+                                             unsigned long long *__restrict__ cbox) {
   __shared__ unsigned long long red[BT / 64][6];
   const int64_t s = chunk_start[blockIdx.x], e = chunk_start[blockIdx.x + 1];
   unsigned long long k[6] = {~0ull, ~0ull, ~0ull, 0ull, 0ull, 0ull};
-  for (int64_t i = s + threadIdx.x; i < e; i += BT) {
-    int t = ctype[i];
-    if (t < 0 || t >= ntypes) {
-      atomicOr(flags, (unsigned)TM_FLAG_CTYPE);
-      t = 0;
-    }
+  constexpr int U = TM_BBOX_CHUNK / BT;  // a chunk's cells per thread, loaded together
+  double xs[U], ys[U], zs[U];
+  int ts[U];
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    const int64_t i = min(s + u * BT + (int64_t)threadIdx.x, e - 1);  // repeats the last cell
+    xs[u] = x[i];
+    ys[u] = y[i];
+    zs[u] = z[i];
+    ts[u] = ctype[i];
+  }
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    const int t = ts[u] < 0 || ts[u] >= ntypes ? 0 : ts[u];  // k_keys flags it
     const double ext = types[t].h + 0.01;  // src/octree.c:167
-    const double px = x[i], py = y[i], pz = z[i];
+    const double px = xs[u], py = ys[u], pz = zs[u];
     const unsigned long long v[6] = {ord_key(px - ext), ord_key(py - ext), ord_key(pz - ext),
                                      ord_key(px + ext), ord_key(py + ext), ord_key(pz + ext)};
 #pragma unroll
@@ -147,14 +157,18 @@ __global__ __launch_bounds__(BT) void k_bbox(const double *__restrict__ x, const
   }
 }
 
-// src/octree.c:175-180: one wave per colony reduces its chunks' boxes
-__global__ __launch_bounds__(64) void k_affine(const unsigned long long *__restrict__ cbox,
+// src/octree.c:175-180: one workgroup per colony reduces its chunks' boxes; the
+// first clears the build's flags
+constexpr int AT = 512;
+__global__ __launch_bounds__(AT) void k_affine(const unsigned long long *__restrict__ cbox,
                                                const int64_t *__restrict__ col_chunk, int ncol,
-                                               double4 *__restrict__ aff) {
+                                               double4 *__restrict__ aff, unsigned int *__restrict__ flags) {
+  __shared__ unsigned long long red[AT / 64][6];
   const int c = blockIdx.x;
   if (c >= ncol) return;
+  if (c == 0 && threadIdx.x < 4) flags[threadIdx.x] = 0;
   unsigned long long k[6] = {~0ull, ~0ull, ~0ull, 0ull, 0ull, 0ull};
-  for (int64_t q = col_chunk[c] + threadIdx.x; q < col_chunk[c + 1]; q += 64) {
+  for (int64_t q = col_chunk[c] + threadIdx.x; q < col_chunk[c + 1]; q += AT) {
 #pragma unroll
     for (int a = 0; a < 3; ++a) {
       const unsigned long long lo = cbox[6 * q + a], hi = cbox[6 * q + 3 + a];
@@ -171,7 +185,15 @@ __global__ __launch_bounds__(64) void k_affine(const unsigned long long *__restr
       k[a + 3] = u > k[a + 3] ? u : k[a + 3];
     }
   }
+  if ((threadIdx.x & 63) == 0)
+    for (int a = 0; a < 6; ++a) red[threadIdx.x >> 6][a] = k[a];
+  __syncthreads();
   if (threadIdx.x != 0) return;
+  for (int q = 1; q < AT / 64; ++q)
+    for (int a = 0; a < 3; ++a) {
+      k[a] = red[q][a] < k[a] ? red[q][a] : k[a];
+      k[a + 3] = red[q][a + 3] > k[a + 3] ? red[q][a + 3] : k[a + 3];
+    }
   double mn[3], mx[3];
   for (int a = 0; a < 3; ++a) {
     mn[a] = unord_key(k[a]);
@@ -183,19 +205,25 @@ __global__ __launch_bounds__(64) void k_affine(const unsigned long long *__restr
   aff[c] = make_double4(mn[0], mn[1], mn[2], s);
 }
 
-// Morton keys, and the cell inputs packed in reference order (one 32-byte and
-// one 16-byte record per cell) so the Morton gather below reads two records
-// per cell instead of seven scattered arrays.
+// Morton keys, and the cell inputs and codes packed in reference order, one
+// aligned 64-byte record per cell: the Morton gather below, whose order is
+// random in it, reads one line per cell.  A 32-byte and a 16-byte record, two
+// lines a cell: 95 us the gather of 2M cells, 296 us of 6M; now 75 and 226.
+// Both kernels are bound by memory.  The records leave through LDS in whole
+// lines and past the caches: written by their own lanes, 64 bytes apart, they
+// took 56 us against 38 us at 2M, 176 against 110 us at 6M; through the caches
+// the gather takes 81 and 239 us.
 __global__ __launch_bounds__(BT) void k_keys(const double *__restrict__ x, const double *__restrict__ y,
                                              const double *__restrict__ z, const double *__restrict__ size,
                                              const float *__restrict__ young, const int32_t *__restrict__ ctype,
                                              const int32_t *__restrict__ phase, int64_t n,
                                              const int64_t *__restrict__ off, int ncol, int cb, int ntypes,
                                              const double4 *__restrict__ aff, uint64_t *__restrict__ key,
-                                             int32_t *__restrict__ val, double4 *__restrict__ pos_o,
-                                             uint4 *__restrict__ aux_o) {
-  int64_t i = (int64_t)blockIdx.x * BT + threadIdx.x;
-  if (i >= n) return;
+                                             int32_t *__restrict__ val, CellRec *__restrict__ rec,
+                                             unsigned int *__restrict__ flags) {
+  typedef uint32_t V4 __attribute__((ext_vector_type(4)));
+  __shared__ V4 stage[BT][5];  // a record's four quarters, the rows on different banks
+  const int64_t i0 = (int64_t)blockIdx.x * BT, i = min(i0 + (int64_t)threadIdx.x, n - 1);
   const int cid = ncol > 1 ? colony_of(off, ncol, i) : 0;
   const double4 a = aff[cid];
   const double px = x[i], py = y[i], pz = z[i];
@@ -204,16 +232,30 @@ __global__ __launch_bounds__(BT) void k_keys(const double *__restrict__ x, const
   if (cb > 0) k = ((uint64_t)cid << (64 - cb)) | (k >> cb);
   key[i] = k;
   val[i] = (int32_t)i;
-  pos_o[i] = make_double4(px, py, pz, size[i]);
   const int32_t t = ctype[i];
-  aux_o[i] = make_uint4(__float_as_uint(young ? young[i] : 0.0f),
-                        (uint32_t)((t < 0 || t >= ntypes) ? 0 : t),  // out-of-range types were flagged by k_bbox
-                        (uint32_t)(phase ? phase[i] : 1), (uint32_t)cid);
+  const bool bad = t < 0 || t >= ntypes;
+  if (bad) atomicOr(flags, (unsigned)TM_FLAG_CTYPE);
+  union {
+    CellRec r;
+    V4 q[4];
+  } u;
+  u.r.pos = make_double4(px, py, pz, size[i]);
+  u.r.aux = make_uint4(__float_as_uint(young ? young[i] : 0.0f), (uint32_t)(bad ? 0 : t),
+                       (uint32_t)(phase ? phase[i] : 1), (uint32_t)cid);
+  u.r.code = make_uint4(cx, cy, cz, (uint32_t)cid);
+#pragma unroll
+  for (int q = 0; q < 4; ++q) stage[threadIdx.x][q] = u.q[q];
+  __syncthreads();
+  V4 *dst = reinterpret_cast<V4 *>(rec + i0);
+#pragma unroll
+  for (int s = 0; s < 4; ++s) {
+    const int e = s * BT + threadIdx.x;
+    if (i0 + (e >> 2) < n) __builtin_nontemporal_store(stage[e >> 2][e & 3], dst + e);
+  }
 }
 
 __global__ __launch_bounds__(BT) void k_gather(const int32_t *__restrict__ perm, int64_t n,
-                                               const double4 *__restrict__ pos_o, const uint4 *__restrict__ aux_o,
-                                               const double4 *__restrict__ aff, uint4 *__restrict__ code,
+                                               const CellRec *__restrict__ rec, const double4 *__restrict__ aff, uint4 *__restrict__ code,
                                                double4 *__restrict__ pos, float4 *__restrict__ posf,
                                                float *__restrict__ young_s, int32_t *__restrict__ ctype_s,
                                                int32_t *__restrict__ phase_s) {
@@ -222,10 +264,10 @@ __global__ __launch_bounds__(BT) void k_gather(const int32_t *__restrict__ perm,
   if (i >= n) return;
   int64_t o = perm[i];
   if (o < 0 || o >= n) o = 0;  // unreachable for a valid permutation; bounds the gathers
-  const double4 P = pos_o[o];
-  const uint4 X = aux_o[o];
+  const double4 P = rec[o].pos;
+  const uint4 X = rec[o].aux;
+  code[i] = rec[o].code;
   const double4 a = aff[X.w];
-  code[i] = make_uint4(loc_code(P.x, a.x, a.w), loc_code(P.y, a.y, a.w), loc_code(P.z, a.z, a.w), X.w);
   pos[i] = P;
   // the walk's screening copy: x, y, z relative to the colony's lower
   // corner, formed in FP64 and rounded to FP32
@@ -541,11 +583,6 @@ __global__ __launch_bounds__(BT) void k_clear_chain(uint32_t *__restrict__ chain
   if (i < n) chain[i] = 0u;
 }
 
-__global__ void k_zero_u32(unsigned int *p, int n) {
-  int i = threadIdx.x;
-  if (i < n) p[i] = 0;
-}
-
 }  // namespace
 
 tm_status tm_run_build(tm_ctx *c) {
@@ -559,22 +596,21 @@ tm_status tm_run_build(tm_ctx *c) {
     return TM_OK;
   }
   hipStream_t st = c->stream;
-  k_zero_u32<<<1, 64, 0, st>>>(c->d_flags, 4);
   // bounding boxes and affine maps
   if (c->nchunks > 0)
     k_bbox<<<(unsigned)c->nchunks, BT, 0, st>>>(c->x, c->y, c->z, c->ctype, c->d_chunk_start, c->d_chunk_cid,
-                                                 c->d_types, c->ntypes, c->d_cbox, c->d_flags);
-  k_affine<<<(unsigned)c->ncol, 64, 0, st>>>(c->d_cbox, c->d_col_chunk, c->ncol, c->d_aff);
+                                                 c->d_types, c->ntypes, c->d_cbox);
+  k_affine<<<(unsigned)c->ncol, AT, 0, st>>>(c->d_cbox, c->d_col_chunk, c->ncol, c->d_aff, c->d_flags);
   TM_HIP(c, hipGetLastError());
   // Morton keys and the sort
   int cb = 0;
   while ((1ll << cb) < c->ncol) ++cb;
   k_keys<<<tm_blocks(n, BT), BT, 0, st>>>(c->x, c->y, c->z, c->size, c->young, c->ctype, c->phase, n, c->d_col_off,
-                                           c->ncol, cb, c->ntypes, c->d_aff, c->d_key, c->d_perm, c->d_pos_o,
-                                           c->d_aux_o);
+                                           c->ncol, cb, c->ntypes, c->d_aff, c->d_key, c->d_perm, c->d_rec,
+                                           c->d_flags);
   TM_HIP(c, hipGetLastError());
   TM_TRY(tm_sort_pairs(c, c->d_key, c->d_perm, n, SORT_LO_BIT));
-  k_gather<<<tm_blocks(n, BT), BT, 0, st>>>(c->d_perm, n, c->d_pos_o, c->d_aux_o, c->d_aff, c->d_code, c->d_pos,
+  k_gather<<<tm_blocks(n, BT), BT, 0, st>>>(c->d_perm, n, c->d_rec, c->d_aff, c->d_code, c->d_pos,
                                              c->d_posf, c->d_young_s, c->d_ctype_s, c->d_phase_s);
   k_fixties<<<tm_blocks(n, BT), BT, 0, st>>>(c->d_key, n, c->d_perm, c->d_code, c->d_pos, c->d_posf,
                                               c->d_young_s, c->d_ctype_s, c->d_phase_s, c->d_flags);

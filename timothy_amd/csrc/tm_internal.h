@@ -16,7 +16,7 @@
 #define TM_FLAG_ROOT 2
 #define TM_FLAG_CTYPE 4
 #define TM_FLAG_WALK 8
-#define TM_BBOX_CHUNK 2048
+#define TM_BBOX_CHUNK 1024
 // LDS tiles: the pair kernels take cells in tiles of tile_width (128, 256 or
 // 512; TM_TILE by default) consecutive (Morton-order) cells; the distinct
 // neighbours of a tile, at most
@@ -39,6 +39,13 @@
 // [TM_HFLAGS_CG, TM_HFLAGS_WORDS) the environment solve's state read back
 #define TM_HFLAGS_WORDS 32
 #define TM_HFLAGS_CG 16
+
+// A cell's inputs and location codes, in reference order.
+struct alignas(64) CellRec {
+  double4 pos;  // x, y, z, size
+  uint4 aux;    // young bits, ctype, phase, colony
+  uint4 code;   // location codes, colony
+};
 
 // Per cell-type constants, derived on the host with the reference's own
 // expressions (src/inline.h:45-46,71-72) so the device reads identical values.
@@ -110,9 +117,8 @@ struct tm_ctx {
   int64_t *d_chunk_start = nullptr;  // nchunks + 1
   int32_t *d_chunk_cid = nullptr;
   unsigned long long *d_cbox = nullptr;  // per chunk 6 ordered keys: its cells' bounding box
-  // inputs packed in reference order by the key kernel
-  double4 *d_pos_o = nullptr;  // x, y, z, size
-  uint4 *d_aux_o = nullptr;    // young bits, ctype, phase, colony
+  // written by the key kernel
+  CellRec *d_rec = nullptr;
 
   // per colony
   double4 *d_aff = nullptr;              // shift.xyz, scale
