@@ -86,12 +86,42 @@ tm_status alloc_colonies(tm_ctx *c, int ncol) {
   free_ptr(c->d_col_chunk);
   free_ptr(c->d_colroot);
   c->cap_col = 0;
+  c->tables_valid = false;
   if (hipMalloc((void **)&c->d_col_off, sizeof(int64_t) * (ncol + 1)) != hipSuccess ||
       hipMalloc((void **)&c->d_aff, sizeof(double4) * ncol) != hipSuccess ||
       hipMalloc((void **)&c->d_col_chunk, sizeof(int64_t) * (ncol + 1)) != hipSuccess ||
       hipMalloc((void **)&c->d_colroot, sizeof(int32_t) * ncol) != hipSuccess)
     return tm_fail(c, TM_ERR_NOMEM, "hipMalloc failed for colony arrays");
   c->cap_col = ncol;
+  return TM_OK;
+}
+
+// Pinned memory of the context for one transfer of `bytes`, or null: many small
+// copies from or to pageable memory cost 10 to 15 us each, so up to STAGE_MAX
+// bytes go as one, through here.  Upload and results of 20K cells: 119 and 117
+// us by 11 and 6 copies, 25 and 71 us by one each; 60K: 171 and 189, 55 and 147.
+// At 200K (16 MB) the copy through here costs what it saves.
+constexpr size_t STAGE_MAX = 4u << 20;
+tm_status pinned_stage(tm_ctx *c, size_t bytes, char **out) {
+  *out = nullptr;
+  if (bytes > STAGE_MAX) return TM_OK;
+  if (c->stage_busy) {
+    TM_HIP(c, hipStreamSynchronize(c->stream));
+    c->stage_busy = false;
+  }
+  if (bytes > c->cap_stage) {
+    if (c->h_stage) (void)hipHostFree(c->h_stage);
+    c->h_stage = nullptr;
+    c->cap_stage = 0;
+    const size_t cap = std::min(STAGE_MAX, std::max<size_t>(64u << 10, bytes + bytes / 2));
+    if (hipHostMalloc((void **)&c->h_stage, cap, hipHostMallocDefault) != hipSuccess) {
+      (void)hipGetLastError();
+      c->h_stage = nullptr;
+      return TM_OK;
+    }
+    c->cap_stage = cap;
+  }
+  *out = c->h_stage;
   return TM_OK;
 }
 
@@ -124,39 +154,46 @@ tm_status set_cells(tm_ctx *c, int64_t n, int32_t ncol, const int64_t *off, cons
   c->n = n;
   c->ncol = ncol;
   c->col_off = o;
-  TM_HIP(c, hipMemcpyAsync(c->d_col_off, o.data(), sizeof(int64_t) * (ncol + 1), hipMemcpyHostToDevice, c->stream));
-  // bounding-box chunks: each covers at most TM_BBOX_CHUNK cells of one colony
-  std::vector<int64_t> cs, cfirst;
-  std::vector<int32_t> cc;
-  for (int k = 0; k < ncol; ++k) {
-    cfirst.push_back((int64_t)cc.size());
-    for (int64_t s = o[k]; s < o[k + 1]; s += TM_BBOX_CHUNK) {
-      cs.push_back(s);
-      cc.push_back(k);
+  // The colonies' offsets and the bounding-box chunks (each covers at most
+  // TM_BBOX_CHUNK cells of one colony) depend on the offsets alone: an upload
+  // with the last one's makes none of their four copies.
+  if (!c->tables_valid || o != c->tables_off) {
+    c->tables_valid = false;
+    std::vector<int64_t> cs, cfirst;
+    std::vector<int32_t> cc;
+    for (int k = 0; k < ncol; ++k) {
+      cfirst.push_back((int64_t)cc.size());
+      for (int64_t s = o[k]; s < o[k + 1]; s += TM_BBOX_CHUNK) {
+        cs.push_back(s);
+        cc.push_back(k);
+      }
     }
-  }
-  cfirst.push_back((int64_t)cc.size());
-  cs.push_back(n);
-  c->nchunks = (int64_t)cc.size();
-  if (c->nchunks + 1 > c->cap_chunks) {
-    free_ptr(c->d_chunk_start);
-    free_ptr(c->d_chunk_cid);
-    free_ptr(c->d_cbox);
-    c->cap_chunks = 0;
-    if (hipMalloc((void **)&c->d_chunk_start, sizeof(int64_t) * (c->nchunks + 1)) != hipSuccess ||
-        hipMalloc((void **)&c->d_chunk_cid, sizeof(int32_t) * (c->nchunks + 1)) != hipSuccess ||
-        hipMalloc((void **)&c->d_cbox, sizeof(unsigned long long) * 6 * (c->nchunks + 1)) != hipSuccess)
-      return tm_fail(c, TM_ERR_NOMEM, "hipMalloc failed for bounding-box chunks");
-    c->cap_chunks = c->nchunks + 1;
-  }
-  TM_HIP(c, hipMemcpyAsync(c->d_col_chunk, cfirst.data(), sizeof(int64_t) * cfirst.size(), hipMemcpyHostToDevice,
-                           c->stream));
-  TM_HIP(c, hipMemcpyAsync(c->d_chunk_start, cs.data(), sizeof(int64_t) * cs.size(), hipMemcpyHostToDevice,
-                           c->stream));
-  if (c->nchunks > 0)
-    TM_HIP(c, hipMemcpyAsync(c->d_chunk_cid, cc.data(), sizeof(int32_t) * cc.size(), hipMemcpyHostToDevice,
+    cfirst.push_back((int64_t)cc.size());
+    cs.push_back(n);
+    c->nchunks = (int64_t)cc.size();
+    if (c->nchunks + 1 > c->cap_chunks) {
+      free_ptr(c->d_chunk_start);
+      free_ptr(c->d_chunk_cid);
+      free_ptr(c->d_cbox);
+      c->cap_chunks = 0;
+      if (hipMalloc((void **)&c->d_chunk_start, sizeof(int64_t) * (c->nchunks + 1)) != hipSuccess ||
+          hipMalloc((void **)&c->d_chunk_cid, sizeof(int32_t) * (c->nchunks + 1)) != hipSuccess ||
+          hipMalloc((void **)&c->d_cbox, sizeof(unsigned long long) * 6 * (c->nchunks + 1)) != hipSuccess)
+        return tm_fail(c, TM_ERR_NOMEM, "hipMalloc failed for bounding-box chunks");
+      c->cap_chunks = c->nchunks + 1;
+    }
+    TM_HIP(c, hipMemcpyAsync(c->d_col_off, o.data(), sizeof(int64_t) * (ncol + 1), hipMemcpyHostToDevice, c->stream));
+    TM_HIP(c, hipMemcpyAsync(c->d_col_chunk, cfirst.data(), sizeof(int64_t) * cfirst.size(), hipMemcpyHostToDevice,
                              c->stream));
-  TM_HIP(c, hipStreamSynchronize(c->stream));
+    TM_HIP(c, hipMemcpyAsync(c->d_chunk_start, cs.data(), sizeof(int64_t) * cs.size(), hipMemcpyHostToDevice,
+                             c->stream));
+    if (c->nchunks > 0)
+      TM_HIP(c, hipMemcpyAsync(c->d_chunk_cid, cc.data(), sizeof(int32_t) * cc.size(), hipMemcpyHostToDevice,
+                               c->stream));
+    TM_HIP(c, hipStreamSynchronize(c->stream));
+    c->tables_off = o;
+    c->tables_valid = true;
+  }
   if (device) {
     c->external = true;
     c->x = x;
@@ -168,44 +205,52 @@ tm_status set_cells(tm_ctx *c, int64_t n, int32_t ncol, const int64_t *off, cons
     c->phase = phase;
   } else {
     c->external = false;
-    // owned copies sized to the per-cell capacity
-    auto realloc_own = [&](void **p, size_t elt) -> tm_status {
-      if (*p) (void)hipFree(*p);
-      *p = nullptr;
-      if (hipMalloc(p, elt * (size_t)c->cap_n) != hipSuccess) {
-        *p = nullptr;
+    // owned copies in one block sized to the per-cell capacity, an array after
+    // the other, each padded to 64 elements
+    const size_t np = ((size_t)n + 63) & ~(size_t)63, cap = ((size_t)c->cap_n + 63) & ~(size_t)63;
+    if (!c->own || c->own_cap < (int64_t)cap) {
+      free_ptr(c->own);
+      c->own_cap = 0;
+      if (hipMalloc((void **)&c->own, 44 * cap) != hipSuccess) {
+        c->own = nullptr;
         return tm_fail(c, TM_ERR_NOMEM, "hipMalloc failed for cell inputs");
       }
-      return TM_OK;
-    };
-    if (!c->own_x || c->own_cap < c->cap_n) {
-      TM_TRY(realloc_own((void **)&c->own_x, 8));
-      TM_TRY(realloc_own((void **)&c->own_y, 8));
-      TM_TRY(realloc_own((void **)&c->own_z, 8));
-      TM_TRY(realloc_own((void **)&c->own_size, 8));
-      TM_TRY(realloc_own((void **)&c->own_young, 4));
-      TM_TRY(realloc_own((void **)&c->own_ctype, 4));
-      TM_TRY(realloc_own((void **)&c->own_phase, 4));
-      c->own_cap = c->cap_n;
+      c->own_cap = (int64_t)cap;
     }
+    const struct {
+      const void *src;
+      size_t elt, at;
+    } in[] = {{x, 8, 0},           {y, 8, 8 * np},      {z, 8, 16 * np},    {size, 8, 24 * np},
+              {young, 4, 32 * np}, {ctype, 4, 36 * np}, {phase, 4, 40 * np}};
+    const size_t bytes = 40 * np + (phase ? 4 * (size_t)n : 0);
     if (n > 0) {
-      TM_HIP(c, hipMemcpyAsync(c->own_x, x, 8 * n, hipMemcpyHostToDevice, c->stream));
-      TM_HIP(c, hipMemcpyAsync(c->own_y, y, 8 * n, hipMemcpyHostToDevice, c->stream));
-      TM_HIP(c, hipMemcpyAsync(c->own_z, z, 8 * n, hipMemcpyHostToDevice, c->stream));
-      TM_HIP(c, hipMemcpyAsync(c->own_size, size, 8 * n, hipMemcpyHostToDevice, c->stream));
-      TM_HIP(c, hipMemcpyAsync(c->own_ctype, ctype, 4 * n, hipMemcpyHostToDevice, c->stream));
-      if (young) TM_HIP(c, hipMemcpyAsync(c->own_young, young, 4 * n, hipMemcpyHostToDevice, c->stream));
-      else TM_HIP(c, hipMemsetAsync(c->own_young, 0, 4 * n, c->stream));
-      if (phase) TM_HIP(c, hipMemcpyAsync(c->own_phase, phase, 4 * n, hipMemcpyHostToDevice, c->stream));
+      char *stage = nullptr;
+      TM_TRY(pinned_stage(c, bytes, &stage));
+      if (stage) {  // (returns while the copy is under way: the host arrays have been read)
+        for (auto &a : in) {
+          if (a.src) std::memcpy(stage + a.at, a.src, a.elt * (size_t)n);
+          else if (a.at < bytes) std::memset(stage + a.at, 0, a.elt * (size_t)n);
+        }
+        TM_HIP(c, hipMemcpyAsync(c->own, stage, bytes, hipMemcpyHostToDevice, c->stream));
+        c->stage_busy = true;
+      } else {
+        for (auto &a : in) {
+          if (a.src) TM_HIP(c, hipMemcpyAsync(c->own + a.at, a.src, a.elt * n, hipMemcpyHostToDevice, c->stream));
+          else if (a.at < bytes) TM_HIP(c, hipMemsetAsync(c->own + a.at, 0, a.elt * n, c->stream));
+        }
+        TM_HIP(c, hipStreamSynchronize(c->stream));  // host arrays may be freed after return
+      }
     }
+    c->own_x = (double *)c->own;
+    c->own_y = c->own_x + np;
+    c->own_z = c->own_y + np;
     c->x = c->own_x;
     c->y = c->own_y;
     c->z = c->own_z;
-    c->size = c->own_size;
-    c->young = c->own_young;
-    c->ctype = c->own_ctype;
-    c->phase = phase ? c->own_phase : nullptr;
-    TM_HIP(c, hipStreamSynchronize(c->stream));  // host arrays may be freed after return
+    c->size = c->own_z + np;
+    c->young = (const float *)(c->own + 32 * np);
+    c->ctype = (const int32_t *)(c->own + 36 * np);
+    c->phase = phase ? (const int32_t *)(c->own + 40 * np) : nullptr;
   }
   c->stage = 1;
   return TM_OK;
@@ -329,13 +374,8 @@ void tm_destroy(tm_ctx *c) {
   free_ptr(c->d_aff);
   free_ptr(c->d_col_chunk);
   free_ptr(c->d_colroot);
-  free_ptr(c->own_x);
-  free_ptr(c->own_y);
-  free_ptr(c->own_z);
-  free_ptr(c->own_size);
-  free_ptr(c->own_young);
-  free_ptr(c->own_ctype);
-  free_ptr(c->own_phase);
+  free_ptr(c->own);
+  if (c->h_stage) (void)hipHostFree(c->h_stage);
   free_ptr(c->d_types);
   free_ptr(c->d_flags);
   free_ptr(c->d_split);
@@ -533,6 +573,15 @@ tm_status tm_get_results(tm_ctx *c, double *density, double *v, double *mindist,
   if (n == 0) return TM_OK;
   TM_TRY(tm_run_unpermute(c));
   double *dst[6] = {density, v, mindist, fx, fy, fz};
+  char *stage = nullptr;
+  TM_TRY(pinned_stage(c, 48 * (size_t)n, &stage));
+  if (stage) {
+    TM_HIP(c, hipMemcpyAsync(stage, c->d_out, 48 * n, hipMemcpyDeviceToHost, c->stream));
+    TM_HIP(c, hipStreamSynchronize(c->stream));
+    for (int j = 0; j < 6; ++j)
+      if (dst[j]) std::memcpy(dst[j], stage + 8 * n * j, 8 * n);
+    return TM_OK;
+  }
   for (int j = 0; j < 6; ++j)
     if (dst[j]) TM_HIP(c, hipMemcpyAsync(dst[j], c->d_out + j * n, 8 * n, hipMemcpyDeviceToHost, c->stream));
   TM_HIP(c, hipStreamSynchronize(c->stream));

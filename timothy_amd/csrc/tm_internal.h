@@ -106,10 +106,14 @@ struct tm_ctx {
   const double *x = nullptr, *y = nullptr, *z = nullptr, *size = nullptr;
   const float *young = nullptr;
   const int32_t *ctype = nullptr, *phase = nullptr;
-  double *own_x = nullptr, *own_y = nullptr, *own_z = nullptr, *own_size = nullptr;
-  float *own_young = nullptr;
-  int32_t *own_ctype = nullptr, *own_phase = nullptr;
+  char *own = nullptr;  // the uploaded cells' arrays (44 bytes a cell), x, y and z first
+  double *own_x = nullptr, *own_y = nullptr, *own_z = nullptr;
   int64_t own_cap = 0;
+  std::vector<int64_t> tables_off;  // the colony offsets that the tables below were made for
+  bool tables_valid = false;
+  char *h_stage = nullptr;  // pinned
+  size_t cap_stage = 0;
+  bool stage_busy = false;  // an upload may still read it
   int64_t *d_col_off = nullptr;
   int64_t cap_col = 0;
   // bounding-box work split: chunks of at most TM_BBOX_CHUNK cells of one colony
