@@ -78,7 +78,7 @@ __device__ __forceinline__ bool cic_inrange(const GridDev &g, const int64_t ci[3
 #define TM_DEP_DT 16
 #endif
 #ifndef TM_DEP_THREADS
-#define TM_DEP_THREADS 256
+#define TM_DEP_THREADS 512
 #endif
 #ifndef TM_DEP_HEAVY
 #define TM_DEP_HEAVY 1024
@@ -223,10 +223,9 @@ __global__ __launch_bounds__(256) void k_dep_count(const double4 *__restrict__ p
 // set for a G0 cell under weight mode 0 (its weight is 0.75).  The rank-0
 // cell of each key clears the key's count (the scan has read it), so the
 // counts are zero after the deposit.
-__global__ __launch_bounds__(256) void k_dep_place(const uint64_t *__restrict__ kr, int64_t n, uint32_t nkeys,
-                                                   const uint32_t *__restrict__ offs, uint32_t *__restrict__ cnt,
-                                                   uint32_t *__restrict__ idx) {
-  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+__device__ __forceinline__ void dep_place(int64_t i, const uint64_t *__restrict__ kr, int64_t n, uint32_t nkeys,
+                                          const uint32_t *__restrict__ offs, uint32_t *__restrict__ cnt,
+                                          uint32_t *__restrict__ idx) {
   if (i >= n) return;
   const uint64_t e = kr[i];
   const uint32_t k = (uint32_t)e, r = (uint32_t)(e >> 32) & 0x7FFFFFFFu;
@@ -326,9 +325,9 @@ static_assert(1 + 2 * DEP_R <= DEP_SLOT, "slot record");
 // at least DEP_HEAVY own cells take slots from the front, so that the
 // longest workgroups start first; the rest from the back.  ctr[0..1]
 // (front, back) start at zero.
-__global__ __launch_bounds__(256) void k_dep_order(const uint32_t *__restrict__ offs, DepGrid g, uint32_t ntiles,
-                                                   uint32_t *__restrict__ ctr, uint32_t *__restrict__ slots) {
-  const uint32_t t = blockIdx.x * 256 + threadIdx.x;
+__device__ __forceinline__ void dep_order(uint32_t t, const uint32_t *__restrict__ offs, const DepGrid &g,
+                                          uint32_t ntiles, uint32_t *__restrict__ ctr,
+                                          uint32_t *__restrict__ slots) {
   if (t >= ntiles) return;
   const int tz = (int)(t % (uint32_t)g.nt[2]), ty = (int)((t / (uint32_t)g.nt[2]) % (uint32_t)g.nt[1]),
             tx = (int)(t / ((uint32_t)g.nt[2] * (uint32_t)g.nt[1]));
@@ -357,6 +356,18 @@ __global__ __launch_bounds__(256) void k_dep_order(const uint32_t *__restrict__ 
   }
 }
 
+// Both need the offsets alone, so one launch does both, the tiles' records, a
+// few long chains of loads, in its first workgroups: as two kernels they took
+// 6 and 8 us of a deposit's 105 (2M cells, 256^3).
+__global__ __launch_bounds__(256) void k_dep_place(const uint64_t *__restrict__ kr, int64_t n, uint32_t nkeys,
+                                                   const uint32_t *__restrict__ offs, uint32_t *__restrict__ cnt,
+                                                   uint32_t *__restrict__ idx, DepGrid g, uint32_t ntiles,
+                                                   uint32_t *__restrict__ ctr, uint32_t *__restrict__ slots) {
+  const uint32_t norder = (ntiles + 255) / 256;
+  if (blockIdx.x < norder) dep_order(blockIdx.x * 256 + threadIdx.x, offs, g, ntiles, ctr, slots);
+  else dep_place((int64_t)(blockIdx.x - norder) * 256 + threadIdx.x, kr, n, nkeys, offs, cnt, idx);
+}
+
 // adds the corners of a cell that fall in the tile's owned in-grid nodes:
 // local corner index l (relative to the tile's first node) per axis, node
 // l + o owned when 0 <= l + o <= vhi; weights t = 1 - d and d as the
@@ -380,7 +391,7 @@ __device__ __forceinline__ void dep_cell(const double4 &R, const int l[3], const
   }
 }
 
-constexpr int DEP_U = 4;  // cells per thread and round in k_dep_tile
+constexpr int DEP_U = 2;  // cells per thread and round in k_dep_tile
 
 // One workgroup per tile, in launch-slot order.  The tile's runs are laid
 // end to end as one index space that every thread strides through, DEP_U
@@ -388,6 +399,10 @@ constexpr int DEP_U = 4;  // cells per thread and round in k_dep_tile
 // weights are formed here from its position, as the key was (its corner
 // index relative to this tile's first node is -1 for a cell of a lower
 // neighbour's last plane).
+// Bound by the crowded tiles, then by the stores: 512 threads and two cells a
+// thread and round against 256 and four, a deposit's time: 2M Gaussian cells on
+// 256^3 97 against 105 us, 2M of a ball on 128^3 104 / 108, 30K on 64^3 23 / 26;
+// 1,024 threads 103, 100, 22.
 __global__ __launch_bounds__(DEP_T) void k_dep_tile(const double4 *__restrict__ pos, int weight_mode,
                                                   const uint32_t *__restrict__ idx,
                                                   const uint32_t *__restrict__ slots, DepGrid g, int64_t ls1,
@@ -670,9 +685,8 @@ tm_status tm_run_deposit(tm_ctx *c, const tm_grid *grid, int weight_mode, double
   } else {
     TM_TRY(tm_scan_u32(c, cnt, offs, nkeys + 1));
   }
-  if (n > 0)
-    k_dep_place<<<tm_blocks(n, 256), 256, 0, c->stream>>>(c->d_dkr, n, (uint32_t)nkeys, offs, cnt, c->d_didx);
-  k_dep_order<<<tm_blocks(ntiles, 256), 256, 0, c->stream>>>(offs, g, (uint32_t)ntiles, ctr, slots);
+  k_dep_place<<<tm_blocks(ntiles, 256) + tm_blocks(n, 256), 256, 0, c->stream>>>(
+      c->d_dkr, n, (uint32_t)nkeys, offs, cnt, c->d_didx, g, (uint32_t)ntiles, ctr, slots);
   // with no cells every offset is 0 and no cell is read
   k_dep_tile<<<(unsigned)ntiles, DEP_T, 0, c->stream>>>(c->d_pos, weight_mode, c->d_didx, slots, g,
                                                         grid->localsize[1], grid->localsize[2], prod);
