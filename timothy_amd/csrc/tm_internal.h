@@ -178,7 +178,7 @@ struct tm_ctx {
   int tile_cap4 = 1;  // cap the staged records at TM_TILE_LDS4 when few tiles are larger
   int tile_window = 1;  // k_tiles orders the neighbours near a tile's middle by bitmap (0: all by hash set)
   int64_t tiles_over = 0;  // over-full tiles at the last checked tile build
-  uint32_t *d_tile_idx = nullptr;   // per tile: distinct neighbours, ascending (TM_TILE_MAX slots)
+  uint32_t *d_tile_idx = nullptr;   // per tile: distinct neighbours (TM_TILE_MAX slots)
   uint32_t *d_tile_cnt = nullptr;   // per tile: their number, or TM_TILE_OVER
   uint16_t *d_tile_cell = nullptr;  // per tile: cell offset of each rank (longest list first)
   uint16_t *d_nbr16 = nullptr;      // slot k of rank r of tile g at tm_nbr16_at(g*TS + r, k, nbr_alloc)
@@ -289,6 +289,7 @@ tm_status tm_ensure_tree(tm_ctx *c);
 // tiles: also the LDS tiles (otherwise tm_run_sph makes them where it needs them)
 tm_status tm_run_neighbors(tm_ctx *c, bool check, bool tiles);
 tm_status tm_run_tiles(tm_ctx *c, bool check);
+void tm_size_tiles(tm_ctx *c);  // the staging LDS, from the tile counters in h_flags
 tm_status tm_run_sph(tm_ctx *c, tm_precision prec);
 tm_status tm_run_unpermute(tm_ctx *c);
 tm_status tm_run_deposit(tm_ctx *c, const tm_grid *g, int weight_mode, double *prod);

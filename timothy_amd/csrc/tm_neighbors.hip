@@ -996,6 +996,7 @@ tm_status tm_run_neighbors(tm_ctx *c, bool check, bool tiles) {
     c->stage = 3;
     return TM_OK;
   }
+  c->tiles_ts = 0;
   for (int attempt = 0; attempt < 2; ++attempt) {
     const int64_t need = tm_slot_elems(n, c->nbr_cap);
     if (c->nbr_elems < need || !c->d_nbr) {
@@ -1024,8 +1025,11 @@ tm_status tm_run_neighbors(tm_ctx *c, bool check, bool tiles) {
     else if (c->walk_window == 512 && 2 * n - 1 >= 512) launch_walk<256, 512>(c);
     else launch_walk<256, 0>(c);
     TM_HIP(c, hipGetLastError());
+    // the tiles are made before the host knows that no list overflowed (then
+    // both are repeated): one wait for both
+    if (tiles) TM_TRY(tm_run_tiles(c, false));
     if (!check) break;
-    TM_HIP(c, hipMemcpyAsync(c->h_flags, c->d_flags, 4 * sizeof(unsigned int), hipMemcpyDeviceToHost, c->stream));
+    TM_HIP(c, hipMemcpyAsync(c->h_flags, c->d_flags, 16 * sizeof(unsigned int), hipMemcpyDeviceToHost, c->stream));
     TM_HIP(c, hipStreamSynchronize(c->stream));
     if (c->h_flags[0] & TM_FLAG_DEGENERATE)
       return tm_fail(c, TM_ERR_DEGENERATE,
@@ -1038,10 +1042,9 @@ tm_status tm_run_neighbors(tm_ctx *c, bool check, bool tiles) {
     if (mx <= c->nbr_alloc) break;
     c->nbr_cap = (mx + 7) & ~7ll;  // grow to the largest count seen, rounded up
   }
-  c->tiles_ts = 0;
+  if (tiles && check) tm_size_tiles(c);
   c->lists_tiles = tm_tiles_serve(c);
   c->direct_sums = 0;
-  if (tiles) TM_TRY(tm_run_tiles(c, check));
   c->stage = 3;
   return TM_OK;
 }

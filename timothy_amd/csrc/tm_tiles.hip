@@ -7,8 +7,9 @@
 // stages the distinct ones in LDS once and reads every pair from there
 // instead of gathering 32-byte records through the vector memory path per
 // pair.  Per tile this kernel produces:
-//   tile_idx   the distinct neighbour indices, ascending (so the staging
-//              loads run along the Morton order), at most TM_TILE_MAX
+//   tile_idx   the distinct neighbour indices, at most TM_TILE_MAX: those
+//              near the tile ascending (so the staging loads run along the
+//              Morton order), then the others
 //   tile_cnt   their number, or TM_TILE_OVER when there are more
 //   tile_cell  a ranking of the tile's cells by list length, longest first,
 //              so each wave of the pair kernel takes cells of similar length
@@ -43,72 +44,12 @@ struct TileCfg {
   static constexpr uint32_t RESERVE = TM_TILE_MAX + TS;
   static_assert(HASH == 1 << HBITS && HASH > (int)RESERVE, "hash slots");
 };
-constexpr int SORTN = 2048;  // power of two >= TM_TILE_MAX
 constexpr int WB = 16384;    // cells around a tile's middle whose order a bitmap gives
 constexpr uint32_t EMPTY = 0xFFFFFFFFu;
 
 template <int HBITS>
 __device__ __forceinline__ uint32_t hslot(uint32_t q) {
   return (q * 2654435761u) >> (32 - HBITS);
-}
-
-// Ascending bitonic sort of list[0, m) (m <= TS E) by the TS threads of
-// the workgroup, each holding E consecutive elements (padding EMPTY sorts
-// last).  A compare-exchange partner at distance j lies in the same thread
-// (j < E), in another lane of the same wave (j < 64 E: a shuffle), or in
-// another wave (through LDS, the only stages that need the workgroup's
-// barrier).  Element i keeps the smaller of itself and i ^ j when its place
-// in the pair (i & j) matches the direction of its run (i & size).
-__device__ __forceinline__ uint32_t bitonic_pick(uint32_t x, uint32_t y, uint32_t i, uint32_t j, uint32_t size) {
-  const bool lower = (i & j) == 0, asc = (i & size) == 0;
-  return lower == asc ? min(x, y) : max(x, y);
-}
-
-template <int TS, int E>
-__device__ void tile_sort(uint32_t *list, uint32_t m, uint32_t t) {
-  constexpr uint32_t N = (uint32_t)TS * E;
-  static_assert(N <= SORTN, "sort buffer");
-  uint32_t a[E];
-#pragma unroll
-  for (int e = 0; e < E; ++e) {
-    const uint32_t i = t * E + e;
-    a[e] = i < m ? list[i] : 0xFFFFFFFFu;
-  }
-  for (uint32_t size = 2; size <= N; size <<= 1) {
-    for (uint32_t j = size >> 1; j > 0; j >>= 1) {
-      if (j >= 64u * E) {
-        __syncthreads();  // the previous stage's readers are done
-#pragma unroll
-        for (int e = 0; e < E; ++e) list[t * E + e] = a[e];
-        __syncthreads();
-#pragma unroll
-        for (int e = 0; e < E; ++e) {
-          const uint32_t i = t * E + e;
-          a[e] = bitonic_pick(a[e], list[i ^ j], i, j, size);
-        }
-      } else if (j >= (uint32_t)E) {
-#pragma unroll
-        for (int e = 0; e < E; ++e) {
-          const uint32_t i = t * E + e;
-          const uint32_t y = (uint32_t)__shfl_xor((int)a[e], (int)(j / E), 64);
-          a[e] = bitonic_pick(a[e], y, i, j, size);
-        }
-      } else {
-        uint32_t b[E];
-#pragma unroll
-        for (int e = 0; e < E; ++e) b[e] = a[e ^ j];
-#pragma unroll
-        for (int e = 0; e < E; ++e) a[e] = bitonic_pick(a[e], b[e], t * E + e, j, size);
-      }
-    }
-  }
-  __syncthreads();
-#pragma unroll
-  for (int e = 0; e < E; ++e) {
-    const uint32_t i = t * E + e;
-    if (i < m) list[i] = a[e];
-  }
-  __syncthreads();
 }
 
 // exclusive prefix sum over the threads of the workgroup (wsum: one word
@@ -129,7 +70,14 @@ __device__ __forceinline__ uint32_t block_scan(uint32_t v, uint32_t *wsum) {
   return base + inc - v;
 }
 
-// win: WB, or 0 to send every key through the hash set (same outputs)
+// Bound by LDS traffic, two accesses a list slot at least.  A word of the bitmap
+// and the marks before it lie together (one 8-byte read), and the set's keys
+// keep their slots' order: read apart, and with the keys sorted for the staging
+// loads' sake, 156 us at 2M Gaussian cells, 60 at 300K and 75 for a 1M ball; now
+// 135, 51 and 65, the sums over them unchanged.  Marking the bitmap only where a
+// read finds the bit clear gains nothing.
+//
+// win: WB, or 0 to send every key through the hash set (same sums)
 template <int TS>
 __global__ __launch_bounds__(TS) void k_tiles(int64_t n, int64_t cap, uint32_t win, const uint32_t *__restrict__ nbr,
                                               const uint32_t *__restrict__ count, uint32_t *__restrict__ tile_idx,
@@ -140,28 +88,21 @@ __global__ __launch_bounds__(TS) void k_tiles(int64_t n, int64_t cap, uint32_t w
   constexpr int WPT = WB / 32 / TS;  // bitmap words per thread
   static_assert(WPT * TS * 32 == WB, "bitmap words");
   __shared__ uint32_t keys[HASH];
-  __shared__ uint32_t list[SORTN];
-  // list's words are shared by two arrays whose lives do not meet its own:
-  // the ranking's bins (dead before the barrier that ends the neighbour
-  // pass, after which list is first written) and the hash set's positions
-  // (written after every lane has read the sorted set into registers).  The
-  // smaller footprint lets seven workgroups share a CU instead of five.
-  static_assert(TS <= SORTN && HASH * sizeof(uint16_t) <= sizeof(list), "arrays inside list");
-  uint32_t *const bins = list;
-  uint16_t *const vals = reinterpret_cast<uint16_t *>(list);
+  __shared__ uint16_t vals[HASH];  // their positions
+  __shared__ uint32_t bins[TS];
   __shared__ uint32_t rcnt[TS];
   __shared__ uint16_t order[TS];
   __shared__ uint32_t wsum[TS / 64];
-  __shared__ uint32_t bm[WB / 32], pre[WB / 32];
-  __shared__ uint32_t distinct, nwin, nbelow, hfull;
+  __shared__ uint2 bm[WB / 32];  // a word of the bitmap, the marks before it
+  __shared__ uint32_t distinct, nwin, hfull;
   const int64_t g = blockIdx.x;
   const uint32_t t = threadIdx.x;
   const int64_t cell = g * TS + t;
   const uint32_t cnt = cell < n ? min(count[cell], (uint32_t)cap) : 0u;
   for (int i = t; i < HASH; i += TS) keys[i] = EMPTY;
-  for (int i = t; i < WB / 32; i += TS) bm[i] = 0;
+  for (int i = t; i < WB / 32; i += TS) bm[i] = make_uint2(0u, 0u);
   bins[t] = 0;
-  if (t == 0) distinct = nbelow = hfull = 0;
+  if (t == 0) distinct = hfull = 0;
   __syncthreads();
 
   // rank the cells by list length, longest first (counting sort; the order
@@ -192,10 +133,9 @@ __global__ __launch_bounds__(TS) void k_tiles(int64_t n, int64_t cap, uint32_t w
   // Distinct neighbours of the tile.  Most lie within WB / 2 cells of its
   // middle (84% in the 2M-cell Gaussian colony): those are marked in a
   // bitmap, whose popcount prefix later gives their ascending order and
-  // their positions; the others go into the hash set and are sorted.  The
-  // set's order is: the sorted ones below the window, the window's, the
-  // sorted ones above it.  (Stop counting past TM_TILE_MAX; a lane reads 8
-  // list slots per round so their loads overlap.)
+  // their positions; the others go into the hash set and take the places
+  // after them.  (Stop counting past TM_TILE_MAX; a lane reads 8 list slots
+  // per round so their loads overlap.)
   const int64_t wlo = g * TS + TS / 2 - (int64_t)(win / 2);  // may be negative
   auto insert8 = [&](const uint32_t (&qs)[8]) {
 #pragma unroll
@@ -204,7 +144,7 @@ __global__ __launch_bounds__(TS) void k_tiles(int64_t n, int64_t cap, uint32_t w
       if (q == EMPTY) continue;
       const int64_t r = (int64_t)q - wlo;
       if (r >= 0 && r < (int64_t)win) {
-        atomicOr(&bm[r >> 5], 1u << (r & 31));
+        atomicOr(&bm[r >> 5].x, 1u << (r & 31));
         continue;
       }
       // look it up first (most occurrences are repeats); slots are never
@@ -248,7 +188,7 @@ __global__ __launch_bounds__(TS) void k_tiles(int64_t n, int64_t cap, uint32_t w
   uint32_t bw[WPT], cw = 0;
 #pragma unroll
   for (int e = 0; e < WPT; ++e) {
-    bw[e] = bm[WPT * t + e];
+    bw[e] = bm[WPT * t + e].x;
     cw += __popc(bw[e]);
   }
   const uint32_t pw = block_scan(cw, wsum);
@@ -256,7 +196,7 @@ __global__ __launch_bounds__(TS) void k_tiles(int64_t n, int64_t cap, uint32_t w
     uint32_t run = pw;
 #pragma unroll
     for (int e = 0; e < WPT; ++e) {
-      pre[WPT * t + e] = run;
+      bm[WPT * t + e].y = run;
       run += __popc(bw[e]);
     }
   }
@@ -271,54 +211,21 @@ __global__ __launch_bounds__(TS) void k_tiles(int64_t n, int64_t cap, uint32_t w
     }
     return;
   }
-  // compact the hash set in slot order, then sort it ascending
-  uint32_t mine = 0, low = 0;
+  // positions: the window's first, in order, then the set's, by slot ...
+  uint32_t mine = 0;
+#pragma unroll
+  for (int i = 0; i < HASH / TS; ++i) mine += keys[t + TS * i] != EMPTY;
+  uint32_t w = mw + block_scan(mine, wsum);
+#pragma unroll
   for (int i = 0; i < HASH / TS; ++i) {
-    const uint32_t k = keys[t * (HASH / TS) + i];
+    const uint32_t k = keys[t + TS * i];
     if (k == EMPTY) continue;
-    ++mine;
-    low += (int64_t)k < wlo;
+    vals[t + TS * i] = (uint16_t)w;
+    tile_idx[g * TM_TILE_MAX + w++] = k;
   }
-  if (low) atomicAdd(&nbelow, low);
-  uint32_t w = block_scan(mine, wsum);
-  for (int i = 0; i < HASH / TS; ++i) {
-    const uint32_t k = keys[t * (HASH / TS) + i];
-    if (k != EMPTY) list[w++] = k;
-  }
-  __syncthreads();
-  const uint32_t mb = nbelow;
-  // mo <= TM_TILE_MAX <= SORTN: the largest sort below has TS E = SORTN
-  static_assert(SORTN >= TM_TILE_MAX && SORTN % TS == 0, "tile_sort sizes");
-  if (mo == 0) {
-    // all in the window: nothing to sort
-  } else if (mo <= TS) tile_sort<TS, 1>(list, mo, t);
-  else if (mo <= 2 * TS) tile_sort<TS, 2>(list, mo, t);
-  else if (TS * 4 <= SORTN && mo <= 4 * TS) tile_sort<TS, (TS * 4 <= SORTN ? 4 : 1)>(list, mo, t);
-  else if (TS * 8 <= SORTN && mo <= 8 * TS) tile_sort<TS, (TS * 8 <= SORTN ? 8 : 1)>(list, mo, t);
-  else tile_sort<TS, SORTN / TS>(list, mo, t);
-  // positions: the sorted ones (read out of list before vals overwrites it) ...
-  constexpr int EV = SORTN / TS;
-  uint32_t qv[EV];
-#pragma unroll
-  for (int e = 0; e < EV; ++e) {
-    const uint32_t i = t + (uint32_t)TS * e;
-    qv[e] = i < mo ? list[i] : EMPTY;
-  }
-  __syncthreads();
-#pragma unroll
-  for (int e = 0; e < EV; ++e) {
-    const uint32_t i = t + (uint32_t)TS * e;
-    if (i >= mo) break;
-    const uint32_t q = qv[e];
-    const uint32_t pos = i < mb ? i : i + mw;
-    uint32_t h = hslot<HBITS>(q);
-    while (keys[h] != q) h = (h + 1) & (HASH - 1);
-    vals[h] = (uint16_t)pos;
-    tile_idx[g * TM_TILE_MAX + pos] = q;
-  }
-  // ... and the window's, in order
+  // ... and the window's
   {
-    uint32_t pos = mb + pw;
+    uint32_t pos = pw;
     for (int e = 0; e < WPT; ++e) {
       uint32_t bits = bw[e];
       const int64_t q0 = wlo + 32 * (WPT * (int64_t)t + e);
@@ -354,7 +261,8 @@ __global__ __launch_bounds__(TS) void k_tiles(int64_t n, int64_t cap, uint32_t w
         const int64_t rr = (int64_t)q - wlo;
         if (rr >= 0 && rr < (int64_t)win) {
           const uint32_t wd = (uint32_t)(rr >> 5), bt = (uint32_t)(rr & 31);
-          v[j] = mb + pre[wd] + __popc(bm[wd] & ((1u << bt) - 1u));
+          const uint2 b = bm[wd];
+          v[j] = b.y + __popc(b.x & ((1u << bt) - 1u));
         } else {
           uint32_t h = hslot<HBITS>(q);
           while (keys[h] != q) h = (h + 1) & (HASH - 1);
@@ -391,6 +299,22 @@ void launch_tiles(tm_ctx *c, int64_t nt) {
 
 }  // namespace
 
+void tm_size_tiles(tm_ctx *c) {
+  const int TS = c->tiles_ts;
+  if (!TS) return;
+  const int64_t nt = (c->n + TS - 1) / TS;
+  c->tiles_over = c->h_flags[14];
+  // records staged per tile: the largest tile plus the far stand-in, rounded
+  // (at least TS: the pair kernel also parks a tile's sums there) ...
+  int64_t lds = std::max<int64_t>(TS, std::min<int64_t>(TM_TILE_MAX + 1, ((int64_t)c->h_flags[4] + 1 + 63) & ~63ll));
+  // ... but no more than four workgroups' worth per CU when at most one tile
+  // in twenty is larger: those take the pair kernel's global-record path and
+  // every other tile runs at the higher occupancy
+  if (lds > TM_TILE_LDS4 && c->tile_cap4 && 20 * (int64_t)c->h_flags[5] <= nt) lds = TM_TILE_LDS4;
+  c->tile_lds = (uint32_t)lds;
+  c->tile_lds_ts = TS;
+}
+
 tm_status tm_run_tiles(tm_ctx *c, bool check) {
   const int64_t n = c->n;
   if (!c->sph_tiles || n == 0) {
@@ -413,21 +337,9 @@ tm_status tm_run_tiles(tm_ctx *c, bool check) {
   TM_HIP(c, hipGetLastError());
   c->tiles_ts = TS;
   if (check) {
-    TM_HIP(c, hipMemcpyAsync(c->h_flags + 4, c->d_flags + 4, 2 * sizeof(unsigned int), hipMemcpyDeviceToHost,
-                             c->stream));
-    TM_HIP(c, hipMemcpyAsync(c->h_flags + 14, c->d_flags + 14, sizeof(unsigned int), hipMemcpyDeviceToHost,
-                             c->stream));
+    TM_HIP(c, hipMemcpyAsync(c->h_flags, c->d_flags, 16 * sizeof(unsigned int), hipMemcpyDeviceToHost, c->stream));
     TM_HIP(c, hipStreamSynchronize(c->stream));
-    c->tiles_over = c->h_flags[14];
-    // records staged per tile: the largest tile plus the far stand-in, rounded
-    // (at least TS: the pair kernel also parks a tile's sums there) ...
-    int64_t lds = std::max<int64_t>(TS, std::min<int64_t>(TM_TILE_MAX + 1, ((int64_t)c->h_flags[4] + 1 + 63) & ~63ll));
-    // ... but no more than four workgroups' worth per CU when at most one tile
-    // in twenty is larger: those take the pair kernel's global-record path and
-    // every other tile runs at the higher occupancy
-    if (lds > TM_TILE_LDS4 && c->tile_cap4 && 20 * (int64_t)c->h_flags[5] <= nt) lds = TM_TILE_LDS4;
-    c->tile_lds = (uint32_t)lds;
-    c->tile_lds_ts = TS;
+    tm_size_tiles(c);
   } else if (c->tile_lds == 0 || c->tile_lds_ts != TS) {
     // unsized, or sized for another width (the sums of TS cells must fit):
     // stage the most a tile can hold
