@@ -30,13 +30,16 @@ __device__ __forceinline__ unsigned long long tm_match8(uint32_t d, bool valid) 
   return m;
 }
 
+// zero: a histogram cleared for the pass after this one (or null)
 template <int RS_ITEMS, bool FEW>
 __global__ __launch_bounds__(RS_THREADS) void k_rs_hist(const uint64_t *__restrict__ keys, int64_t n, int shift,
-                                                        uint32_t *__restrict__ hist, int nblocks) {
+                                                        uint32_t *__restrict__ hist, int nblocks,
+                                                        uint32_t *__restrict__ zero) {
   constexpr int RS_TILE = RS_THREADS * RS_ITEMS;
   __shared__ uint32_t h[RS_WAVES][256];
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
   for (int j = tid; j < RS_WAVES * 256; j += RS_THREADS) (&h[0][0])[j] = 0;
+  if (zero) zero[(int64_t)blockIdx.x * 256 + tid] = 0u;
   __syncthreads();
   const int64_t base = (int64_t)blockIdx.x * RS_TILE + (int64_t)w * (64 * RS_ITEMS);
   uint32_t dg[RS_ITEMS];  // all of this lane's digits are loaded before any is counted
@@ -93,12 +96,17 @@ __global__ __launch_bounds__(RS_THREADS) void k_rs_rowscan(uint32_t *__restrict_
 // The tile's keys are ranked stably (by digit, then input order), placed in
 // LDS in that order, and written out from there: consecutive lanes write
 // consecutive slots of one digit's run instead of 64 scattered records.
+// next: the following pass's histogram, to which every key is added where it
+// arrives (FEW; a pass is then one launch: 30K keys 8.5 against 9.5 us, while at
+// 300K the atomics take 20 us and the kernel they replace 7); zero: the one
+// after that, cleared.
 template <int RS_ITEMS, bool FEW>
 __global__ __launch_bounds__(RS_THREADS) void k_rs_scatter(const uint64_t *__restrict__ keys,
                                                            const int32_t *__restrict__ vals,
                                                            uint64_t *__restrict__ okeys, int32_t *__restrict__ ovals,
                                                            int64_t n, int shift, const uint32_t *__restrict__ offs,
-                                                           int nblocks) {
+                                                           int nblocks, uint32_t *__restrict__ next,
+                                                           uint32_t *__restrict__ zero) {
   constexpr int RS_TILE = RS_THREADS * RS_ITEMS;
   __shared__ uint32_t cnt[RS_WAVES][256];
   __shared__ uint32_t pre[RS_WAVES][256];
@@ -109,6 +117,7 @@ __global__ __launch_bounds__(RS_THREADS) void k_rs_scatter(const uint64_t *__res
   __shared__ int32_t sval[RS_TILE];
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
   for (int j = tid; j < RS_WAVES * 256; j += RS_THREADS) (&cnt[0][0])[j] = 0;
+  if (zero) zero[(int64_t)blockIdx.x * 256 + tid] = 0u;
   const int64_t tile0 = (int64_t)blockIdx.x * RS_TILE;
   const int64_t base = tile0 + (int64_t)w * (64 * RS_ITEMS);
   uint64_t k[RS_ITEMS];
@@ -214,6 +223,10 @@ __global__ __launch_bounds__(RS_THREADS) void k_rs_scatter(const uint64_t *__res
     if (pos >= 0 && pos < n) {  // always true for a consistent histogram; keeps a bad scan from writing out of bounds
       okeys[pos] = key;
       ovals[pos] = sval[j];
+      if (next) {
+        const uint32_t t1 = (uint32_t)pos / RS_TILE, d1 = (uint32_t)((key >> (shift + 8)) & 255u);
+        atomicAdd(next + (FEW ? (int64_t)t1 * 256 + d1 : (int64_t)d1 * nblocks + t1), 1u);
+      }
     }
   }
 }
@@ -314,24 +327,6 @@ tm_status tm_scan_u32(tm_ctx *c, const uint32_t *in, uint32_t *out, int64_t n) {
   return TM_OK;
 }
 
-template <int ITEMS, bool FEW>
-static tm_status sort_passes(tm_ctx *c, uint64_t *keys, int32_t *vals, int64_t n, int lo_bit) {
-  const int64_t tile = RS_THREADS * ITEMS;
-  const int nblocks = (int)((n + tile - 1) / tile);
-  TM_TRY(tm_ensure(c, &c->d_hist, c->cap_hist, (int64_t)256 * nblocks + 256, "radix histogram"));
-  uint64_t *k0 = keys, *k1 = c->d_key_alt;
-  int32_t *v0 = vals, *v1 = c->d_val_alt;
-  for (int shift = lo_bit; shift < 64; shift += 8) {
-    k_rs_hist<ITEMS, FEW><<<nblocks, RS_THREADS, 0, c->stream>>>(k0, n, shift, c->d_hist, nblocks);
-    if (!FEW) k_rs_rowscan<<<256, RS_THREADS, 0, c->stream>>>(c->d_hist, nblocks);
-    k_rs_scatter<ITEMS, FEW><<<nblocks, RS_THREADS, 0, c->stream>>>(k0, v0, k1, v1, n, shift, c->d_hist, nblocks);
-    TM_HIP(c, hipGetLastError());
-    std::swap(k0, k1);
-    std::swap(v0, v1);
-  }
-  return TM_OK;
-}
-
 // Keys a tile, by the number of keys.  A tile's items are ranked one after the
 // other, so that few keys, whose passes are latency, take small tiles on more
 // CUs; many keys take large ones, whose runs of a digit are written in longer
@@ -341,6 +336,34 @@ static tm_status sort_passes(tm_ctx *c, uint64_t *keys, int32_t *vals, int64_t n
 // the scatter against scanning them in a kernel of their own: 4K 65 against 79 us,
 // 30K 76 / 85, 65K 91 / 90, 150K 128 / 106.
 constexpr int64_t FEW_N = 1 << 16, SMALL_N = 3 << 18, MEDIUM_N = 1 << 22;
+
+template <int ITEMS, bool FEW>
+static tm_status sort_passes(tm_ctx *c, uint64_t *keys, int32_t *vals, int64_t n, int lo_bit) {
+  const int64_t tile = RS_THREADS * ITEMS;
+  const int nblocks = (int)((n + tile - 1) / tile);
+  const int64_t row = (int64_t)256 * nblocks + 256;
+  TM_TRY(tm_ensure(c, &c->d_hist, c->cap_hist, (FEW ? 3 : 1) * row, "radix histogram"));
+  // this pass's histogram, the next one's and the one to be cleared
+  uint32_t *h0 = c->d_hist, *h1 = FEW ? h0 + row : nullptr, *h2 = FEW ? h1 + row : nullptr;
+  uint64_t *k0 = keys, *k1 = c->d_key_alt;
+  int32_t *v0 = vals, *v1 = c->d_val_alt;
+  for (int shift = lo_bit; shift < 64; shift += 8) {
+    if (!FEW || shift == lo_bit)
+      k_rs_hist<ITEMS, FEW><<<nblocks, RS_THREADS, 0, c->stream>>>(k0, n, shift, h0, nblocks, h1);
+    if (!FEW) k_rs_rowscan<<<256, RS_THREADS, 0, c->stream>>>(h0, nblocks);
+    const bool more = FEW && shift + 8 < 64;
+    k_rs_scatter<ITEMS, FEW><<<nblocks, RS_THREADS, 0, c->stream>>>(k0, v0, k1, v1, n, shift, h0, nblocks,
+                                                                    more ? h1 : nullptr, more ? h2 : nullptr);
+    if (FEW) {
+      std::swap(h0, h1);
+      std::swap(h1, h2);
+    }
+    TM_HIP(c, hipGetLastError());
+    std::swap(k0, k1);
+    std::swap(v0, v1);
+  }
+  return TM_OK;
+}
 
 // Stable sort of (keys, vals) by key bits [lo_bit, 64) (lo_bit a multiple
 // of 16, so the passes are even in number); the result ends in the input
