@@ -158,15 +158,18 @@ __global__ __launch_bounds__(BT) void k_bbox(const double *__restrict__ x, const
 }
 
 // src/octree.c:175-180: one workgroup per colony reduces its chunks' boxes; the
-// first clears the build's flags
+// first clears the build's flags and what the sort wants cleared
 constexpr int AT = 512;
 __global__ __launch_bounds__(AT) void k_affine(const unsigned long long *__restrict__ cbox,
                                                const int64_t *__restrict__ col_chunk, int ncol,
-                                               double4 *__restrict__ aff, unsigned int *__restrict__ flags) {
+                                               double4 *__restrict__ aff, unsigned int *__restrict__ flags,
+                                               uint32_t *__restrict__ clear, int64_t words) {
   __shared__ unsigned long long red[AT / 64][6];
   const int c = blockIdx.x;
   if (c >= ncol) return;
   if (c == 0 && threadIdx.x < 4) flags[threadIdx.x] = 0;
+  if (c == 0)
+    for (int64_t i = threadIdx.x; i < words; i += AT) clear[i] = 0u;
   unsigned long long k[6] = {~0ull, ~0ull, ~0ull, 0ull, 0ull, 0ull};
   for (int64_t q = col_chunk[c] + threadIdx.x; q < col_chunk[c + 1]; q += AT) {
 #pragma unroll
@@ -600,7 +603,10 @@ tm_status tm_run_build(tm_ctx *c) {
   if (c->nchunks > 0)
     k_bbox<<<(unsigned)c->nchunks, BT, 0, st>>>(c->x, c->y, c->z, c->ctype, c->d_chunk_start, c->d_chunk_cid,
                                                  c->d_types, c->ntypes, c->d_cbox);
-  k_affine<<<(unsigned)c->ncol, AT, 0, st>>>(c->d_cbox, c->d_col_chunk, c->ncol, c->d_aff, c->d_flags);
+  uint32_t *clear = nullptr;
+  int64_t words = 0;
+  TM_TRY(tm_sort_prepare(c, n, &clear, &words));
+  k_affine<<<(unsigned)c->ncol, AT, 0, st>>>(c->d_cbox, c->d_col_chunk, c->ncol, c->d_aff, c->d_flags, clear, words);
   TM_HIP(c, hipGetLastError());
   // Morton keys and the sort
   int cb = 0;

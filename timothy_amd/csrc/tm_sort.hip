@@ -2,8 +2,8 @@
 // pairs, 8-bit digits, for the Morton ordering of cells.
 //
 // Each pass: histogram per tile (LDS atomics) -> exclusive scan of the
-// digit-major histogram (up to FEW_N keys each tile of the scatter adds up the
-// tiles' histograms itself) -> stable scatter.  Stable ranks inside a tile
+// digit-major histogram (up to MEDIUM_N keys each tile of the scatter adds up
+// histograms itself) -> stable scatter.  Stable ranks inside a tile
 // come from 64-lane ballots: the lanes holding the same digit are found with
 // eight ballots, the leader of each group advances a per-wave digit counter
 // in LDS.
@@ -12,6 +12,11 @@
 namespace {
 
 constexpr int RS_THREADS = 256;
+constexpr int RS_GROUP = 32;  // tiles a group
+// how the scatter finds a tile's first slot of a digit: from rows scanned by a
+// kernel in between, from the tiles' histograms, from those of its group of
+// tiles and the sums of the groups
+enum Prefix { SCANNED, FEW, GROUPED };
 constexpr int RS_WAVES = RS_THREADS / 64;
 
 constexpr int SC_THREADS = 256;
@@ -31,15 +36,16 @@ __device__ __forceinline__ unsigned long long tm_match8(uint32_t d, bool valid) 
 }
 
 // zero: a histogram cleared for the pass after this one (or null)
-template <int RS_ITEMS, bool FEW>
+template <int RS_ITEMS, Prefix P>
 __global__ __launch_bounds__(RS_THREADS) void k_rs_hist(const uint64_t *__restrict__ keys, int64_t n, int shift,
                                                         uint32_t *__restrict__ hist, int nblocks,
-                                                        uint32_t *__restrict__ zero) {
+                                                        uint32_t *__restrict__ group, uint32_t *__restrict__ zero) {
   constexpr int RS_TILE = RS_THREADS * RS_ITEMS;
   __shared__ uint32_t h[RS_WAVES][256];
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
   for (int j = tid; j < RS_WAVES * 256; j += RS_THREADS) (&h[0][0])[j] = 0;
-  if (zero) zero[(int64_t)blockIdx.x * 256 + tid] = 0u;
+  if (P == FEW) zero[(int64_t)blockIdx.x * 256 + tid] = 0u;
+  if (P == GROUPED && blockIdx.x % RS_GROUP == 0) zero[blockIdx.x / RS_GROUP * 256 + tid] = 0u;
   __syncthreads();
   const int64_t base = (int64_t)blockIdx.x * RS_TILE + (int64_t)w * (64 * RS_ITEMS);
   uint32_t dg[RS_ITEMS];  // all of this lane's digits are loaded before any is counted
@@ -57,7 +63,8 @@ __global__ __launch_bounds__(RS_THREADS) void k_rs_hist(const uint64_t *__restri
   uint32_t s = 0;
 #pragma unroll
   for (int k = 0; k < RS_WAVES; ++k) s += h[k][tid];
-  hist[FEW ? (int64_t)blockIdx.x * 256 + tid : (int64_t)tid * nblocks + blockIdx.x] = s;
+  hist[P != SCANNED ? (int64_t)blockIdx.x * 256 + tid : (int64_t)tid * nblocks + blockIdx.x] = s;
+  if (P == GROUPED && s) atomicAdd(group + blockIdx.x / RS_GROUP * 256 + tid, s);
 }
 
 // Exclusive scan of each digit's row of per-tile counts (one workgroup per
@@ -100,13 +107,13 @@ __global__ __launch_bounds__(RS_THREADS) void k_rs_rowscan(uint32_t *__restrict_
 // arrives (FEW; a pass is then one launch: 30K keys 8.5 against 9.5 us, while at
 // 300K the atomics take 20 us and the kernel they replace 7); zero: the one
 // after that, cleared.
-template <int RS_ITEMS, bool FEW>
+template <int RS_ITEMS, Prefix P>
 __global__ __launch_bounds__(RS_THREADS) void k_rs_scatter(const uint64_t *__restrict__ keys,
                                                            const int32_t *__restrict__ vals,
                                                            uint64_t *__restrict__ okeys, int32_t *__restrict__ ovals,
                                                            int64_t n, int shift, const uint32_t *__restrict__ offs,
-                                                           int nblocks, uint32_t *__restrict__ next,
-                                                           uint32_t *__restrict__ zero) {
+                                                           int nblocks, const uint32_t *__restrict__ group,
+                                                           uint32_t *__restrict__ next, uint32_t *__restrict__ zero) {
   constexpr int RS_TILE = RS_THREADS * RS_ITEMS;
   __shared__ uint32_t cnt[RS_WAVES][256];
   __shared__ uint32_t pre[RS_WAVES][256];
@@ -135,17 +142,26 @@ __global__ __launch_bounds__(RS_THREADS) void k_rs_scatter(const uint64_t *__res
   // digits (the digits' totals, scanned here)
   {
     uint32_t rt = 0, before = 0;
-    if constexpr (FEW) {
-      for (int b = 0; b < nblocks; b += 16) {
+    // adds rows [0, end) to rt, those before `own` also to before
+    auto add = [&](const uint32_t *__restrict__ rows, int end, int own) {
+      for (int b = 0; b < end; b += 16) {
         uint32_t h[16];
 #pragma unroll
-        for (int q = 0; q < 16; ++q) h[q] = b + q < nblocks ? offs[(b + q) * 256 + tid] : 0u;
+        for (int q = 0; q < 16; ++q) h[q] = b + q < end ? rows[(b + q) * 256 + tid] : 0u;
 #pragma unroll
         for (int q = 0; q < 16; ++q) {
           rt += h[q];
-          if (b + q < (int)blockIdx.x) before += h[q];
+          if (b + q < own) before += h[q];
         }
       }
+    };
+    if constexpr (P == FEW) {
+      add(offs, nblocks, (int)blockIdx.x);
+    } else if constexpr (P == GROUPED) {
+      const int g = (int)blockIdx.x / RS_GROUP, in = (int)blockIdx.x % RS_GROUP;
+      add(offs + (int64_t)g * RS_GROUP * 256, in, in);
+      rt = 0;
+      add(group, (nblocks + RS_GROUP - 1) / RS_GROUP, g);
     } else {
       rt = offs[(int64_t)256 * nblocks + tid];
       before = offs[(int64_t)tid * nblocks + blockIdx.x];
@@ -223,9 +239,9 @@ __global__ __launch_bounds__(RS_THREADS) void k_rs_scatter(const uint64_t *__res
     if (pos >= 0 && pos < n) {  // always true for a consistent histogram; keeps a bad scan from writing out of bounds
       okeys[pos] = key;
       ovals[pos] = sval[j];
-      if (next) {
+      if (P == FEW && next) {
         const uint32_t t1 = (uint32_t)pos / RS_TILE, d1 = (uint32_t)((key >> (shift + 8)) & 255u);
-        atomicAdd(next + (FEW ? (int64_t)t1 * 256 + d1 : (int64_t)d1 * nblocks + t1), 1u);
+        atomicAdd(next + (int64_t)t1 * 256 + d1, 1u);
       }
     }
   }
@@ -331,37 +347,52 @@ tm_status tm_scan_u32(tm_ctx *c, const uint32_t *in, uint32_t *out, int64_t n) {
 // other, so that few keys, whose passes are latency, take small tiles on more
 // CUs; many keys take large ones, whose runs of a digit are written in longer
 // pieces, and fewer of them to scan.  Times of a build, 4096 / 2048 / 1024 keys a
-// tile: 300K cells 174 / 138 / 129 us, 800K 222 / 195 / 197, 1.2M 274 / 245 /
-// 258, 2M 364 / 357 / 407, 6M 914 / 953 / 1115.  Adding up the histograms in
-// the scatter against scanning them in a kernel of their own: 4K 65 against 79 us,
-// 30K 76 / 85, 65K 91 / 90, 150K 128 / 106.
+// tile, rows scanned: 300K cells 174 / 138 / 129 us, 800K 222 / 195 / 197, 1.2M
+// 274 / 245 / 258, 2M 364 / 357 / 407, 6M 914 / 953 / 1115.
+// The prefix of a tile: scanned / from all tiles' histograms / from its group's
+// and the groups' sums: 4K cells 79 / 65 / 68 us, 30K 85 / 76 / 77, 65K 90 / 91 /
+// 81 (82 with one launch a pass, which the second allows), 300K 125 / - / 114, 2M
+// 331 / - / 313; 4096 keys a tile: 6M 838 / - / 853, 33M 4.80 / - / 5.69 ms.
 constexpr int64_t FEW_N = 1 << 16, SMALL_N = 3 << 18, MEDIUM_N = 1 << 22;
 
-template <int ITEMS, bool FEW>
+static int64_t group_words(int64_t nblocks) { return (nblocks + RS_GROUP - 1) / RS_GROUP * 256; }
+
+template <int ITEMS, Prefix P>
 static tm_status sort_passes(tm_ctx *c, uint64_t *keys, int32_t *vals, int64_t n, int lo_bit) {
   const int64_t tile = RS_THREADS * ITEMS;
   const int nblocks = (int)((n + tile - 1) / tile);
   const int64_t row = (int64_t)256 * nblocks + 256;
-  TM_TRY(tm_ensure(c, &c->d_hist, c->cap_hist, (FEW ? 3 : 1) * row, "radix histogram"));
-  // this pass's histogram, the next one's and the one to be cleared
-  uint32_t *h0 = c->d_hist, *h1 = FEW ? h0 + row : nullptr, *h2 = FEW ? h1 + row : nullptr;
+  // this pass's histogram, and with FEW the next one's and the one to be
+  // cleared; with GROUPED the groups' sums and the next pass's
+  uint32_t *h0 = c->d_hist, *h1 = P == FEW ? h0 + row : nullptr, *h2 = P == FEW ? h1 + row : nullptr;
+  uint32_t *g0 = P == GROUPED ? h0 + row : nullptr, *g1 = P == GROUPED ? g0 + group_words(nblocks) : nullptr;
   uint64_t *k0 = keys, *k1 = c->d_key_alt;
   int32_t *v0 = vals, *v1 = c->d_val_alt;
   for (int shift = lo_bit; shift < 64; shift += 8) {
-    if (!FEW || shift == lo_bit)
-      k_rs_hist<ITEMS, FEW><<<nblocks, RS_THREADS, 0, c->stream>>>(k0, n, shift, h0, nblocks, h1);
-    if (!FEW) k_rs_rowscan<<<256, RS_THREADS, 0, c->stream>>>(h0, nblocks);
-    const bool more = FEW && shift + 8 < 64;
-    k_rs_scatter<ITEMS, FEW><<<nblocks, RS_THREADS, 0, c->stream>>>(k0, v0, k1, v1, n, shift, h0, nblocks,
-                                                                    more ? h1 : nullptr, more ? h2 : nullptr);
-    if (FEW) {
-      std::swap(h0, h1);
-      std::swap(h1, h2);
-    }
+    if (P != FEW || shift == lo_bit)
+      k_rs_hist<ITEMS, P><<<nblocks, RS_THREADS, 0, c->stream>>>(k0, n, shift, h0, nblocks, g0, P == FEW ? h1 : g1);
+    if (P == SCANNED) k_rs_rowscan<<<256, RS_THREADS, 0, c->stream>>>(h0, nblocks);
+    const bool more = P == FEW && shift + 8 < 64;
+    k_rs_scatter<ITEMS, P><<<nblocks, RS_THREADS, 0, c->stream>>>(k0, v0, k1, v1, n, shift, h0, nblocks, g0,
+                                                                  more ? h1 : nullptr, more ? h2 : nullptr);
+    std::swap(h0, P == FEW ? h1 : h0);
+    std::swap(h1, h2);
+    std::swap(g0, g1);
     TM_HIP(c, hipGetLastError());
     std::swap(k0, k1);
     std::swap(v0, v1);
   }
+  return TM_OK;
+}
+
+// Sizes the sort's workspace for n keys; the *words first words at the address
+// returned must be zero when the sort starts.
+tm_status tm_sort_prepare(tm_ctx *c, int64_t n, uint32_t **clear, int64_t *words) {
+  const int64_t tile = RS_THREADS * (n <= SMALL_N ? 4 : n <= MEDIUM_N ? 8 : 16), nblocks = (n + tile - 1) / tile;
+  const int64_t row = 256 * nblocks + 256, gw = n > FEW_N && n <= MEDIUM_N ? group_words(nblocks) : 0;
+  TM_TRY(tm_ensure(c, &c->d_hist, c->cap_hist, n <= FEW_N ? 3 * row : row + 2 * gw, "radix histogram"));
+  *clear = c->d_hist + row;
+  *words = gw;
   return TM_OK;
 }
 
@@ -371,8 +402,8 @@ static tm_status sort_passes(tm_ctx *c, uint64_t *keys, int32_t *vals, int64_t n
 tm_status tm_sort_pairs(tm_ctx *c, uint64_t *keys, int32_t *vals, int64_t n, int lo_bit) {
   if (n <= 1) return TM_OK;
   if (lo_bit < 0 || lo_bit >= 64 || lo_bit % 16) return tm_fail(c, TM_ERR_INVALID, "sort: lo_bit");
-  if (n <= FEW_N) return sort_passes<4, true>(c, keys, vals, n, lo_bit);
-  if (n <= SMALL_N) return sort_passes<4, false>(c, keys, vals, n, lo_bit);
-  if (n <= MEDIUM_N) return sort_passes<8, false>(c, keys, vals, n, lo_bit);
-  return sort_passes<16, false>(c, keys, vals, n, lo_bit);
+  if (n <= FEW_N) return sort_passes<4, FEW>(c, keys, vals, n, lo_bit);
+  if (n <= SMALL_N) return sort_passes<4, GROUPED>(c, keys, vals, n, lo_bit);
+  if (n <= MEDIUM_N) return sort_passes<8, GROUPED>(c, keys, vals, n, lo_bit);
+  return sort_passes<16, SCANNED>(c, keys, vals, n, lo_bit);
 }
