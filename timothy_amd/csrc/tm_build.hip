@@ -55,6 +55,12 @@ __device__ __forceinline__ uint64_t morton_prefix64(uint32_t cx, uint32_t cy, ui
   return (k63 << 1) | ((cz >> 7) & 1u);
 }
 
+// (colony id : cb bits, the Morton key's leading 64 - cb bits)
+__device__ __forceinline__ uint64_t sort_key(uint4 c, int cb) {
+  const uint64_t k = morton_prefix64(c.x, c.y, c.z);
+  return cb > 0 ? ((uint64_t)c.w << (64 - cb)) | (k >> cb) : k;
+}
+
 // full-key order of two cells (same colony): true if a < b
 __device__ __forceinline__ bool morton_less(uint4 a, uint4 b) {
   if (a.w != b.w) return a.w < b.w;
@@ -231,9 +237,7 @@ __global__ __launch_bounds__(BT) void k_keys(const double *__restrict__ x, const
   const double4 a = aff[cid];
   const double px = x[i], py = y[i], pz = z[i];
   const uint32_t cx = loc_code(px, a.x, a.w), cy = loc_code(py, a.y, a.w), cz = loc_code(pz, a.z, a.w);
-  uint64_t k = morton_prefix64(cx, cy, cz);
-  if (cb > 0) k = ((uint64_t)cid << (64 - cb)) | (k >> cb);
-  key[i] = k;
+  key[i] = sort_key(make_uint4(cx, cy, cz, (uint32_t)cid), cb);
   val[i] = (int32_t)i;
   const int32_t t = ctype[i];
   const bool bad = t < 0 || t >= ntypes;
@@ -258,7 +262,8 @@ __global__ __launch_bounds__(BT) void k_keys(const double *__restrict__ x, const
 }
 
 __global__ __launch_bounds__(BT) void k_gather(const int32_t *__restrict__ perm, int64_t n,
-                                               const CellRec *__restrict__ rec, const double4 *__restrict__ aff, uint4 *__restrict__ code,
+                                               const CellRec *__restrict__ rec, int cb, uint64_t *__restrict__ key,
+                                               const double4 *__restrict__ aff, uint4 *__restrict__ code,
                                                double4 *__restrict__ pos, float4 *__restrict__ posf,
                                                float *__restrict__ young_s, int32_t *__restrict__ ctype_s,
                                                int32_t *__restrict__ phase_s) {
@@ -269,7 +274,9 @@ __global__ __launch_bounds__(BT) void k_gather(const int32_t *__restrict__ perm,
   if (o < 0 || o >= n) o = 0;  // unreachable for a valid permutation; bounds the gathers
   const double4 P = rec[o].pos;
   const uint4 X = rec[o].aux;
-  code[i] = rec[o].code;
+  const uint4 c = rec[o].code;
+  code[i] = c;
+  key[i] = sort_key(c, cb);
   const double4 a = aff[X.w];
   pos[i] = P;
   // the walk's screening copy: x, y, z relative to the colony's lower
@@ -616,7 +623,7 @@ tm_status tm_run_build(tm_ctx *c) {
                                            c->d_flags);
   TM_HIP(c, hipGetLastError());
   TM_TRY(tm_sort_pairs(c, c->d_key, c->d_perm, n, SORT_LO_BIT));
-  k_gather<<<tm_blocks(n, BT), BT, 0, st>>>(c->d_perm, n, c->d_rec, c->d_aff, c->d_code, c->d_pos,
+  k_gather<<<tm_blocks(n, BT), BT, 0, st>>>(c->d_perm, n, c->d_rec, cb, c->d_key, c->d_aff, c->d_code, c->d_pos,
                                              c->d_posf, c->d_young_s, c->d_ctype_s, c->d_phase_s);
   k_fixties<<<tm_blocks(n, BT), BT, 0, st>>>(c->d_key, n, c->d_perm, c->d_code, c->d_pos, c->d_posf,
                                               c->d_young_s, c->d_ctype_s, c->d_phase_s, c->d_flags);
