@@ -302,8 +302,8 @@ def environment_solve(tm, ctx, grid, prod):
     field.free()
     per = ms / max(it, 1)
     return {"z": D * dt / (res * res), "iterations": it, "relative_residual": rel, "ms": ms,
-            "ms_per_iteration": per, "gbs_per_iteration": 80.0 * nodes / (per * 1e-3) / 1e9,
-            "note": "wall time of the call, host checks of convergence every 8 iterations included"}
+            "ms_per_iteration": per, "gbs_per_iteration": 64.0 * nodes / (per * 1e-3) / 1e9,
+            "note": "wall time of the call, host checks of convergence included"}
 
 
 def time_sph(tm, ctx, a, n, P):
