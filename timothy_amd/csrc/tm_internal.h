@@ -36,9 +36,11 @@
 // squared distance stays finite in FP32
 #define TM_FAR 1.0e12
 // pinned host words of a context: [0, 16) copies of the device flags,
-// [TM_HFLAGS_CG, TM_HFLAGS_WORDS) the environment solve's state read back
+// [TM_HFLAGS_CG, TM_HFLAGS_PROGRESS) the environment solve's state read back,
+// TM_HFLAGS_PROGRESS where its kernels tell how far they are
 #define TM_HFLAGS_WORDS 32
 #define TM_HFLAGS_CG 16
+#define TM_HFLAGS_PROGRESS 31
 
 // A cell's inputs and location codes, in reference order.
 struct alignas(64) CellRec {

@@ -467,9 +467,8 @@ __global__ __launch_bounds__(BS) void k_neighbors(const double4 *__restrict__ po
 // cells lie in many places: a wave then takes fewer cells (launch_union).
 // Walk alone, per-lane before and this: 20 K-cell ball 119 and 43 us, 300 K
 // ball 208 and 175 us, 2M Gaussian 1,729 and 858 us, 4M cells in 128 colonies
-// 3,358 and 1,900 us, 3M of two types 3,605 and 1,580 us; the build, which no
-// longer makes the radix tree for it, 168 -> 143, 216 -> 178, 498 -> 367,
-// 872 -> 620 and 718 -> 531 us.  Also measured: the per-lane walk's tree read
+// 3,358 and 1,900 us, 3M of two types 3,605 and 1,580 us; and the build need not
+// make the radix tree (130 us of 500 at 2M).  Also measured: the per-lane walk's tree read
 // 64 slots at a time in its pre-order (103 dependent loads per wave against 48
 // here) 450 us of a 1.46 ms walk; distances on the vector unit 5% slower at
 // 2M; blocks of 32 cells 8% more loads.

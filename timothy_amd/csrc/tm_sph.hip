@@ -535,7 +535,7 @@ void launch_sph(tm_ctx *c) {
 }  // namespace
 
 // FP64 sums over one set of lists before tiles are made for more: at 2M cells
-// a sum takes 152 us without and 133 us with them, and they take 150 us
+// a sum takes 152 us without and 135 us with them, and they take 134 us
 static constexpr int DIRECT_SUMS = 8;
 
 tm_status tm_run_sph(tm_ctx *c, tm_precision prec) {
