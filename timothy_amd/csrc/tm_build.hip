@@ -165,19 +165,18 @@ __global__ __launch_bounds__(BT) void k_bbox(const double *__restrict__ x, const
 
 // src/octree.c:175-180: one workgroup per colony reduces its chunks' boxes; the
 // first clears the build's flags and what the sort wants cleared
-constexpr int AT = 512;
-__global__ __launch_bounds__(AT) void k_affine(const unsigned long long *__restrict__ cbox,
+template <int T>
+__global__ __launch_bounds__(T) void k_affine(const unsigned long long *__restrict__ cbox,
                                                const int64_t *__restrict__ col_chunk, int ncol,
                                                double4 *__restrict__ aff, unsigned int *__restrict__ flags,
                                                uint32_t *__restrict__ clear, int64_t words) {
-  __shared__ unsigned long long red[AT / 64][6];
+  __shared__ unsigned long long red[T / 64][6];
   const int c = blockIdx.x;
   if (c >= ncol) return;
   if (c == 0 && threadIdx.x < 4) flags[threadIdx.x] = 0;
-  if (c == 0)
-    for (int64_t i = threadIdx.x; i < words; i += AT) clear[i] = 0u;
+  for (int64_t i = (int64_t)c * T + threadIdx.x; i < words; i += (int64_t)gridDim.x * T) clear[i] = 0u;
   unsigned long long k[6] = {~0ull, ~0ull, ~0ull, 0ull, 0ull, 0ull};
-  for (int64_t q = col_chunk[c] + threadIdx.x; q < col_chunk[c + 1]; q += AT) {
+  for (int64_t q = col_chunk[c] + threadIdx.x; q < col_chunk[c + 1]; q += T) {
 #pragma unroll
     for (int a = 0; a < 3; ++a) {
       const unsigned long long lo = cbox[6 * q + a], hi = cbox[6 * q + 3 + a];
@@ -198,7 +197,7 @@ __global__ __launch_bounds__(AT) void k_affine(const unsigned long long *__restr
     for (int a = 0; a < 6; ++a) red[threadIdx.x >> 6][a] = k[a];
   __syncthreads();
   if (threadIdx.x != 0) return;
-  for (int q = 1; q < AT / 64; ++q)
+  for (int q = 1; q < T / 64; ++q)
     for (int a = 0; a < 3; ++a) {
       k[a] = red[q][a] < k[a] ? red[q][a] : k[a];
       k[a + 3] = red[q][a + 3] > k[a + 3] ? red[q][a + 3] : k[a + 3];
@@ -613,7 +612,11 @@ tm_status tm_run_build(tm_ctx *c) {
   uint32_t *clear = nullptr;
   int64_t words = 0;
   TM_TRY(tm_sort_prepare(c, n, &clear, &words));
-  k_affine<<<(unsigned)c->ncol, AT, 0, st>>>(c->d_cbox, c->d_col_chunk, c->ncol, c->d_aff, c->d_flags, clear, words);
+  // a wave where the colonies are small (20,000 of 20 cells: 19 us, with eight
+  // waves each 140)
+  auto affine = c->nchunks > 64 * (int64_t)c->ncol ? k_affine<512> : k_affine<64>;
+  affine<<<(unsigned)c->ncol, c->nchunks > 64 * (int64_t)c->ncol ? 512 : 64, 0, st>>>(
+      c->d_cbox, c->d_col_chunk, c->ncol, c->d_aff, c->d_flags, clear, words);
   TM_HIP(c, hipGetLastError());
   // Morton keys and the sort
   int cb = 0;
