@@ -24,10 +24,10 @@ def grid_of(ls, res):
 
 @pytest.mark.parametrize("ls", [(1, 1, 1), (3, 1, 1), (1, 5, 1), (2, 1, 7), (16, 16, 20), (17, 17, 18), (8, 10, 128),
                                 (11, 7, 133), (7, 9, 257), (33, 8, 128), (5, 63, 65), (1, 130, 129), (130, 1, 129),
-                                (4, 32776, 2)])
+                                (4, 32776, 2), (40, 65, 8), (31, 70, 5), (30, 40, 16), (15, 35, 31), (11, 31, 32)])
 def test_diffusion_grid_shapes(tm, oracle_mod, ctx, ls):
     """axes of one node, one workgroup's grids and the first past them (5,120 and 10,240
-    nodes), partial tiles and runs, more tiles than workgroups: the oracle's solution,
+    nodes), partial tiles and runs, every tile shape, more tiles than workgroups: the oracle's solution,
     over one step and two and where the iterations run out.  Both sides stop at residuals
     of 1e-12 |b| <= 1e-12 (1 + 12 z) |u|, and the operator's least eigenvalue is above one:
     2 steps, 2 sides, z = 0.7: 4e-11 |u|"""

@@ -92,7 +92,8 @@ __device__ __forceinline__ double rhs(const Op &A, double u, int64_t i, int64_t 
 }
 
 // The three streaming passes, marching along i: a workgroup owns an MJ x MK
-// block of (j, k) columns over a run of planes.  Per plane the operand of the
+// block of (j, k) columns over a run of planes (MK the next power of two from
+// the grid's extent along k, 8 to 64: 512^2 x 3 with 8 x 64 took twice the time).  Per plane the operand of the
 // stencil (x, p_new or p) is formed once per node, and once per node of the
 // block's edge ring (which the neighbouring blocks also form), into LDS; the
 // values of its own column one plane before and after stay in registers.
@@ -117,16 +118,18 @@ struct Blocks {
   unsigned int nk, nj, run;  // blocks along k and j, planes a run
   unsigned int count;        // workgroups' worth of work: at most MAXBLK are launched
 };
-constexpr int MJ = 8, MK = 64, MT = MJ * MK;
-constexpr int MHALO = 2 * MJ + 2 * MK;  // the edge ring without its corners
+constexpr int MT = 512;
 
-template <int PASS>
+template <int PASS, int MK>
 __global__ __launch_bounds__(MT) void k_cg(Op A, const double *__restrict__ src, double *__restrict__ x,
                                            double *__restrict__ r, const double *__restrict__ pold,
                                            double *__restrict__ pnew, Blocks B, int iter,
                                            CGState *__restrict__ st, const double *__restrict__ in,
                                            double *__restrict__ out, double *__restrict__ out2,
                                            unsigned int *progress) {
+  constexpr int MJ = MT / MK;
+  constexpr int MHALO = 2 * MJ + 2 * MK;  // the edge ring without its corners
+  static_assert(MHALO <= MT, "a thread forms one ring node");
   __shared__ double pl[2][MJ + 2][MK + 2];
   __shared__ double sh[2][MT / 64];
   constexpr bool down = PASS == UPDATE;
@@ -466,7 +469,8 @@ static double *scratch_addr[MAX_DEVICES];
 // fullest of 256 CUs the fewest planes, each run costing RUN_COST planes more
 // (it reads one more at either end, and every workgroup adds all the partial
 // sums).  A CU needs two workgroups to be busy, so one counts as two.
-static Blocks blocks_for(int64_t lx, int64_t ly, int64_t lz) {
+static Blocks blocks_for(int64_t lx, int64_t ly, int64_t lz, int MK) {
+  const int MJ = MT / MK;
   constexpr int64_t CUS = 256, FULL = 1024 / MT, MOST = 4 * FULL * CUS / 2, MIN_RUN = 2, RUN_COST = 3;
   Blocks B;
   B.nk = (unsigned int)((lz + MK - 1) / MK);
@@ -535,7 +539,8 @@ static tm_status run_diffusion(tm_ctx *c, double *work, const tm_grid *g, const 
     kern<<<1, ST, 0, c->stream>>>(A, src, field, d->tol, d->maxiter, d->substeps, st);
     TM_TRY(read_state());
   } else {
-    const Blocks B = blocks_for(lx, ly, lz);
+    const int mk = lz <= 8 ? 8 : lz <= 16 ? 16 : lz <= 32 ? 32 : 64;
+    const Blocks B = blocks_for(lx, ly, lz, mk);
     const int nblk = (int)std::min<unsigned int>(MAXBLK, B.count);
     // Iterations are launched until one of them is seen to have ended the solve,
     // three ahead of it up to CG's bound on their number and one beyond: enough
@@ -547,11 +552,16 @@ static tm_status run_diffusion(tm_ctx *c, double *work, const tm_grid *g, const 
     const int32_t bound = (int32_t)std::min(iterations_for(A, d->tol) + 1.0, 1e9);
     unsigned int *const progress = c->h_flags + TM_HFLAGS_PROGRESS;
     volatile unsigned int *const seen = progress;
+    auto pass = [&](auto k8, auto k16, auto k32, auto k64, const double *source, double *x, double *p, double *next,
+                    int iter, const double *in, double *out, double *out2) {
+      auto kern = mk == 8 ? k8 : mk == 16 ? k16 : mk == 32 ? k32 : k64;
+      kern<<<nblk, MT, 0, c->stream>>>(A, source, x, r, p, next, B, iter, st, in, out, out2, progress);
+    };
     for (int s = 0; s < d->substeps; ++s) {
       const int32_t before = it_total;
       *seen = 0u;
-      k_cg<INIT><<<nblk, MT, 0, c->stream>>>(A, src, field, r, nullptr, nullptr, B, 0, st, nullptr, part2, partb,
-                                             progress);
+      pass(k_cg<INIT, 8>, k_cg<INIT, 16>, k_cg<INIT, 32>, k_cg<INIT, 64>, src, field, nullptr, nullptr, 0, nullptr,
+           part2, partb);
       k_cg_start<<<1, 256, 0, c->stream>>>(part2, partb, nblk, d->tol, d->maxiter, st, progress);
       // the first direction is r; the two arrays then alternate
       double *pold = p0, *pnew = p1;
@@ -571,10 +581,10 @@ static tm_status run_diffusion(tm_ctx *c, double *work, const tm_grid *g, const 
           at = *seen;
         }
         if (at == ENDED) break;
-        k_cg<DIR><<<nblk, MT, 0, c->stream>>>(A, nullptr, nullptr, r, pold, pnew, B, launched, st, part2, part,
-                                              nullptr, progress);
-        k_cg<UPDATE><<<nblk, MT, 0, c->stream>>>(A, nullptr, field, r, pnew, nullptr, B, launched, st, part, part2,
-                                                 nullptr, progress);
+        pass(k_cg<DIR, 8>, k_cg<DIR, 16>, k_cg<DIR, 32>, k_cg<DIR, 64>, nullptr, nullptr, pold, pnew, launched, part2,
+             part, nullptr);
+        pass(k_cg<UPDATE, 8>, k_cg<UPDATE, 16>, k_cg<UPDATE, 32>, k_cg<UPDATE, 64>, nullptr, field, pnew, nullptr,
+             launched, part, part2, nullptr);
         std::swap(pold, pnew);
       }
       if (at != ENDED && launched > 0)
