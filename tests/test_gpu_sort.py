@@ -28,8 +28,8 @@ def morton(x, y, z, ext):
     return words
 
 
-# one tile, a tile's edges, the last and first size of each tile rule
-@pytest.mark.parametrize("n", [2, 1023, 1024, 1025, 16 * 1024 + 1, 65536, 65537, 786432, 786433, 4194304, 4194305])
+# one workgroup's sort, a tile's edges, the last and first size of each rule
+@pytest.mark.parametrize("n", [2, 63, 1025, 2048, 2049, 4095, 4096, 4097, 16 * 1024 + 1, 65536, 65537, 786432, 786433, 4194304, 4194305])
 def test_order_is_morton_order(tm, ctx, n):
     pos = np.random.default_rng(n).random((n, 3)) * max(n, 1000) ** (1 / 3)
     col = gen._cells(pos, np.zeros(n, np.int32), gen.Stream(7, 2), gen.CELLTYPES)

@@ -249,6 +249,91 @@ __global__ __launch_bounds__(RS_THREADS) void k_rs_scatter(const K *__restrict__
   }
 }
 
+// All passes of up to OT RS_ITEMS keys in one workgroup: the keys stay in
+// registers and change places through LDS.  Missing keys are all ones, after
+// the others in every pass.  Latency: one launch instead of seven; a build of 1K
+// cells 48 -> 32 us, of 2K 52 -> 33, of 4K 55 -> 44 (8K, eight keys a thread, 58
+// -> 63: not taken).
+constexpr int OT = 1024, OW = OT / 64;
+template <int RS_ITEMS>
+__global__ __launch_bounds__(OT) void k_rs_one(const uint64_t *__restrict__ keys, int32_t *__restrict__ vals, int n,
+                                               int lo_bit) {
+  __shared__ uint32_t cnt[OW][256];
+  __shared__ uint32_t tstart[256];
+  __shared__ uint32_t wsum[4];
+  __shared__ uint64_t skey[OT * RS_ITEMS];
+  __shared__ uint16_t sval[OT * RS_ITEMS];
+  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+  const int base = w * (64 * RS_ITEMS) + lane;
+  uint64_t k[RS_ITEMS];
+  uint32_t v[RS_ITEMS], rank[RS_ITEMS];
+#pragma unroll
+  for (int it = 0; it < RS_ITEMS; ++it) {
+    const int i = base + it * 64;
+    k[it] = i < n ? keys[i] : ~0ull;
+    v[it] = i < n ? (uint32_t)vals[i] : 0u;
+  }
+  for (int shift = lo_bit; shift < 64; shift += 8) {
+    for (int j = tid; j < OW * 256; j += OT) (&cnt[0][0])[j] = 0;
+    __syncthreads();
+#pragma unroll
+    for (int it = 0; it < RS_ITEMS; ++it) {
+      const uint32_t d = (uint32_t)(k[it] >> shift) & 255u;
+      const unsigned long long peers = tm_match8(d, true);
+      const uint32_t before = (uint32_t)__popcll(peers & tm_lanemask_lt());
+      const uint32_t c0 = cnt[w][d];
+      __builtin_amdgcn_wave_barrier();
+      if (before == 0) cnt[w][d] = c0 + (uint32_t)__popcll(peers);
+      __builtin_amdgcn_wave_barrier();
+      rank[it] = c0 + before;
+    }
+    __syncthreads();
+    uint32_t total = 0, inc = 0;
+    if (tid < 256) {
+      uint32_t c[OW];
+#pragma unroll
+      for (int q = 0; q < OW; ++q) c[q] = cnt[q][tid];
+#pragma unroll
+      for (int q = 0; q < OW; ++q) {
+        cnt[q][tid] = total;
+        total += c[q];
+      }
+      inc = total;
+#pragma unroll
+      for (int o = 1; o < 64; o <<= 1) {
+        const uint32_t y = __shfl_up(inc, o, 64);
+        if (lane >= o) inc += y;
+      }
+      if (lane == 63) wsum[w] = inc;
+    }
+    __syncthreads();
+    if (tid < 256) {
+      uint32_t wb = 0;
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+        if (q < w) wb += wsum[q];
+      tstart[tid] = wb + inc - total;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int it = 0; it < RS_ITEMS; ++it) {
+      const uint32_t d = (uint32_t)(k[it] >> shift) & 255u;
+      const uint32_t lp = tstart[d] + cnt[w][d] + rank[it];
+      skey[lp] = k[it];
+      sval[lp] = (uint16_t)v[it];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int it = 0; it < RS_ITEMS; ++it) {
+      k[it] = skey[base + it * 64];
+      v[it] = sval[base + it * 64];
+    }
+  }
+#pragma unroll
+  for (int it = 0; it < RS_ITEMS; ++it)
+    if (base + it * 64 < n) vals[base + it * 64] = (int32_t)v[it];
+}
+
 // ---- scan ----------------------------------------------------------------
 
 __device__ __forceinline__ uint32_t wave_incl_scan(uint32_t x) {
@@ -408,13 +493,20 @@ tm_status tm_sort_prepare(tm_ctx *c, int64_t n, uint32_t **clear, int64_t *words
 
 // Stable sort of (keys, vals) by key bits [lo_bit, 64) (lo_bit a multiple
 // of 16, so the passes are even in number); the passes ping-pong through
-// c->d_key_alt / d_val_alt.  vals ends sorted; once a pass has used the last bit
-// below 32 it hands on the keys' upper halves only, which lie sorted in the
-// first half of keys at the end (16 instead of 24 bytes a key and pass, and less
-// LDS; a build of 2M cells 312 -> 304 us, of 33M 4.33 -> 4.15 ms).
+// c->d_key_alt / d_val_alt.  vals, which starts as 0, 1, ..., n - 1, ends sorted;
+// the keys' own order at the end is left open: once a pass has used the last bit
+// below 32 it hands on the keys' upper halves only (16 instead of 24 bytes a key
+// and pass, and less LDS; a build of 2M cells 312 -> 304 us, of 33M 4.33 -> 4.15
+// ms).
 tm_status tm_sort_pairs(tm_ctx *c, uint64_t *keys, int32_t *vals, int64_t n, int lo_bit) {
   if (n <= 1) return TM_OK;
   if (lo_bit < 0 || lo_bit >= 32 || lo_bit % 16) return tm_fail(c, TM_ERR_INVALID, "sort: lo_bit");
+  if (n <= 4 * OT) {
+    auto one = n <= 2 * OT ? k_rs_one<2> : k_rs_one<4>;
+    one<<<1, OT, 0, c->stream>>>(keys, vals, (int)n, lo_bit);
+    TM_HIP(c, hipGetLastError());
+    return TM_OK;
+  }
   if (n <= FEW_N) return sort_passes<4, FEW>(c, keys, vals, n, lo_bit);
   if (n <= SMALL_N) return sort_passes<4, GROUPED>(c, keys, vals, n, lo_bit);
   if (n <= MEDIUM_N) return sort_passes<8, GROUPED>(c, keys, vals, n, lo_bit);
