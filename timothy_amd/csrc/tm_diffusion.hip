@@ -53,6 +53,14 @@ __device__ __forceinline__ void tell(unsigned int *progress, unsigned int what) 
   __hip_atomic_store(progress, what, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
+// what the host reads of the state, in pinned host memory, once the stream is done
+__device__ __forceinline__ void report(const CGState *st, CGState *host) {
+  host->bb = st->bb;
+  host->last = st->last;
+  host->iters = st->iters;
+  host->done = st->done;
+}
+
 struct Op {
   int64_t lx, ly, lz;
   double diag, z, zbc;
@@ -113,6 +121,8 @@ __device__ __forceinline__ double rhs(const Op &A, double u, int64_t i, int64_t 
 // two workgroups a CU: 4 x 64 in four takes 205 us, 16 x 64 in one 189 us but
 // 20 % more than 8 x 64 at 64^3 and below; one workgroup a CU takes 250 us,
 // four 217 us.
+// At most 80 registers (6 waves a SIMD), so that three workgroups fit where the
+// runs ask for them: 200x201x203 5.7 against 6.7 ms with 81.
 enum Pass { INIT, DIR, UPDATE };
 struct Blocks {
   unsigned int nk, nj, run;  // blocks along k and j, planes a run
@@ -121,12 +131,12 @@ struct Blocks {
 constexpr int MT = 512;
 
 template <int PASS, int MK>
-__global__ __launch_bounds__(MT) void k_cg(Op A, const double *__restrict__ src, double *__restrict__ x,
+__global__ __launch_bounds__(MT, 6) void k_cg(Op A, const double *__restrict__ src, double *__restrict__ x,
                                            double *__restrict__ r, const double *__restrict__ pold,
                                            double *__restrict__ pnew, Blocks B, int iter,
                                            CGState *__restrict__ st, const double *__restrict__ in,
                                            double *__restrict__ out, double *__restrict__ out2,
-                                           unsigned int *progress) {
+                                           unsigned int *progress, CGState *host) {
   constexpr int MJ = MT / MK;
   constexpr int MHALO = 2 * MJ + 2 * MK;  // the edge ring without its corners
   static_assert(MHALO <= MT, "a thread forms one ring node");
@@ -217,7 +227,10 @@ __global__ __launch_bounds__(MT) void k_cg(Op A, const double *__restrict__ src,
               st->rr[iter & 1] = rr;
               st->last = rr;
               st->iters = (unsigned long long)iter;
-              if (end) st->done = pass + 1u;
+              if (end) {
+                st->done = pass + 1u;
+                report(st, host);
+              }
               tell(progress, end ? ENDED : (unsigned int)iter);
             }
             if (end) return;
@@ -232,6 +245,7 @@ __global__ __launch_bounds__(MT) void k_cg(Op A, const double *__restrict__ src,
           if (!(pAp > 0.0)) {  // breakdown: the residual is zero (or the operator is not positive definite)
             if (blockIdx.x == 0 && threadIdx.x == 0) {
               st->done = pass + 1u;
+              report(st, host);
               tell(progress, ENDED);
             }
             return;
@@ -300,7 +314,7 @@ __global__ __launch_bounds__(MT) void k_cg(Op A, const double *__restrict__ src,
 
 __global__ __launch_bounds__(256) void k_cg_start(const double *__restrict__ part_rr,
                                                   const double *__restrict__ part_bb, int nblk, double tol,
-                                                  int maxiter, CGState *st, unsigned int *progress) {
+                                                  int maxiter, CGState *st, unsigned int *progress, CGState *host) {
   __shared__ double sh[2][4];
   const double rr = sum_parts<256>(part_rr, nblk, sh[0]), bb = sum_parts<256>(part_bb, nblk, sh[1]);
   if (threadIdx.x == 0) {
@@ -309,20 +323,22 @@ __global__ __launch_bounds__(256) void k_cg_start(const double *__restrict__ par
     st->tol2 = tol * tol;
     st->iters = 0;
     st->done = (rr <= st->tol2 * bb || maxiter <= 0) ? 1u : 0u;
+    if (st->done) report(st, host);
     tell(progress, st->done ? ENDED : 0u);
   }
 }
 
 // after `iters` iterations: their residual, and whether to stop
 __global__ __launch_bounds__(256) void k_cg_check(const double *__restrict__ part, int nblk, int iters, int maxiter,
-                                                  CGState *st) {
+                                                  CGState *st, CGState *host) {
   __shared__ double sh[4];
-  if (st->done) return;
+  if (st->done) return;  // (reported)
   const double rr = sum_parts<256>(part, nblk, sh);
   if (threadIdx.x == 0) {
     st->last = rr;
     st->iters = (unsigned long long)iters;
     if (rr <= st->tol2 * st->bb || iters >= maxiter) st->done = 1u;
+    report(st, host);
   }
 }
 
@@ -524,11 +540,10 @@ static tm_status run_diffusion(tm_ctx *c, double *work, const tm_grid *g, const 
   A.zbc = A.z * d->boundary;
   int32_t it_total = 0;
   double last_res = 0.0;
-  // the state is read back into pinned host memory set aside at tm_create
+  // the kernels report the state in pinned host memory set aside at tm_create
   CGState &h = *reinterpret_cast<CGState *>(c->h_flags + TM_HFLAGS_CG);
   auto read_state = [&]() -> tm_status {
     TM_HIP(c, hipGetLastError());
-    TM_HIP(c, hipMemcpyAsync(&h, st, sizeof(CGState), hipMemcpyDeviceToHost, c->stream));
     TM_HIP(c, hipStreamSynchronize(c->stream));
     last_res = h.bb > 0.0 ? sqrt(h.last / h.bb) : sqrt(h.last);
     it_total += (int32_t)h.iters;
@@ -536,7 +551,7 @@ static tm_status run_diffusion(tm_ctx *c, double *work, const tm_grid *g, const 
   };
   if (total <= SMALL_NODES && d->substeps > 0) {
     auto kern = total <= ST * 5 ? k_cg_small<5> : k_cg_small<10>;
-    kern<<<1, ST, 0, c->stream>>>(A, src, field, d->tol, d->maxiter, d->substeps, st);
+    kern<<<1, ST, 0, c->stream>>>(A, src, field, d->tol, d->maxiter, d->substeps, &h);
     TM_TRY(read_state());
   } else {
     const int mk = lz <= 8 ? 8 : lz <= 16 ? 16 : lz <= 32 ? 32 : 64;
@@ -555,21 +570,21 @@ static tm_status run_diffusion(tm_ctx *c, double *work, const tm_grid *g, const 
     auto pass = [&](auto k8, auto k16, auto k32, auto k64, const double *source, double *x, double *p, double *next,
                     int iter, const double *in, double *out, double *out2) {
       auto kern = mk == 8 ? k8 : mk == 16 ? k16 : mk == 32 ? k32 : k64;
-      kern<<<nblk, MT, 0, c->stream>>>(A, source, x, r, p, next, B, iter, st, in, out, out2, progress);
+      kern<<<nblk, MT, 0, c->stream>>>(A, source, x, r, p, next, B, iter, st, in, out, out2, progress, &h);
     };
     for (int s = 0; s < d->substeps; ++s) {
       const int32_t before = it_total;
       *seen = 0u;
       pass(k_cg<INIT, 8>, k_cg<INIT, 16>, k_cg<INIT, 32>, k_cg<INIT, 64>, src, field, nullptr, nullptr, 0, nullptr,
            part2, partb);
-      k_cg_start<<<1, 256, 0, c->stream>>>(part2, partb, nblk, d->tol, d->maxiter, st, progress);
+      k_cg_start<<<1, 256, 0, c->stream>>>(part2, partb, nblk, d->tol, d->maxiter, st, progress, &h);
       // the first direction is r; the two arrays then alternate
       double *pold = p0, *pnew = p1;
       int32_t launched = 0;
       unsigned int at = 0u;
       for (; launched < d->maxiter; ++launched) {
         if (launched == bound) {  // (next to no coupling: the bound is the number)
-          k_cg_check<<<1, 256, 0, c->stream>>>(part2, nblk, launched, d->maxiter, st);
+          k_cg_check<<<1, 256, 0, c->stream>>>(part2, nblk, launched, d->maxiter, st, &h);
           TM_TRY(read_state());
           at = h.done ? ENDED : 0u;
           if (at == ENDED) break;
@@ -588,7 +603,7 @@ static tm_status run_diffusion(tm_ctx *c, double *work, const tm_grid *g, const 
         std::swap(pold, pnew);
       }
       if (at != ENDED && launched > 0)
-        k_cg_check<<<1, 256, 0, c->stream>>>(part2, nblk, launched, d->maxiter, st);
+        k_cg_check<<<1, 256, 0, c->stream>>>(part2, nblk, launched, d->maxiter, st, &h);
       it_total = before;
       TM_TRY(read_state());
     }
