@@ -56,3 +56,20 @@ def test_gradient_and_interp_grid_shapes(tm, oracle_mod, ctx, ls, dtype):
     assert np.array_equal(out.get().reshape(-1, 4), ref)
     for a in (f_d, g_d, out):
         a.free()
+
+
+@pytest.mark.parametrize("ls", [(64, 2, 2), (43, 3, 2), (300, 2, 3), (2, 2, 31), (9, 31, 2), (70, 7, 9), (70, 8, 8)])
+def test_gradient_thin_planes(tm, oracle_mod, ctx, ls):
+    """planes of less than 64 nodes, one lane a node: whole and partial workgroups, and the
+    first plane past the rule; bit-exact in both types"""
+    res = np.float32(1.7)
+    grid = dict(lower=np.zeros(3), resolution=res, loweridx=np.zeros(3, int), upperidx=np.array(ls) - 1,
+                localsize=np.array(ls))
+    f = np.random.default_rng(int(np.prod(ls))).standard_normal(int(np.prod(ls)))
+    for dtype in (np.float64, np.float32):
+        print(f"thin gradient {ls} {np.dtype(dtype).name}", flush=True)
+        v = f.astype(dtype)
+        f_d, g_d = tm.DeviceArray.from_host(ctx, v), tm.DeviceArray(ctx, 3 * f.size, dtype)
+        ctx.field_gradient(grid, f_d, g_d)
+        want = oracle_mod.fieldgradient(ls, res, v) if dtype == np.float64 else gradient_f32(v.reshape(ls), res)
+        assert np.array_equal(g_d.get(), want)

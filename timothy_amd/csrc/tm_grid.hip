@@ -576,9 +576,11 @@ __global__ __launch_bounds__(256) void k_interp(const double4 *__restrict__ pos,
   }
 }
 
-// interior (f[i+1]-f[i-1])/res; faces one-sided (no neighbouring ranks):
-// (f[1]-f[0])/res, (f[L-1]-f[L-2])/res
-//
+// one component of the gradient: interior (f[i+1]-f[i-1])/res; faces one-sided
+// (no neighbouring ranks): (f[1]-f[0])/res, (f[L-1]-f[L-2])/res
+__device__ __forceinline__ double slope(double hi, double lo, float res) { return (hi - lo) / (double)res; }
+__device__ __forceinline__ float slope(float hi, float lo, float res) { return (hi - lo) / res; }
+
 // A lane owns one (j, k) column of a run of planes and marches along i, so that
 // its i neighbours stay in registers; the j and k neighbours come from the
 // caches.  A wave's 64 nodes are consecutive in the plane: their 192 results go
@@ -619,15 +621,9 @@ __global__ __launch_bounds__(256) void k_gradient(const F *__restrict__ f, F *__
       if (i + 2 < lx) after = c[2 * plane];
       xn = cross(c + plane);
     }
-    if constexpr (sizeof(F) == 8) {
-      st[3 * lane + 0] = (F)(((double)next - (double)prev) / (double)res);
-      st[3 * lane + 1] = (F)(((double)x.jp - (double)x.jm) / (double)res);
-      st[3 * lane + 2] = (F)(((double)x.kp - (double)x.km) / (double)res);
-    } else {
-      st[3 * lane + 0] = (next - prev) / (F)res;
-      st[3 * lane + 1] = (x.jp - x.jm) / (F)res;
-      st[3 * lane + 2] = (x.kp - x.km) / (F)res;
-    }
+    st[3 * lane + 0] = slope(next, prev, res);
+    st[3 * lane + 1] = slope(x.jp, x.jm, res);
+    st[3 * lane + 2] = slope(x.kp, x.km, res);
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
     __builtin_amdgcn_wave_barrier();
     F *dst = g + 3 * (i * plane + m0);
@@ -641,6 +637,25 @@ __global__ __launch_bounds__(256) void k_gradient(const F *__restrict__ f, F *__
     next = after;
     x = xn;
   }
+}
+
+// The same with a lane per node, for planes that would leave lanes of the march
+// idle.  FP64, this against the march (there with up to 16 times as many, shorter
+// runs): 200,000 x 2 x 2 8 and 48 us, 100,000 x 3 x 5 12 and 30 us,
+// 50,000 x 7 x 7 17 and 22 us; 20,000 x 8 x 8 10.5 and 9.6 us.
+template <typename F>
+__global__ __launch_bounds__(256) void k_gradient_thin(const F *__restrict__ f, F *__restrict__ g, int64_t lx,
+                                                       unsigned int ly, unsigned int lz, float res) {
+  const unsigned int plane = ly * lz;
+  const int64_t node = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (node >= lx * plane) return;
+  const int64_t i = node / plane;
+  const unsigned int m = (unsigned int)(node - i * plane), j = m / lz, k = m - j * lz;
+  const F *c = f + node;
+  F *dst = g + 3 * node;
+  dst[0] = slope(i < lx - 1 ? c[plane] : c[0], i > 0 ? *(c - plane) : c[0], res);
+  dst[1] = slope(j < ly - 1 ? c[lz] : c[0], j > 0 ? *(c - lz) : c[0], res);
+  dst[2] = slope(k < lz - 1 ? c[1] : c[0], k > 0 ? *(c - 1) : c[0], res);
 }
 
 }  // namespace
@@ -729,12 +744,19 @@ static tm_status gradient_impl(tm_ctx *c, const tm_grid *grid, const F *field, F
   if (!c) return TM_ERR_INVALID;
   TM_TRY(check_grid(c, grid));
   if (!field || !gradient) return tm_fail(c, TM_ERR_INVALID, "field or gradient is NULL");
+  const int64_t lx = grid->localsize[0], ly = grid->localsize[1], lz = grid->localsize[2];
+  if (ly * lz < 64) {
+    k_gradient_thin<F><<<tm_blocks(lx * ly * lz, 256), 256, 0, c->stream>>>(field, gradient, lx, (unsigned)ly,
+                                                                            (unsigned)lz, grid->resolution);
+    TM_HIP(c, hipGetLastError());
+    return TM_OK;
+  }
   // chunks of 256 columns times runs of planes: about 2,048 workgroups, runs of
   // at least four planes
-  const int64_t lx = grid->localsize[0], nchunk = tm_blocks(grid->localsize[1] * grid->localsize[2], 256);
+  const int64_t nchunk = tm_blocks(ly * lz, 256);
   const int64_t want = std::max<int64_t>(1, std::min<int64_t>((lx + 3) / 4, 2048 / nchunk)), run = (lx + want - 1) / want;
   k_gradient<F><<<(unsigned)(nchunk * ((lx + run - 1) / run)), 256, 0, c->stream>>>(
-      field, gradient, lx, grid->localsize[1], grid->localsize[2], (unsigned)nchunk, run, grid->resolution);
+      field, gradient, lx, ly, lz, (unsigned)nchunk, run, grid->resolution);
   TM_HIP(c, hipGetLastError());
   return TM_OK;
 }
