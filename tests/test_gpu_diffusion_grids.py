@@ -51,3 +51,37 @@ def test_diffusion_grid_shapes(tm, oracle_mod, ctx, ls):
         assert np.linalg.norm(got - ref) <= 4e-11 * np.linalg.norm(ref)
     f.free()
     s.free()
+
+
+# long grids of thin planes, taken with a lane per node: few and many planes, rows across
+# workgroups, several nodes a lane (beyond 524,288); planes that fill just less than half
+# the lanes of the march's blocks, and half; the march with more tiles than workgroups
+@pytest.mark.parametrize("ls", [(5121, 2, 1), (2561, 2, 2), (1153, 3, 3), (5000, 3, 2), (160, 5, 13), (45, 15, 16),
+                                (45, 16, 16), (81, 33, 33), (19, 9, 65), (60001, 3, 3), (262145, 2, 1), (131073, 2, 2),
+                                (1, 1500, 1500)])
+def test_diffusion_thin_planes(tm, oracle_mod, ctx, ls):
+    """as above, with the same bound"""
+    test_diffusion_grid_shapes(tm, oracle_mod, ctx, ls)
+
+
+def test_diffusion_thin_planes_take_no_longer(tm, ctx):
+    """a solve of two iterations on 100,000 x 3 x 3 nodes against one on as many in a
+    cube: about its time with a lane per node, 8 times it in blocks of mostly idle lanes"""
+    import time
+
+    best = {}
+    for ls in ((100000, 3, 3), (96, 96, 98)):
+        u0 = np.full(int(np.prod(ls)), 0.15)
+        f = tm.DeviceArray.from_host(ctx, u0)
+        par = tm.Diffusion.make(1.8e-5 * 4.0, 1.0, 0.1575, 0.0, 1e-12, 400, 1)
+        ts = []
+        for _ in range(12):
+            f.set(u0)
+            ctx.sync()
+            t0 = time.perf_counter()
+            it, _rel = ctx.diffusion_step(grid_of(ls, 2.0), par, f)
+            ts.append(time.perf_counter() - t0)
+        say(f"{ls}: {it} iterations, {1e6 * min(ts):.0f} us")
+        best[ls] = min(ts)
+        f.free()
+    assert best[(100000, 3, 3)] <= 3.0 * best[(96, 96, 98)]

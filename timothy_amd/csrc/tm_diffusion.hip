@@ -26,6 +26,7 @@
 // the remaining iterations return at once, so the host launches a few iterations
 // ahead and reads the state once.
 #include <mutex>
+#include <type_traits>
 
 #include "tm_internal.h"
 
@@ -130,6 +131,50 @@ struct Blocks {
 };
 constexpr int MT = 512;
 
+// What DIR and UPDATE start with: the scalar of the pass from the partial sums of
+// the one before (sh: as for block_sum), or false where there is nothing to do.
+template <int PASS>
+__device__ __forceinline__ bool begin(int iter, CGState *st, const double *__restrict__ in, double *sh,
+                                      unsigned int *progress, CGState *host, double &scale) {
+  const unsigned int pass = 2u * (unsigned int)iter + (PASS == DIR ? 1u : 2u), mark = st->done;
+  if constexpr (PASS == DIR) {
+    if (iter > 0) {
+      const double before = st->rr[(iter - 1) & 1], limit = st->tol2 * st->bb;
+      const double rr = sum_parts<MT>(in, (int)gridDim.x, sh);
+      if (mark && mark <= pass) return false;
+      const bool end = rr <= limit;
+      if (blockIdx.x == 0 && threadIdx.x == 0) {
+        st->rr[iter & 1] = rr;
+        st->last = rr;
+        st->iters = (unsigned long long)iter;
+        if (end) {
+          st->done = pass + 1u;
+          report(st, host);
+        }
+        tell(progress, end ? ENDED : (unsigned int)iter);
+      }
+      if (end) return false;
+      scale = rr / before;
+    } else if (mark) {
+      return false;
+    }
+  } else {
+    const double rr = st->rr[iter & 1];
+    const double pAp = sum_parts<MT>(in, (int)gridDim.x, sh);
+    if (mark && mark <= pass) return false;
+    if (!(pAp > 0.0)) {  // breakdown: the residual is zero (or the operator is not positive definite)
+      if (blockIdx.x == 0 && threadIdx.x == 0) {
+        st->done = pass + 1u;
+        report(st, host);
+        tell(progress, ENDED);
+      }
+      return false;
+    }
+    scale = rr / pAp;
+  }
+  return true;
+}
+
 template <int PASS, int MK>
 __global__ __launch_bounds__(MT, 6) void k_cg(Op A, const double *__restrict__ src, double *__restrict__ x,
                                            double *__restrict__ r, const double *__restrict__ pold,
@@ -215,44 +260,8 @@ __global__ __launch_bounds__(MT, 6) void k_cg(Op A, const double *__restrict__ s
       }
     }
     if (c == b0) {
-      if constexpr (PASS != INIT) {
-        const unsigned int pass = 2u * (unsigned int)iter + (PASS == DIR ? 1u : 2u), mark = st->done;
-        if constexpr (PASS == DIR) {
-          if (iter > 0) {
-            const double before = st->rr[(iter - 1) & 1], limit = st->tol2 * st->bb;
-            const double rr = sum_parts<MT>(in, (int)gridDim.x, sh[0]);
-            if (mark && mark <= pass) return;
-            const bool end = rr <= limit;
-            if (blockIdx.x == 0 && threadIdx.x == 0) {
-              st->rr[iter & 1] = rr;
-              st->last = rr;
-              st->iters = (unsigned long long)iter;
-              if (end) {
-                st->done = pass + 1u;
-                report(st, host);
-              }
-              tell(progress, end ? ENDED : (unsigned int)iter);
-            }
-            if (end) return;
-            scale = rr / before;
-          } else if (mark) {
-            return;
-          }
-        } else {
-          const double rr = st->rr[iter & 1];
-          const double pAp = sum_parts<MT>(in, (int)gridDim.x, sh[0]);
-          if (mark && mark <= pass) return;
-          if (!(pAp > 0.0)) {  // breakdown: the residual is zero (or the operator is not positive definite)
-            if (blockIdx.x == 0 && threadIdx.x == 0) {
-              st->done = pass + 1u;
-              report(st, host);
-              tell(progress, ENDED);
-            }
-            return;
-          }
-          scale = rr / pAp;
-        }
-      }
+      if constexpr (PASS != INIT)
+        if (!begin<PASS>(iter, st, in, sh[0], progress, host, scale)) return;
     } else {
       __syncthreads();  // the buffers' last readers are done
     }
@@ -302,6 +311,67 @@ __global__ __launch_bounds__(MT, 6) void k_cg(Op A, const double *__restrict__ s
       }
       behind = cur;
       cur = ahead;
+    }
+  }
+  const double s = block_sum<MT>(acc, sh[1]);
+  if (threadIdx.x == 0) out[b0] = s;
+  if constexpr (PASS == INIT) {
+    const double s2 = block_sum<MT>(acc2, sh[0]);
+    if (threadIdx.x == 0) out2[b0] = s2;
+  }
+}
+
+// The passes with a lane per node, for planes that would leave more than half the
+// march's lanes idle.  The operand at a node and its six neighbours comes from
+// memory, through the caches, which hold such planes.  Latency on small grids,
+// then the loads' issue.  At most 1,024 workgroups, whose partial sums every one
+// adds: with 2,048 100,000x3x3 takes 635 against 571 us.
+constexpr int64_t NODE_BLOCKS = 1024;
+template <int PASS>
+__global__ __launch_bounds__(MT) void k_cg_nodes(Op A, const double *__restrict__ src, double *__restrict__ x,
+                                                 double *__restrict__ r, const double *__restrict__ pold,
+                                                 double *__restrict__ pnew, int64_t chunk, int iter,
+                                                 CGState *__restrict__ st, const double *__restrict__ in,
+                                                 double *__restrict__ out, double *__restrict__ out2,
+                                                 unsigned int *progress, CGState *host) {
+  __shared__ double sh[2][MT / 64];
+  double scale = 0.0;  // beta or alpha
+  if constexpr (PASS != INIT)
+    if (!begin<PASS>(iter, st, in, sh[0], progress, host, scale)) return;
+  const int64_t b0 = tm_xcd_block();
+  const int64_t total = A.lx * A.ly * A.lz, lo = b0 * chunk, hi = lo + chunk < total ? lo + chunk : total;
+  const int64_t sx = A.ly * A.lz, sy = A.lz;
+  const double *const u = PASS == INIT ? x : PASS == UPDATE ? pold : r;
+  auto at = [&](int64_t node) -> double {
+    if constexpr (PASS == DIR) return iter > 0 ? u[node] + scale * pold[node] : u[node];
+    return u[node];
+  };
+  double acc = 0.0, acc2 = 0.0;
+  for (int64_t node = lo + threadIdx.x; node < hi; node += MT) {
+    const int64_t i = node / sx, m = node - i * sx, j = m / sy, k = m - j * sy;
+    const double cur = at(node);
+    double nb = 0.0;
+    if (i > 0) nb += at(node - sx);
+    if (i < A.lx - 1) nb += at(node + sx);
+    if (j > 0) nb += at(node - sy);
+    if (j < A.ly - 1) nb += at(node + sy);
+    if (k > 0) nb += at(node - 1);
+    if (k < A.lz - 1) nb += at(node + 1);
+    const double ap = A.diag * cur - A.z * nb;
+    if constexpr (PASS == INIT) {
+      const double bv = rhs(A, cur, i, j, k, src, node);
+      const double res = bv - ap;
+      r[node] = res;
+      acc += res * res;
+      acc2 += bv * bv;
+    } else if constexpr (PASS == DIR) {
+      pnew[node] = cur;
+      acc += cur * ap;
+    } else {
+      x[node] += scale * cur;
+      const double now = r[node] - scale * ap;
+      r[node] = now;
+      acc += now * now;
     }
   }
   const double s = block_sum<MT>(acc, sh[1]);
@@ -556,7 +626,16 @@ static tm_status run_diffusion(tm_ctx *c, double *work, const tm_grid *g, const 
   } else {
     const int mk = lz <= 8 ? 8 : lz <= 16 ? 16 : lz <= 32 ? 32 : 64;
     const Blocks B = blocks_for(lx, ly, lz, mk);
-    const int nblk = (int)std::min<unsigned int>(MAXBLK, B.count);
+    // Where a plane fills less than half the lanes of its blocks, a lane per node.
+    // Solves with a coupling of 0.5, march and lane per node: 100,000x3x3 (2 %) 5,950
+    // and 571 us, 3,000x8x8 (12 %) 544 and 369, 4,000x9x33 (29 %) 1,190 and 971,
+    // 2,000x33x33 (43 %) 1,456 and 1,374, 65^3 (46 %) 566 and 475, 5,000x12x20 (47 %)
+    // 922 and 951; 10,000x16x16 (50 %) 1,315 and 1,399, 1,000x40x40 (62 %) 968 and
+    // 1,204.
+    const bool nodes = 2 * ly * lz < (int64_t)B.nk * B.nj * MT;
+    // (whole rounds of a workgroup's nodes each)
+    const int64_t rounds = (total + MT - 1) / MT, chunk = (rounds + NODE_BLOCKS - 1) / NODE_BLOCKS * MT;
+    const int nblk = nodes ? (int)((total + chunk - 1) / chunk) : (int)std::min<unsigned int>(MAXBLK, B.count);
     // Iterations are launched until one of them is seen to have ended the solve,
     // three ahead of it up to CG's bound on their number and one beyond: enough
     // that the GPU does not wait for the host, and few that find the solve ended
@@ -567,16 +646,23 @@ static tm_status run_diffusion(tm_ctx *c, double *work, const tm_grid *g, const 
     const int32_t bound = (int32_t)std::min(iterations_for(A, d->tol) + 1.0, 1e9);
     unsigned int *const progress = c->h_flags + TM_HFLAGS_PROGRESS;
     volatile unsigned int *const seen = progress;
-    auto pass = [&](auto k8, auto k16, auto k32, auto k64, const double *source, double *x, double *p, double *next,
-                    int iter, const double *in, double *out, double *out2) {
-      auto kern = mk == 8 ? k8 : mk == 16 ? k16 : mk == 32 ? k32 : k64;
+    auto pass = [&](auto which, const double *source, double *x, double *p, double *next, int iter, const double *in,
+                    double *out, double *out2) {
+      constexpr int P = decltype(which)::value;
+      if (nodes) {
+        k_cg_nodes<P><<<nblk, MT, 0, c->stream>>>(A, source, x, r, p, next, chunk, iter, st, in, out, out2, progress, &h);
+        return;
+      }
+      auto kern = mk == 8 ? k_cg<P, 8> : mk == 16 ? k_cg<P, 16> : mk == 32 ? k_cg<P, 32> : k_cg<P, 64>;
       kern<<<nblk, MT, 0, c->stream>>>(A, source, x, r, p, next, B, iter, st, in, out, out2, progress, &h);
     };
+    constexpr std::integral_constant<int, INIT> init;
+    constexpr std::integral_constant<int, DIR> direction;
+    constexpr std::integral_constant<int, UPDATE> update;
     for (int s = 0; s < d->substeps; ++s) {
       const int32_t before = it_total;
       *seen = 0u;
-      pass(k_cg<INIT, 8>, k_cg<INIT, 16>, k_cg<INIT, 32>, k_cg<INIT, 64>, src, field, nullptr, nullptr, 0, nullptr,
-           part2, partb);
+      pass(init, src, field, nullptr, nullptr, 0, nullptr, part2, partb);
       k_cg_start<<<1, 256, 0, c->stream>>>(part2, partb, nblk, d->tol, d->maxiter, st, progress, &h);
       // the first direction is r; the two arrays then alternate
       double *pold = p0, *pnew = p1;
@@ -596,10 +682,8 @@ static tm_status run_diffusion(tm_ctx *c, double *work, const tm_grid *g, const 
           at = *seen;
         }
         if (at == ENDED) break;
-        pass(k_cg<DIR, 8>, k_cg<DIR, 16>, k_cg<DIR, 32>, k_cg<DIR, 64>, nullptr, nullptr, pold, pnew, launched, part2,
-             part, nullptr);
-        pass(k_cg<UPDATE, 8>, k_cg<UPDATE, 16>, k_cg<UPDATE, 32>, k_cg<UPDATE, 64>, nullptr, field, pnew, nullptr,
-             launched, part, part2, nullptr);
+        pass(direction, nullptr, nullptr, pold, pnew, launched, part2, part, nullptr);
+        pass(update, nullptr, field, pnew, nullptr, launched, part, part2, nullptr);
         std::swap(pold, pnew);
       }
       if (at != ENDED && launched > 0)
