@@ -584,12 +584,13 @@ __device__ __forceinline__ float slope(float hi, float lo, float res) { return (
 // A lane owns one (j, k) column of a run of planes and marches along i, so that
 // its i neighbours stay in registers; the j and k neighbours come from the
 // caches.  A wave's 64 nodes are consecutive in the plane: their 192 results go
-// through LDS and out in 16-byte stores that pass by the caches: three times the
-// field, they would push it out of the memory-side cache and be gone before
-// they are read.  256^3 FP64 (134 MB in, 403 MB out): 158 us with a lane per
-// node and strided stores, 149 us marching, 79 us with such stores (6.8 TB/s,
-// the field partly from that cache); 384^3 FP32: 267, 237, 137 us.
-template <typename F>
+// through LDS and out in 16-byte stores.  PAST: the stores pass by the caches,
+// as results too large for the memory-side cache would push the field out of it
+// and be gone before they are read.  256^3 FP64 (134 MB in, 403 MB out): 158 us
+// with a lane per node and strided stores, 149 us marching, 79 us with such
+// stores (6.8 TB/s, the field partly from that cache); 384^3 FP32: 267, 237, 137
+// us.
+template <typename F, bool PAST>
 __global__ __launch_bounds__(256) void k_gradient(const F *__restrict__ f, F *__restrict__ g, int64_t lx, int64_t ly,
                                                   int64_t lz, unsigned int nchunk, int64_t run, float res) {
   constexpr int E = 16 / (int)sizeof(F);
@@ -627,7 +628,11 @@ __global__ __launch_bounds__(256) void k_gradient(const F *__restrict__ f, F *__
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
     __builtin_amdgcn_wave_barrier();
     F *dst = g + 3 * (i * plane + m0);
-    for (int v = lane; v < nv / E; v += 64) __builtin_nontemporal_store(*(const lvec *)(st + E * v), (vec *)(dst + E * v));
+    for (int v = lane; v < nv / E; v += 64) {
+      const lvec w = *(const lvec *)(st + E * v);
+      if constexpr (PAST) __builtin_nontemporal_store(w, (vec *)(dst + E * v));
+      else *(vec *)(dst + E * v) = w;
+    }
     const int rest = nv / E * E + lane;
     if (rest < nv) dst[rest] = st[rest];
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
@@ -639,12 +644,10 @@ __global__ __launch_bounds__(256) void k_gradient(const F *__restrict__ f, F *__
   }
 }
 
-// The same with a lane per node, for planes that would leave lanes of the march
-// idle.  FP64, this against the march (there with up to 16 times as many, shorter
-// runs): 200,000 x 2 x 2 8 and 48 us, 100,000 x 3 x 5 12 and 30 us,
-// 50,000 x 7 x 7 17 and 22 us; 20,000 x 8 x 8 10.5 and 9.6 us.
+// The same with a lane per node, for small grids and for planes that would leave
+// lanes of the march idle.  Latency, and the strided stores of three values.
 template <typename F>
-__global__ __launch_bounds__(256) void k_gradient_thin(const F *__restrict__ f, F *__restrict__ g, int64_t lx,
+__global__ __launch_bounds__(256) void k_gradient_nodes(const F *__restrict__ f, F *__restrict__ g, int64_t lx,
                                                        unsigned int ly, unsigned int lz, float res) {
   const unsigned int plane = ly * lz;
   const int64_t node = (int64_t)blockIdx.x * 256 + threadIdx.x;
@@ -745,18 +748,34 @@ static tm_status gradient_impl(tm_ctx *c, const tm_grid *grid, const F *field, F
   TM_TRY(check_grid(c, grid));
   if (!field || !gradient) return tm_fail(c, TM_ERR_INVALID, "field or gradient is NULL");
   const int64_t lx = grid->localsize[0], ly = grid->localsize[1], lz = grid->localsize[2];
-  if (ly * lz < 64) {
-    k_gradient_thin<F><<<tm_blocks(lx * ly * lz, 256), 256, 0, c->stream>>>(field, gradient, lx, (unsigned)ly,
-                                                                            (unsigned)lz, grid->resolution);
+  // By the bytes of field and gradient, which a sampling of the field reads next.
+  // Gradient and interpolation of 1M Gaussian cells; lane per node, march, march
+  // with stores past the caches, us:  within the L2 caches (8 x 4 MB) FP32 40^3 23.7 /
+  // 25.2 / 35.0, 110^3 33.7 / 35.3 / 56.0, 128^3 (34 MB) 35.6 / 37.1 / 59.9, FP64 96^3
+  // 35.0 / 35.9 / 57.7;  within the memory-side cache (256 MB) FP64 120^3 43.5 / 42.8 /
+  // 64.7, FP32 230^3 (195 MB) 88 / 75 / 107, FP64 184^3 (199 MB) 106 / 111 / 99 (68 / 54
+  // / 62 with 224K cells);  beyond FP64 192^3 (226 MB) 116 / 121 / 106, FP32 256^3 140 /
+  // 141 / 116, FP64 256^3 265 / 259 / 224.
+  // Planes that fill less than three quarters of the lanes of their chunks of 256: a
+  // lane per node within the memory-side cache's size.  FP64 planes of 8 x 9, 9 x 15,
+  // 16 x 17, 21 x 25, lane per node and the march's better form: 150 MB 27 / 37, 30 /
+  // 37, 35 / 37, 35 / 31 us (FP32 35 / 38); 270 MB 52 / 71, 51 / 70, 61 / 70, 61 / 67;
+  // 350 MB 101 / 82, 95 / 86, 91 / 83, 89 / 87.  Planes of less than 64 nodes, of any
+  // size: 200,000 x 2 x 2 8 and 48 us, 437,500 x 5 x 5 100 and 154.
+  const int64_t total = lx * ly * lz, bytes = 4 * (int64_t)sizeof(F) * total, nchunk = tm_blocks(ly * lz, 256);
+  const int64_t most = (int64_t)(4 * ly * lz < 3 * 256 * nchunk ? 256 : 32) << 20;
+  if (ly * lz < 64 || bytes <= most) {
+    k_gradient_nodes<F><<<tm_blocks(total, 256), 256, 0, c->stream>>>(field, gradient, lx, (unsigned)ly, (unsigned)lz,
+                                                                      grid->resolution);
     TM_HIP(c, hipGetLastError());
     return TM_OK;
   }
   // chunks of 256 columns times runs of planes: about 2,048 workgroups, runs of
   // at least four planes
-  const int64_t nchunk = tm_blocks(ly * lz, 256);
   const int64_t want = std::max<int64_t>(1, std::min<int64_t>((lx + 3) / 4, 2048 / nchunk)), run = (lx + want - 1) / want;
-  k_gradient<F><<<(unsigned)(nchunk * ((lx + run - 1) / run)), 256, 0, c->stream>>>(
-      field, gradient, lx, ly, lz, (unsigned)nchunk, run, grid->resolution);
+  auto march = bytes <= (int64_t)192 << 20 ? k_gradient<F, false> : k_gradient<F, true>;
+  march<<<(unsigned)(nchunk * ((lx + run - 1) / run)), 256, 0, c->stream>>>(field, gradient, lx, ly, lz,
+                                                                            (unsigned)nchunk, run, grid->resolution);
   TM_HIP(c, hipGetLastError());
   return TM_OK;
 }
