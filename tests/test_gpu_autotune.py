@@ -118,3 +118,26 @@ def test_autotune_report_and_results(tm, ctx, case):
         check_mixed(ctx.results(), ref)
         ctx.step(tm.FP64)
         check_fp64(ctx.results(), ref)
+
+
+def test_autotune_failed_trial_leaves_the_shapes(tm, ctx, case):
+    """a trial that fails (lists of eight slots, too few for this colony) leaves every launch
+    shape as it was, and the next step works"""
+    col, ref = case
+    keys = ("nbr_block", "walk_window", "walk_coop", "walk_f32", "tile_width", "sph_block", "sph_lanes",
+            "sph_unroll_fp64", "sph_unroll_mixed")
+    ctx.upload_colony(col)
+    ctx.step(tm.FP64)
+    ctx.set_param("walk_coop", 1)
+    ctx.set_param("walk_f32", 1)
+    before = {k: ctx.get_param(k) for k in keys}
+    cap = ctx.get_param("nbr_cap")
+    ctx.set_param("nbr_cap", 8)
+    with pytest.raises(tm.TMError) as e:
+        ctx.autotune(tm.MIXED)
+    say(str(e.value))
+    assert e.value.status == 5  # TM_ERR_STATE: the lists overflowed during timing
+    assert {k: ctx.get_param(k) for k in keys} == before
+    ctx.step(tm.FP64)
+    check_fp64(ctx.results(), ref)
+    ctx.set_param("nbr_cap", cap)

@@ -1000,12 +1000,36 @@ tm_status tm_graph_launch(tm_ctx *c) {
   return TM_OK;
 }
 
+namespace {
+// the launch shapes a context had, given back to it unless others were chosen
+struct KeepShapes {
+  tm_ctx *c;
+  int nbr_block = c->nbr_block, walk_window = c->walk_window, walk_coop = c->walk_coop, walk_f32 = c->walk_f32;
+  int tile_width = c->tile_width, sph_block = c->sph_block, sph_lanes = c->sph_lanes;
+  int unroll_fp64 = c->sph_unroll_fp64, unroll_mixed = c->sph_unroll_mixed;
+  bool chosen = false;
+  ~KeepShapes() {
+    if (chosen) return;
+    c->nbr_block = nbr_block;
+    c->walk_window = walk_window;
+    c->walk_coop = walk_coop;
+    c->walk_f32 = walk_f32;
+    c->tile_width = tile_width;
+    c->sph_block = sph_block;
+    c->sph_lanes = sph_lanes;
+    c->sph_unroll_fp64 = unroll_fp64;
+    c->sph_unroll_mixed = unroll_mixed;
+  }
+};
+}  // namespace
+
 // Report: one line per trial, "trial <stage> key=value ... ms=<time>", then
 // "chosen key=value ...".  Every candidate gives the same results (the FP64
 // sums keep each list's order whatever the shapes).
 tm_status tm_autotune(tm_ctx *c, tm_precision p, char *buf, size_t buflen) {
   if (!c) return TM_ERR_INVALID;
   if (c->stage < 3) TM_TRY(tm_step(c, p));
+  KeepShapes kept{c};  // a trial that fails leaves the shapes as they were
   std::string rep;
   char line[200];
   // A candidate replaces the current shape only when it is faster by more
@@ -1130,6 +1154,7 @@ tm_status tm_autotune(tm_ctx *c, tm_precision p, char *buf, size_t buflen) {
     unroll = best_u;
     if (p == TM_MIXED) c->sph_lanes = best_l;
   }
+  kept.chosen = true;
   snprintf(line, sizeof(line),
            "chosen precision=%s nbr_block=%d walk_window=%d walk_coop=%d walk_f32=%d sph_tiles=%d tile_width=%d "
            "sph_block=%d unroll=%d lanes=%d\n",
