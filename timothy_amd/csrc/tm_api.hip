@@ -505,9 +505,14 @@ tm_status tm_set_param(tm_ctx *c, const char *key, int64_t v) {
 
 tm_status tm_get_param(tm_ctx *c, const char *key, int64_t *v) {
   if (!c || !key || !v) return TM_ERR_INVALID;
-  // the lists' tiles, where the last step made none
-  if ((!strcmp(key, "tile_lds") || !strcmp(key, "tiles_over")) && c->stage >= 3 && c->sph_tiles && c->tiles_ts == 0)
+  const bool of_tiles = !strcmp(key, "tile_lds") || !strcmp(key, "tiles_over");
+  // the lists' tiles, where the last step made none that a sum may yet ask for
+  if (of_tiles && c->stage >= 3 && c->n > 0 && c->lists_tiles && tm_tiles_serve(c) && c->tiles_ts == 0)
     TM_TRY(tm_run_tiles(c, true));
+  if (of_tiles && c->stage >= 3 && c->tiles_ts == 0) {
+    *v = 0;  // lists without tiles
+    return TM_OK;
+  }
   if (!strcmp(key, "nbr_cap")) *v = c->nbr_cap;
   else if (!strcmp(key, "sph_block")) *v = c->sph_block;
   else if (!strcmp(key, "sph_unroll_fp64")) *v = c->sph_unroll_fp64;
