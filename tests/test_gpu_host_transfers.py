@@ -61,3 +61,37 @@ def test_results_of_some_arrays(tm, ctx):
     v = np.full(500, -1.0)
     ctx._check(tm.lib().tm_get_results(ctx.h, None, v.ctypes.data, None, None, None, None))
     assert np.array_equal(v, ref["v"])
+
+
+# around the sizes from which two, one and no arrays between those asked for are copied
+# with them, and at which results no longer go through pinned memory
+@pytest.mark.parametrize("n", [2, 8192, 8193, 16384, 16385, 32768, 32769, 87381, 87382])
+def test_results_of_any_arrays(tm, ctx, n):
+    print(f"results of {n} cells", flush=True)
+    ctx.upload_colony(colony(n, 7))
+    ctx.step(tm.FP64)
+    r = ctx.results()
+    ref = [r["density"], r["v"], r["mindist"]] + [np.ascontiguousarray(r["force"][:, a]) for a in range(3)]
+    for which in range(64):
+        got = [np.full(n, -1.0) if which >> j & 1 else None for j in range(6)]
+        ctx._check(tm.lib().tm_get_results(ctx.h, *[None if g is None else g.ctypes.data for g in got]))
+        assert all(g is None or np.array_equal(g, q) for g, q in zip(got, ref)), which
+
+
+def test_one_array_is_all_that_is_copied(tm, ctx):
+    """one array at the last size that goes through pinned memory takes as long as at the
+    first that does not (2.2 times that where all six were copied)"""
+    import time
+
+    best = {}
+    for n in (87381, 87382):
+        ctx.upload_colony(colony(n, 7))
+        ctx.step(tm.FP64)
+        v, ts = np.empty(n), []
+        for _ in range(60):
+            t0 = time.perf_counter()
+            ctx._check(tm.lib().tm_get_results(ctx.h, None, v.ctypes.data, None, None, None, None))
+            ts.append(time.perf_counter() - t0)
+        best[n] = min(ts)
+        print(f"one array of {n} cells: {1e6 * best[n]:.0f} us", flush=True)
+    assert best[87381] <= 1.5 * best[87382]
