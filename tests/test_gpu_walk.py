@@ -137,3 +137,59 @@ def test_fp64_sums_with_and_without_tiles(tm, ctx):
         for k in got:
             assert np.array_equal(ctx.results()[k], got[k]), k
     ctx.graph_destroy()
+
+
+def sparse(n, fraction, seed=51, shift=0.0, scale=1.0):
+    """a ball with `fraction` of its volume in cells: 0.08 leaves 53 % without a neighbour"""
+    p = gen.uniform_ball(n, (n / fraction) ** (1 / 3), gen.Stream(seed, 1)) * scale + shift
+    return cells(p, [dict(size=scale, h=2 * scale, h2=4 * scale ** 2, h3=8 * scale ** 3, h4=16 * scale ** 4)])
+
+
+# 32 and 64 cells a wave; from a few to all of a wave's cells without a neighbour, beside
+# some candidates and beside more than are kept; far from the origin; squares beyond FP32
+@pytest.mark.parametrize("name,make", [
+    ("32, 0.3", lambda: sparse(140001, 0.3)), ("32, 0.15", lambda: sparse(140011, 0.15)),
+    ("32, 0.05", lambda: sparse(300007, 0.05)), ("32, 0.005", lambda: sparse(140003, 0.005)),
+    ("64, 0.3", lambda: sparse(800011, 0.3)), ("64, 0.12", lambda: sparse(800029, 0.12)),
+    ("64, 0.04", lambda: sparse(800033, 0.04)), ("64, 0.005", lambda: sparse(790001, 0.005)),
+    ("scattered", lambda: scattered(200003)), ("far", lambda: sparse(150001, 0.06, shift=1e6)),
+    ("beyond FP32", lambda: sparse(140009, 0.06, scale=3e17)),
+    ("two cutoffs", lambda: dict(sparse(200001, 0.1), ctype=(np.arange(200001) % 3 == 0).astype(np.int32),
+                                 types=[wide_type(1.1)[0], wide_type(2.3)[0]]))])
+def test_cells_without_a_neighbour(tm, ctx, name, make):
+    ctx.upload_colony(make())
+    ref, got = outputs(tm, ctx, 0, True), outputs(tm, ctx, 1, True)
+    alone = float(np.mean(np.diff(ref["off"]) == 0))
+    print(f"{name}: {100 * alone:.0f} % without a neighbour", flush=True)
+    assert alone > 0.05
+    for k in ref:
+        assert np.array_equal(got[k], ref[k]), k
+
+
+def test_cells_without_a_neighbour_of_many_colonies(tm, ctx):
+    cols = [sparse(40 + 97 * (i % 9), (0.3, 0.08, 0.01)[i % 3], seed=60 + i % 9) for i in range(900)]
+    ctx.upload_colonies(cols)
+    ref, got = outputs(tm, ctx, 0, True), outputs(tm, ctx, 1, True)
+    for k in ref:
+        assert np.array_equal(got[k], ref[k]), k
+
+
+def test_sparse_colony_takes_no_longer(tm, ctx):
+    """a step of 1M cells, three quarters of them without a neighbour, takes about as long as
+    with one lane per cell (0.95 times that; 1.7 times where they went two or one at a time)"""
+    import time
+
+    ctx.upload_colony(sparse(1000000, 0.04))
+    best = {}
+    for coop in (0, 1):
+        ctx.set_param("walk_coop", coop)
+        ts = []
+        for _ in range(12):
+            ctx.sync()
+            t0 = time.perf_counter()
+            ctx.step(tm.FP64)
+            ctx.sync()
+            ts.append(time.perf_counter() - t0)
+        best[coop] = min(ts)
+    print(f"one lane per cell {1e6 * best[0]:.0f} us, together {1e6 * best[1]:.0f} us", flush=True)
+    assert best[1] <= 1.3 * best[0]
