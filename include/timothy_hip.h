@@ -127,8 +127,8 @@ tm_status tm_set_celltypes(tm_ctx *ctx, const tm_celltype *types, int32_t ntypes
  * own from them; a wave whose cells' two boxes exceed "walk_coop_ratio"
  * (default 64) times their mean box volume and hold many candidates takes
  * them in parts; needs walk_f32; 0 = one lane per cell walks the radix tree,
- * as with walk_f32 = 0, where "nbr_block" and "walk_window" apply; results
- * are identical; default 1); a change of "nbr_cap" or "tile_width" retires a captured graph;
+ * as with walk_f32 = 0 or colonies of a few cells, several to a wave, where
+ * "nbr_block" and "walk_window" apply; results are identical; default 1); a change of "nbr_cap" or "tile_width" retires a captured graph;
  * read-only "nbr_alloc" (slots per cell of the
  * current lists), "tile_lds" (records staged per tile, 0 without tiles) and
  * "tiles_over" (tiles with more than 1536 distinct neighbours, which take

@@ -193,3 +193,43 @@ def test_sparse_colony_takes_no_longer(tm, ctx):
         best[coop] = min(ts)
     print(f"one lane per cell {1e6 * best[0]:.0f} us, together {1e6 * best[1]:.0f} us", flush=True)
     assert best[1] <= 1.3 * best[0]
+
+
+# colonies at and past the mean size from which waves take their cells together, for each
+# number of cells a wave
+@pytest.mark.parametrize("m,size", [(1000, 4), (1000, 5), (5000, 8), (5000, 9), (9000, 16), (9000, 17), (30000, 28),
+                                    (30000, 29)])
+def test_many_small_colonies(tm, ctx, m, size):
+    one = [gen.ball_colony(size, 70 + i) for i in range(30)]
+    ctx.upload_colonies([one[i % 30] for i in range(m)])
+    ref, got = outputs(tm, ctx, 0, False), outputs(tm, ctx, 1, False)
+    for k in ref:
+        assert np.array_equal(got[k], ref[k]), k
+    ctx.graph_capture(tm.FP64)
+    for _ in range(2):
+        ctx.graph_launch()
+        again = ctx.results()
+        assert all(np.array_equal(again[k], ref[k]) for k in again)
+    ctx.graph_destroy()
+
+
+def test_many_small_colonies_take_no_longer(tm, ctx):
+    """a step of 50,000 colonies of three cells takes as long as with one lane per cell (1.5
+    times that where a wave took five colonies one after another)"""
+    import time
+
+    one = [gen.ball_colony(3, 70 + i) for i in range(30)]
+    ctx.upload_colonies([one[i % 30] for i in range(50000)])
+    best = {}
+    for coop in (0, 1):
+        ctx.set_param("walk_coop", coop)
+        ts = []
+        for _ in range(12):
+            ctx.sync()
+            t0 = time.perf_counter()
+            ctx.step(tm.FP64)
+            ctx.sync()
+            ts.append(time.perf_counter() - t0)
+        best[coop] = min(ts)
+    print(f"one lane per cell {1e6 * best[0]:.0f} us, by default {1e6 * best[1]:.0f} us", flush=True)
+    assert best[1] <= 1.2 * best[0]

@@ -1075,6 +1075,20 @@ void launch_walk(tm_ctx *c) {
 // 8 / 16 / 32 / 64 cells: Gaussian 30 K cells 81 / 90 / 101 / 294, 65 K 138 /
 // 116 / 173 / 339, 130 K - / 163 / 175 / 346, 260 K - / 275 / 215 / 343, 600 K
 // - / 562 / 398 / 549, 1M - / 910 / 736 / 748; ball 1M - / 591 / 401 / 339.
+int cells_per_wave(int64_t n) { return n <= 1 << 15 ? 8 : n <= 1 << 17 ? 16 : n <= 3 << 18 ? 32 : 64; }
+
+// Whether a wave holds so many colonies, which it takes one after another, that
+// a lane per cell is faster, its radix tree included.  FP64 steps, together and
+// with a lane per cell: 65,536 colonies of 4 cells 632 and 459 us, of 12 789 and
+// 611, of 24 939 and 899, of 28 1,016 and 992, of 32 996 and 1,084; 50,000 of 14
+// (32 a wave) 671 and 534, 30,000 of 32 522 and 582; 50,000 of 2 (16 a wave) 478 and 361,
+// 10,000 of 8 208 and 201, 3,000 of 16 157 and 184; 3,000 of 2 (8 a wave) 156 and 153,
+// of 6 158 and 163.
+bool many_colonies(int64_t n, int64_t ncol) {
+  const int g = cells_per_wave(n);
+  return ncol > 1 && n <= (g == 64 ? 28 : g / 2) * ncol;
+}
+
 template <int G>
 void launch_union(tm_ctx *c) {
   k_union<G><<<tm_blocks(c->n, 64), 4096 / G, 0, c->stream>>>(
@@ -1108,12 +1122,13 @@ tm_status tm_run_neighbors(tm_ctx *c, bool check, bool tiles) {
     }
     c->nbr_alloc = c->nbr_cap;
     const int bs = c->nbr_block;
-    const bool coop = c->walk_coop && c->walk_f32;
+    const bool coop = c->walk_coop && c->walk_f32 && !many_colonies(n, c->ncol);
+    const int g = coop ? cells_per_wave(n) : 0;
     if (!coop) TM_TRY(tm_ensure_tree(c));
-    if (coop && n <= 1 << 15) launch_union<8>(c);
-    else if (coop && n <= 1 << 17) launch_union<16>(c);
-    else if (coop && n <= 3 << 18) launch_union<32>(c);
-    else if (coop) launch_union<64>(c);
+    if (g == 8) launch_union<8>(c);
+    else if (g == 16) launch_union<16>(c);
+    else if (g == 32) launch_union<32>(c);
+    else if (g == 64) launch_union<64>(c);
     else if (bs == 64) launch_walk<64, 0>(c);
     else if (bs == 128) launch_walk<128, 0>(c);
     else if (c->walk_window == 2048 && 2 * n - 1 >= 2048) launch_walk<256, 2048>(c);
