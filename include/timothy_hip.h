@@ -328,7 +328,10 @@ tm_status tm_last_kernel_ms(tm_ctx *ctx, double *ms);
 
 /* -------- captured step -------- */
 /* capture build + neighbors + sph into a hipGraph (no allocation inside);
- * tm_graph_launch replays it and checks the overflow / degeneracy flags */
+ * tm_graph_launch replays it and checks the overflow / degeneracy flags.  A
+ * call that changes the number of cells or colonies, or that frees memory the
+ * graph holds (longer lists, larger tiles), retires it: tm_graph_launch then
+ * reports that there is none until the next capture */
 tm_status tm_graph_capture(tm_ctx *ctx, tm_precision precision);
 /* the same step followed by tm_update_positions with Philox draws: each
  * replay of the graph is one mechanics step of the resident colony (sort,

@@ -30,7 +30,7 @@ void free_ptr(T *&p) {
 tm_status alloc_cells(tm_ctx *c, int64_t n) {
   if (n <= c->cap_n) return TM_OK;
   int64_t cap = n + (n >> 4) + 64;
-  free_ptr(c->d_key);
+  tm_free(c, c->d_key, true);
   free_ptr(c->d_key_alt);
   free_ptr(c->d_val_alt);
   free_ptr(c->d_perm);
@@ -81,7 +81,7 @@ tm_status alloc_cells(tm_ctx *c, int64_t n) {
 
 tm_status alloc_colonies(tm_ctx *c, int ncol) {
   if (ncol <= c->cap_col) return TM_OK;
-  free_ptr(c->d_col_off);
+  tm_free(c, c->d_col_off, true);
   free_ptr(c->d_aff);
   free_ptr(c->d_col_chunk);
   free_ptr(c->d_colroot);
@@ -151,6 +151,8 @@ tm_status set_cells(tm_ctx *c, int64_t n, int32_t ncol, const int64_t *off, cons
   }
   TM_TRY(alloc_cells(c, std::max<int64_t>(n, 1)));
   TM_TRY(alloc_colonies(c, ncol));
+  // a captured graph's launches are for as many cells, colonies and chunks
+  if (n != c->n || ncol != c->ncol) tm_graph_destroy(c);
   c->n = n;
   c->ncol = ncol;
   c->col_off = o;
@@ -170,9 +172,10 @@ tm_status set_cells(tm_ctx *c, int64_t n, int32_t ncol, const int64_t *off, cons
     }
     cfirst.push_back((int64_t)cc.size());
     cs.push_back(n);
+    if (c->nchunks != (int64_t)cc.size()) tm_graph_destroy(c);
     c->nchunks = (int64_t)cc.size();
     if (c->nchunks + 1 > c->cap_chunks) {
-      free_ptr(c->d_chunk_start);
+      tm_free(c, c->d_chunk_start, true);
       free_ptr(c->d_chunk_cid);
       free_ptr(c->d_cbox);
       c->cap_chunks = 0;
@@ -209,7 +212,7 @@ tm_status set_cells(tm_ctx *c, int64_t n, int32_t ncol, const int64_t *off, cons
     // the other, each padded to 64 elements
     const size_t np = ((size_t)n + 63) & ~(size_t)63, cap = ((size_t)c->cap_n + 63) & ~(size_t)63;
     if (!c->own || c->own_cap < (int64_t)cap) {
-      free_ptr(c->own);
+      tm_free(c, c->own, true);
       c->own_cap = 0;
       if (hipMalloc((void **)&c->own, 44 * cap) != hipSuccess) {
         c->own = nullptr;

@@ -631,7 +631,7 @@ tm_status tm_run_build(tm_ctx *c) {
   k_fixties<<<tm_blocks(n, BT), BT, 0, st>>>(c->d_key, n, c->d_perm, c->d_code, c->d_pos, c->d_posf,
                                               c->d_young_s, c->d_ctype_s, c->d_phase_s, c->d_flags);
   const Bvh t = bvh_of(n);
-  TM_TRY(tm_ensure(c, &c->d_bvh, c->cap_bvh, t.total, "tree of boxes"));
+  TM_TRY(tm_ensure(c, &c->d_bvh, c->cap_bvh, t.total, "tree of boxes", true));
   k_leaf<<<tm_blocks(n, LT), LT, 0, st>>>(c->d_code, n, c->d_span, c->d_leaf, c->d_bvh, t.l1, c->d_flags);
   if (n > 1 << 16) k_bvh_up<<<t.l3 - t.l2, 64, 0, st>>>(c->d_bvh + t.l1, t.l2 - t.l1, c->d_bvh + t.l2);
   if (n > 1 << 22) k_bvh_up<<<t.total - t.l3, 64, 0, st>>>(c->d_bvh + t.l2, t.l3 - t.l2, c->d_bvh + t.l3);
@@ -652,10 +652,7 @@ tm_status tm_ensure_tree(tm_ctx *c) {
     } list[] = {{(void **)&c->d_wn, 32},   {(void **)&c->d_wchain, 4}, {(void **)&c->d_range, 8},
                 {(void **)&c->d_delta, 4}, {(void **)&c->d_split, 4},  {(void **)&c->d_parent, 8}};
     c->cap_tree = 0;
-    for (auto &a : list) {
-      if (*a.p) (void)hipFree(*a.p);
-      *a.p = nullptr;
-    }
+    for (auto &a : list) tm_free(c, *a.p, c->graph_tree);
     for (auto &a : list)
       if (hipMalloc(a.p, a.bytes * (size_t)cap) != hipSuccess) {
         *a.p = nullptr;

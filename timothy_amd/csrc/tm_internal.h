@@ -267,11 +267,19 @@ tm_status tm_fail(tm_ctx *c, tm_status s, const std::string &msg);
     if (_s != TM_OK) return _s;      \
   } while (0)
 
+// frees a buffer; a captured graph that holds it is retired
 template <typename T>
-tm_status tm_ensure(tm_ctx *c, T **p, int64_t &cap, int64_t need, const char *what) {
+void tm_free(tm_ctx *c, T *&p, bool in_graph) {
+  if (!p) return;
+  if (in_graph) tm_graph_destroy(c);
+  (void)hipFree((void *)p);
+  p = nullptr;
+}
+
+template <typename T>
+tm_status tm_ensure(tm_ctx *c, T **p, int64_t &cap, int64_t need, const char *what, bool in_graph = false) {
   if (need <= cap && *p) return TM_OK;
-  if (*p) (void)hipFree(*p);
-  *p = nullptr;
+  tm_free(c, *p, in_graph);
   cap = 0;
   if (need <= 0) return TM_OK;
   if (hipMalloc((void **)p, sizeof(T) * (size_t)need) != hipSuccess) {

@@ -1111,7 +1111,7 @@ tm_status tm_run_neighbors(tm_ctx *c, bool check, bool tiles) {
   for (int attempt = 0; attempt < 2; ++attempt) {
     const int64_t need = tm_slot_elems(n, c->nbr_cap);
     if (c->nbr_elems < need || !c->d_nbr) {
-      if (c->d_nbr) (void)hipFree(c->d_nbr);
+      tm_free(c, c->d_nbr, true);
       c->d_nbr = nullptr;
       c->nbr_elems = 0;
       if (hipMalloc((void **)&c->d_nbr, sizeof(uint32_t) * (size_t)need) != hipSuccess) {
@@ -1152,6 +1152,7 @@ tm_status tm_run_neighbors(tm_ctx *c, bool check, bool tiles) {
     if (c->h_flags[0] & TM_FLAG_CTYPE) return tm_fail(c, TM_ERR_INVALID, "ctype out of range");
     const int64_t mx = c->h_flags[1];
     if (mx <= c->nbr_alloc) break;
+    tm_graph_destroy(c);  // a captured graph has lists of the old length
     c->nbr_cap = (mx + 7) & ~7ll;  // grow to the largest count seen, rounded up
   }
   if (tiles && check) tm_size_tiles(c);

@@ -411,7 +411,7 @@ tm_status tm_scan_u32(tm_ctx *c, const uint32_t *in, uint32_t *out, int64_t n) {
   // scratch layout: level sums for up to three levels
   int64_t nb2 = (nb + SC_TILE - 1) / SC_TILE;
   int64_t need = nb + nb2 + 1;
-  TM_TRY(tm_ensure(c, &c->d_scan, c->cap_scan, need, "scan scratch"));
+  TM_TRY(tm_ensure(c, &c->d_scan, c->cap_scan, need, "scan scratch", c->graph_tree));
   uint32_t *sums = c->d_scan;
   uint32_t *sums2 = c->d_scan + nb;
   k_scan_reduce<<<(unsigned)nb, SC_THREADS, 0, c->stream>>>(in, n, sums);
@@ -485,7 +485,7 @@ static tm_status sort_passes(tm_ctx *c, uint64_t *keys, int32_t *vals, int64_t n
 tm_status tm_sort_prepare(tm_ctx *c, int64_t n, uint32_t **clear, int64_t *words) {
   const int64_t tile = RS_THREADS * (n <= SMALL_N ? 4 : n <= MEDIUM_N ? 8 : 16), nblocks = (n + tile - 1) / tile;
   const int64_t row = 256 * nblocks + 256, gw = n > FEW_N && n <= MEDIUM_N ? group_words(nblocks) : 0;
-  TM_TRY(tm_ensure(c, &c->d_hist, c->cap_hist, n <= FEW_N ? 3 * row : row + 2 * gw, "radix histogram"));
+  TM_TRY(tm_ensure(c, &c->d_hist, c->cap_hist, n <= FEW_N ? 3 * row : row + 2 * gw, "radix histogram", true));
   *clear = c->d_hist + row;
   *words = gw;
   return TM_OK;

@@ -324,10 +324,11 @@ tm_status tm_run_tiles(tm_ctx *c, bool check) {
   }
   const int TS = c->tile_width;
   const int64_t nt = (n + TS - 1) / TS;
-  TM_TRY(tm_ensure(c, &c->d_tile_idx, c->cap_tile_idx, nt * TM_TILE_MAX, "tile indices"));
-  TM_TRY(tm_ensure(c, &c->d_tile_cnt, c->cap_tile_cnt, nt, "tile sizes"));
-  TM_TRY(tm_ensure(c, &c->d_tile_cell, c->cap_tile_cell, nt * TS, "tile ranks"));
-  TM_TRY(tm_ensure(c, &c->d_nbr16, c->cap_nbr16, tm_slot_elems(nt * TS, c->nbr_alloc), "tile lists"));
+  const bool held = c->graph_tiles_ts > 0;
+  TM_TRY(tm_ensure(c, &c->d_tile_idx, c->cap_tile_idx, nt * TM_TILE_MAX, "tile indices", held));
+  TM_TRY(tm_ensure(c, &c->d_tile_cnt, c->cap_tile_cnt, nt, "tile sizes", held));
+  TM_TRY(tm_ensure(c, &c->d_tile_cell, c->cap_tile_cell, nt * TS, "tile ranks", held));
+  TM_TRY(tm_ensure(c, &c->d_nbr16, c->cap_nbr16, tm_slot_elems(nt * TS, c->nbr_alloc), "tile lists", held));
   k_zero_tile_flags<<<1, 1, 0, c->stream>>>(c->d_flags);
   switch (TS) {
     case 128: launch_tiles<128>(c, nt); break;
