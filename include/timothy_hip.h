@@ -121,7 +121,8 @@ tm_status tm_set_celltypes(tm_ctx *ctx, const tm_celltype *types, int32_t ntypes
  * build orders the distinct neighbours within 8192 cells of a tile's middle
  * by bitmap and hashes only the rest; 0 = hashes all of them; results are
  * identical; default 1), "tile_width" cells per LDS tile (128, 256, 512;
- * default 256; takes effect at the next tm_neighbors; results are
+ * default 256; takes effect where tiles are next made: by tm_neighbors, or by
+ * a mixed step, a further sum or "tile_lds" on lists without; results are
  * identical), "walk_coop" (1 = each wave looks once for the candidates of all
  * its cells, in a tree of boxes over the Morton order, and each lane picks its
  * own from them; a wave whose cells' two boxes exceed "walk_coop_ratio"
@@ -132,7 +133,7 @@ tm_status tm_set_celltypes(tm_ctx *ctx, const tm_celltype *types, int32_t ntypes
  * read-only "nbr_alloc" (slots per cell of the
  * current lists), "tile_lds" (records staged per tile, 0 without tiles) and
  * "tiles_over" (tiles with more than 1536 distinct neighbours, which take
- * the 32-bit lists, at the last tm_neighbors) */
+ * the 32-bit lists); both make the tiles that an FP64 step left out */
 tm_status tm_set_param(tm_ctx *ctx, const char *key, int64_t value);
 tm_status tm_get_param(tm_ctx *ctx, const char *key, int64_t *value);
 
@@ -288,11 +289,11 @@ tm_status tm_diffusion_step(tm_ctx *ctx, const tm_grid *grid, const tm_diffusion
                             double *field, int32_t *iterations, double *residual);
 /* No counterpart in the reference.  The same solve for callers that cannot
  * allocate device memory (tight stepping loops, harnesses that forbid
- * hipMalloc): identical kernels and results, but the work arrays (right-hand
- * side, residual, two directions, A p, partial sums, solver state) live in
- * one static device buffer of the library, sized for grids of at most
- * TM_NOALLOC_MAX_NODES nodes (about 48 MiB, held on every device the library
- * runs on until the process ends).  The call allocates nothing; larger grids
+ * hipMalloc): identical kernels and results, but the work arrays (residual,
+ * two directions, partial sums, solver state) live in one static device
+ * buffer of the library, sized for grids of at most TM_NOALLOC_MAX_NODES nodes
+ * (about 48 MiB, held on every device the library runs on until the process
+ * ends).  The call allocates nothing; larger grids
  * are refused with TM_ERR_INVALID.  Every context on one device shares that
  * buffer: calls that overlap on one device (two host threads, or two
  * contexts' streams) race and must be serialised by the caller.  Nothing in

@@ -193,7 +193,7 @@ struct tm_ctx {
   int tile_lds_ts = 0;              // the tile width tile_lds was sized for
   int64_t cap_tile_idx = 0, cap_tile_cnt = 0, cap_tile_cell = 0, cap_nbr16 = 0;
 
-  // environment solve: right-hand side, residual, two directions, A p, partial sums, state
+  // environment solve: residual, two directions, partial sums, state
   double *d_cg = nullptr;
   int64_t cap_cg = 0;
   uint32_t tile_lds = 0;            // neighbour records the pair kernel stages per tile (0: no tiles built)

@@ -473,12 +473,13 @@ __global__ __launch_bounds__(BS) void k_neighbors(const double4 *__restrict__ po
 // instructions per wave), below about 500 K cells the longest wave, whose
 // cells lie in many places: a wave then takes fewer cells (launch_union).
 // Walk alone, per-lane before and this: 20 K-cell ball 119 and 43 us, 300 K
-// ball 208 and 175 us, 2M Gaussian 1,729 and 858 us, 4M cells in 128 colonies
-// 3,358 and 1,900 us, 3M of two types 3,605 and 1,580 us; and the build need not
-// make the radix tree (130 us of 500 at 2M).  Also measured: the per-lane walk's tree read
-// 64 slots at a time in its pre-order (103 dependent loads per wave against 48
-// here) 450 us of a 1.46 ms walk; distances on the vector unit 5% slower at
-// 2M; blocks of 32 cells 8% more loads.
+// ball 208 and 175 us, 2M Gaussian 1,729 and 862 us (three seeds: 843 to 897),
+// 4M cells in 128 colonies 3,358 and 1,700 us, 3M of two types 3,605 and
+// 1,580 us; and the build need not make the radix tree (130 us of 500 at 2M).
+// Also measured: the per-lane walk's tree read 64 slots at a time in its
+// pre-order (103 dependent loads per wave against 48 here) 450 us of a 1.46 ms
+// walk; distances on the vector unit 5% slower at 2M; blocks of 32 cells 8%
+// more loads.
 constexpr int CB = 255;  // candidates staged at a time (a byte names one; 255 names none)
 // FP32 rounding of |c|^2 + |p|^2 - 2 c.p (five products and sums, operands
 // rounded to 2^-24) stays within 1.5e-6 (|c|^2 + |p|^2): the squares are

@@ -139,9 +139,10 @@ __global__ __launch_bounds__(RS_THREADS) void k_rs_scatter(const K *__restrict__
     k[it] = valid ? keys[i] : (K)0;
     v[it] = valid ? vals[i] : 0;
   }
-  // this tile's first slot for digit tid: its keys in the tiles before (FEW:
-  // added up here, else scanned by k_rs_rowscan) plus the keys of all smaller
-  // digits (the digits' totals, scanned here)
+  // this tile's first slot for digit tid: its keys in the tiles before (added
+  // up here from the tiles' histograms, FEW, or from those of its group and the
+  // sums of the groups before, GROUPED; or scanned by k_rs_rowscan) plus the keys
+  // of all smaller digits (the digits' totals, scanned here)
   {
     uint32_t rt = 0, before = 0;
     // adds rows [0, end) to rt, those before `own` also to before
